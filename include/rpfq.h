@@ -542,6 +542,42 @@ size_t rpfq_quantize_workspace_bytes(const rpfq_quant_desc* desc);
 int rpfq_quantize_wide(const rpfq_quant_desc* desc, const float* weight, const float* rot, float* a_q,
                        float* scales, uint8_t* codes, void* work, size_t work_bytes, void* stream);
 
+/* Bytes of the device workspace of rpfq_linear_f32 (backward = 0) or
+ * rpfq_linear_f32_grad (backward = 1); 0 if the shape is not taken. */
+size_t rpfq_linear_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int backward);
+
+/*
+ * float32 linear layer y = x w^T + bias, x [M, K], w [N, K], bias [N] or
+ * NULL, y [M, N], all float32 row-major, N and K multiples of 8 up to 4096.
+ * Runs on the fp16 matrix cores with every operand split into two fp16
+ * terms (22 bits) under power-of-two scales, three products per pair summed
+ * in float32: its distance to the exact sum is no larger than a float32
+ * GEMM's.  Rows with inf or NaN are summed in plain float32.
+ * w_parts[n_parts] (device): values whose absolute sum bounds every |w|
+ * (the scales rpfq_quantize_wide wrote for w; 0 only if w is all 0).
+ * x_scale [M] (out): the power-of-two scale of each row of x, read by
+ * rpfq_linear_f32_grad.  x, w, y 16-byte, work 256-byte aligned.
+ * Replaces F.linear(x, A_q, bias) of RPFQ-ViT-main/quant_models/quant_i.py:554
+ * on float32 activations in training.
+ */
+int rpfq_linear_f32(const float* x, const float* w, const float* bias, int64_t M, int64_t N, int64_t K,
+                    const float* w_parts, int n_parts, float* y, float* x_scale, void* work, size_t work_bytes,
+                    void* stream);
+
+/*
+ * Gradients of rpfq_linear_f32: grad_x = grad_y w (NULL: not wanted) and
+ * grad_w = grad_y^T x (NULL: not wanted), in the same arithmetic; x_scale as
+ * the forward wrote it.  grad_w takes row m of x times the scale of grad_y's
+ * row, so a row whose gradients lie below 2^-17 of the largest row's loses
+ * bits of its (equally smaller) share.  The bias gradient is the column sum
+ * of grad_y and is left to the caller.
+ * Replaces the backward of that F.linear (grad_x = grad_output @ weight,
+ * grad_weight = grad_output^T @ x; kernel.py:581-588).
+ */
+int rpfq_linear_f32_grad(const float* grad_y, const float* x, const float* w, int64_t M, int64_t N, int64_t K,
+                         const float* w_parts, int n_parts, const float* x_scale, float* grad_x, float* grad_w,
+                         void* work, size_t work_bytes, void* stream);
+
 /*
  * rpfq_quantize_wide without a workspace argument and without any device
  * allocation: the float64 partials live in a static device array of this

@@ -71,6 +71,15 @@ int check_ln(const void* x, int x_dtype, int64_t M, int64_t C, const float* gamm
     return RPFQ_OK;
 }
 
+int check_linear_f32(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0)
+        return fail(RPFQ_ERR_SHAPE, "M=%lld N=%lld K=%lld must be positive", (long long)M, (long long)N, (long long)K);
+    if (N % 8 != 0 || K % 8 != 0 || N > 4096 || K > 4096)
+        return fail(RPFQ_ERR_SHAPE, "N=%lld K=%lld must be multiples of 8 up to 4096", (long long)N, (long long)K);
+    if (M > (1LL << 24)) return fail(RPFQ_ERR_SHAPE, "M=%lld too large", (long long)M);
+    return RPFQ_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -586,6 +595,46 @@ int rpfq_quantize_wide_noalloc(const rpfq_quant_desc* desc, const float* weight,
     return hip_status(rpfq::launch_quantize_wide(*desc, weight, rot, a_q, scales, codes, work,
                                                  reinterpret_cast<hipStream_t>(stream)),
                       "rpfq_quantize_wide_noalloc");
+}
+
+size_t rpfq_linear_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int backward) {
+    if (check_linear_f32(M, N, K) != RPFQ_OK) return 0;
+    const rpfq::F32Plan p = rpfq::f32_plan(M, N, K);
+    return backward ? p.bwd_bytes : p.fwd_bytes;
+}
+
+int rpfq_linear_f32(const float* x, const float* w, const float* bias, int64_t M, int64_t N, int64_t K,
+                    const float* w_parts, int n_parts, float* y, float* x_scale, void* work, size_t work_bytes,
+                    void* stream) {
+    int rc = check_linear_f32(M, N, K);
+    if (rc) return rc;
+    if (!x || !w || !w_parts || !y || !x_scale || !work) return fail(RPFQ_ERR_NULL, "rpfq_linear_f32: NULL pointer argument");
+    if (n_parts < 1 || n_parts > 1024) return fail(RPFQ_ERR_VALUE, "n_parts=%d must be 1..1024", n_parts);
+    if (!aligned(x, 16) || !aligned(w, 16) || !aligned(y, 16) || !aligned(work, 256))
+        return fail(RPFQ_ERR_ALIGN, "x, w, y must be 16-byte and work 256-byte aligned");
+    const size_t need = rpfq_linear_f32_workspace_bytes(M, N, K, 0);
+    if (work_bytes < need) return fail(RPFQ_ERR_SHAPE, "workspace holds %zu bytes, need %zu", work_bytes, need);
+    return hip_status(rpfq::launch_linear_f32(x, w, bias, M, N, K, w_parts, n_parts, y, x_scale, work,
+                                              reinterpret_cast<hipStream_t>(stream)),
+                      "rpfq_linear_f32");
+}
+
+int rpfq_linear_f32_grad(const float* grad_y, const float* x, const float* w, int64_t M, int64_t N, int64_t K,
+                         const float* w_parts, int n_parts, const float* x_scale, float* grad_x, float* grad_w,
+                         void* work, size_t work_bytes, void* stream) {
+    int rc = check_linear_f32(M, N, K);
+    if (rc) return rc;
+    if (!grad_y || !x || !w || !w_parts || !x_scale || !work || (!grad_x && !grad_w))
+        return fail(RPFQ_ERR_NULL, "rpfq_linear_f32_grad: NULL pointer argument");
+    if (n_parts < 1 || n_parts > 1024) return fail(RPFQ_ERR_VALUE, "n_parts=%d must be 1..1024", n_parts);
+    if (!aligned(grad_y, 16) || !aligned(x, 16) || !aligned(w, 16) || !aligned(grad_x, 16) || !aligned(grad_w, 16) ||
+        !aligned(work, 256))
+        return fail(RPFQ_ERR_ALIGN, "grad_y, x, w and the gradients must be 16-byte and work 256-byte aligned");
+    const size_t need = rpfq_linear_f32_workspace_bytes(M, N, K, 1);
+    if (work_bytes < need) return fail(RPFQ_ERR_SHAPE, "workspace holds %zu bytes, need %zu", work_bytes, need);
+    return hip_status(rpfq::launch_linear_f32_grad(grad_y, x, w, M, N, K, w_parts, n_parts, x_scale, grad_x, grad_w,
+                                                   work, reinterpret_cast<hipStream_t>(stream)),
+                      "rpfq_linear_f32_grad");
 }
 
 }  // extern "C"

@@ -75,6 +75,9 @@ EXPORTED = (
     "rpfq_wide_linear_scaled",
     "rpfq_wide_mlp",
     "rpfq_layer_norm_wide_mlp",
+    "rpfq_linear_f32_workspace_bytes",
+    "rpfq_linear_f32",
+    "rpfq_linear_f32_grad",
 )
 
 
@@ -172,8 +175,13 @@ def load() -> ctypes.CDLL:
         lib.rpfq_wide_mlp.argtypes = [dp, vp, sz, dp, vp, sz, vp, i64, vp, vp, vp, vp, vp]
         lib.rpfq_layer_norm_wide_mlp.argtypes = [dp, vp, sz, dp, vp, sz, vp, i64, vp, vp, ctypes.c_float, vp, vp, vp,
                                                  vp]
+        lib.rpfq_linear_f32_workspace_bytes.argtypes = [i64, i64, i64, i32]
+        lib.rpfq_linear_f32_workspace_bytes.restype = sz
+        lib.rpfq_linear_f32.argtypes = [vp, vp, vp, i64, i64, i64, vp, i32, vp, vp, vp, sz, vp]
+        lib.rpfq_linear_f32_grad.argtypes = [vp, vp, vp, i64, i64, i64, vp, i32, vp, vp, vp, vp, sz, vp]
         for name in EXPORTED[2:]:
-            if name not in ("rpfq_wide_packed_bytes", "rpfq_wide_adjoint_bytes", "rpfq_quantize_workspace_bytes"):
+            if name not in ("rpfq_wide_packed_bytes", "rpfq_wide_adjoint_bytes", "rpfq_quantize_workspace_bytes",
+                            "rpfq_linear_f32_workspace_bytes"):
                 getattr(lib, name).restype = i32
         _lib = lib
         return lib

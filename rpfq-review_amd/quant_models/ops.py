@@ -631,6 +631,42 @@ def quantize_wide(weight: torch.Tensor, kind_u: str, steps_u: int, kind_w: str, 
     return a_q, scales, codes
 
 
+def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, w_parts: torch.Tensor):
+    """(y, x_scale): y = x w^T + bias on contiguous float32 [M, K], [N, K] at
+    float32 accuracy (rpfq_linear_f32); w_parts: float32 values whose absolute
+    sum bounds |w|; x_scale [M] goes to linear_f32_grad."""
+    N.require_device(x, w, bias, w_parts)
+    m, k = x.shape
+    n = w.shape[0]
+    lib = N.load()
+    nbytes = lib.rpfq_linear_f32_workspace_bytes(m, n, k, 0)
+    y = torch.empty(m, n, dtype=torch.float32, device=x.device)
+    scale = torch.empty(m, dtype=torch.float32, device=x.device)
+    work = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    N.check("rpfq_linear_f32", lib.rpfq_linear_f32(
+        x.data_ptr(), w.data_ptr(), N.ptr(bias), m, n, k, w_parts.data_ptr(), w_parts.numel(), y.data_ptr(),
+        scale.data_ptr(), work.data_ptr(), nbytes, N.stream_of(x)))
+    return y, scale
+
+
+def linear_f32_grad(grad_y: torch.Tensor, x: torch.Tensor, w: torch.Tensor, w_parts: torch.Tensor,
+                    x_scale: torch.Tensor, want_x: bool = True, want_w: bool = True):
+    """(grad_x or None, grad_w or None) of linear_f32 (rpfq_linear_f32_grad)
+    for a contiguous float32 grad_y [M, N]."""
+    N.require_device(grad_y, x, w, w_parts, x_scale)
+    m, k = x.shape
+    n = w.shape[0]
+    lib = N.load()
+    nbytes = lib.rpfq_linear_f32_workspace_bytes(m, n, k, 1)
+    gx = torch.empty_like(x) if want_x else None
+    gw = torch.empty_like(w) if want_w else None
+    work = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    N.check("rpfq_linear_f32_grad", lib.rpfq_linear_f32_grad(
+        grad_y.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k, w_parts.data_ptr(), w_parts.numel(),
+        x_scale.data_ptr(), N.ptr(gx), N.ptr(gw), work.data_ptr(), nbytes, N.stream_of(x)))
+    return gx, gw
+
+
 def make_desc(n_complex, k_complex, codebook, stages, block, rotation) -> N.WideDesc:
     d = N.WideDesc()
     d.n_complex = int(n_complex)

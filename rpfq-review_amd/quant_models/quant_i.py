@@ -325,6 +325,9 @@ PRESCALED_LN = os.environ.get("RPFQ_PRESCALED_LN", "1") != "0"
 # a host read of each rotated layer's angles cost more than the kernel,
 # which is slower than the library's fp16 GEMM on the decoded weight).
 QAT_PACKED_GRAD = os.environ.get("RPFQ_QAT_PACKED_GRAD", "0")
+# float32 training products of at least this many operations (2 M N K) run on
+# split fp16 operands (_split_linear_pays)
+SPLIT_LINEAR_MIN = 4.5e9
 
 _HIP_KINDS = {
     "complex_phase_v1": ("axis", 1),
@@ -359,7 +362,8 @@ def _blocks(a: torch.Tensor):
 
 
 class _HipWideQuantSTE(torch.autograd.Function):
-    """A_q from the float32 master weight by rpfq_quantize_wide; backward:
+    """A_q from the float32 master weight by rpfq_quantize_wide, and its
+    scales (whose sum bounds |A_q|); backward:
     the weight gets the A_q gradient unchanged (split and recombination are
     inverse linear maps and the quantizer is straight-through), the rotation
     angles get rotation_grad."""
@@ -372,14 +376,15 @@ class _HipWideQuantSTE(torch.autograd.Function):
         if theta_u is not None:
             tu, tw = theta_u.detach().float().reshape(1), theta_w.detach().float().reshape(1)
             rot = torch.cat((torch.cos(tu), torch.sin(tu), torch.cos(tw), torch.sin(tw)))
-        a_q, _, _ = ops.quantize_wide(weight.detach(), *spec, rot=rot)
+        a_q, scales, _ = ops.quantize_wide(weight.detach(), *spec, rot=rot)
         ctx.rotated = theta_u is not None
         if ctx.rotated:
             ctx.save_for_backward(weight, a_q)
-        return a_q
+        ctx.mark_non_differentiable(scales)
+        return a_q, scales
 
     @staticmethod
-    def backward(ctx, grad):
+    def backward(ctx, grad, _):
         if not ctx.rotated:
             return grad, None, None, None
         weight, a_q = ctx.saved_tensors
@@ -478,10 +483,66 @@ def records_grad(module: nn.Module, x: torch.Tensor) -> bool:
     return torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in module.parameters()))
 
 
-def _linear(x: torch.Tensor, q_weight: torch.Tensor, bias):
-    """F.linear(x, A_q, bias) (quant_i.py:554).  Reduced-precision x outside
+class _SplitLinearFn(torch.autograd.Function):
+    """F.linear of float32 x and A_q on the split-fp16 matrix-core kernels
+    (rpfq_linear_f32, float32 accuracy); the bias gradient is the column sum.
+    A backward that autograd records (create_graph) runs torch's products."""
+
+    @staticmethod
+    def forward(ctx, x, w, bias, parts):
+        from . import ops
+
+        x2 = ops._aligned_rows(x.reshape(-1, x.shape[-1]))
+        y, scale = ops.linear_f32(x2, w, bias, parts)
+        ctx.has_bias = bias is not None
+        ctx.save_for_backward(x, w, parts, scale)
+        return y.reshape(*x.shape[:-1], w.shape[0])
+
+    @staticmethod
+    def backward(ctx, grad):
+        from . import ops
+
+        x, w, parts, scale = ctx.saved_tensors
+        g2, x2 = grad.reshape(-1, grad.shape[-1]), x.reshape(-1, x.shape[-1])
+        want_x, want_w = ctx.needs_input_grad[:2]
+        if torch.is_grad_enabled():
+            gx = g2 @ w if want_x else None
+            gw = g2.t() @ x2 if want_w else None
+        elif want_x or want_w:
+            gx, gw = ops.linear_f32_grad(ops._aligned_rows(g2), ops._aligned_rows(x2), w, parts, scale, want_x, want_w)
+        else:
+            gx = gw = None
+        gb = g2.sum(0) if ctx.has_bias and ctx.needs_input_grad[2] else None
+        return None if gx is None else gx.reshape(x.shape), gw, gb, None
+
+
+def _split_linear_pays(x: torch.Tensor, w: torch.Tensor, bias) -> bool:
+    """Whether float32 x and A_q take _SplitLinearFn: shapes the kernels hold
+    (rpfq_linear_f32) and enough work to cover the operand splits, and none of
+    the transforms that an autograd function without their rules refuses.
+    MI355X, forward + backward against the float32 library GEMMs, us: 12,608
+    rows, 3072 x 768 (59 GFLOP a product) 596 against 1,492; 768 x 768 (15)
+    235 against 452; 3,152 rows, 1000 x 768 (4.8) 130 against 190; 1,576 rows,
+    768 x 768 (1.9) 97 against 75; 512 rows, 4096 x 1024 (4.3) 163 against
+    115."""
+    n, k = w.shape
+    m = x.numel() // k
+    if not (x.is_cuda and x.dtype == w.dtype == torch.float32 and (bias is None or bias.dtype == torch.float32)
+            and n % 8 == 0 and k % 8 == 0 and n <= 4096 and k <= 4096 and m <= 1 << 24
+            and w.is_contiguous() and w.data_ptr() % 16 == 0 and m >= 1024 and 2 * m * n * k >= SPLIT_LINEAR_MIN):
+        return False
+    if torch.is_autocast_enabled(x.device.type) or torch._C._are_functorch_transforms_active():
+        return False
+    return torch.autograd.forward_ad._current_level < 0
+
+
+def _linear(x: torch.Tensor, q_weight: torch.Tensor, bias, parts=None):
+    """F.linear(x, A_q, bias) (quant_i.py:554); parts: the scales of A_q where
+    the HIP quantizer wrote them.  Reduced-precision x outside
     autocast meets A_q and the bias cast to x's dtype, as autocast casts
     them (autograd flows through the casts)."""
+    if parts is not None and _split_linear_pays(x, q_weight, bias):
+        return _SplitLinearFn.apply(x, q_weight, bias, parts)
     if x.dtype != q_weight.dtype and not torch.is_autocast_enabled(x.device.type):
         q_weight = q_weight.to(x.dtype)
         bias = None if bias is None else bias.to(x.dtype)
@@ -569,15 +630,15 @@ class QATLinearComplexPhase(nn.Linear):
         if spec is not None and spec[0] == spec[2] and spec[1] == spec[3] and self._packed_grad():
             return self._qat_forward_packed_grad(x, spec)
         if spec is not None:
-            q_weight = _HipWideQuantSTE.apply(self.weight, self.quantizer_u.rotation_angle,
-                                              self.quantizer_w.rotation_angle, spec)
+            q_weight, scales = _HipWideQuantSTE.apply(self.weight, self.quantizer_u.rotation_angle,
+                                                      self.quantizer_w.rotation_angle, spec)
             if self.act_quantizer is not None:
                 if x.dtype == torch.float32:
                     x = _HipActQuantSTE.apply(x, self.act_quantizer.num_bits)
                 else:  # reduced-precision activations: the reference's per-op rounding
                     h = self.in_features // 2
                     x = torch.cat(self.act_quantizer(x[..., :h], x[..., h:]), dim=-1)
-            return _linear(x, q_weight, self.bias)
+            return _linear(x, q_weight, self.bias, scales)
         q_weight = self.quantized_weight()
         if self.act_quantizer is not None:
             h = self.in_features // 2

@@ -1,0 +1,191 @@
+"""float32 linear layer and gradients on split fp16 operands (rpfq_linear_f32,
+rpfq_linear_f32_grad) against float64.
+
+Bar, per output: two 22-bit operands and the dropped low x low product cost
+at most 2^-20 of sum |a| |b|, each of the 3 K / 16 float32 accumulations of
+an output at most 2^-23 of it (the partial sums a matrix instruction rounds),
+and values below 2^-39 of their row's largest (gw: of the tensor's) are lost.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+DEV = "cuda"
+
+
+def _bound(a, b, con, floor):
+    return (2.0 ** -20 + 3 * (con / 16 + 1) * 2.0 ** -23) * (a.abs() @ b.abs()) + floor
+
+
+def _inputs(m, n, k, seed=0, dev=DEV):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    x = torch.randn(m, k, device=dev, generator=g)
+    x *= torch.exp2(torch.randint(-3, 4, (m, 1), device=dev, generator=g).float())
+    w = torch.randn(n, k, device=dev, generator=g) * 0.02
+    gy = torch.randn(m, n, device=dev, generator=g) * 1e-3
+    return x, w, torch.randn(n, device=dev, generator=g), gy
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(1, 8, 8), (15, 40, 24), (16, 256, 32), (65, 264, 40), (96, 128, 64), (127, 8, 776),
+                                   (129, 1000, 264), (385, 512, 96), (2048, 136, 4096), (1300, 4096, 256)])
+def test_linear_f32_and_grad_match_float64(m, n, k):
+    from quant_models import ops
+
+    x, w, b, gy = _inputs(m, n, k)
+    parts = w.abs().max().reshape(1)
+    y, scale = ops.linear_f32(x, w, b, parts)
+    gx, gw = ops.linear_f32_grad(gy, x, w, parts, scale)
+    xd, wd, gd = x.double(), w.double(), gy.double()
+    wmax = float(wd.abs().max())
+    rowx, rowg = xd.abs().amax(1, keepdim=True), gd.abs().amax(1, keepdim=True)
+    ey = xd @ wd.t() + b.double()
+    assert bool(((y.double() - ey).abs() <= _bound(xd, wd.t(), k, k * 2.0 ** -38 * rowx * wmax) + 2.0 ** -23 * ey.abs()).all())
+    assert bool(((gx.double() - gd @ wd).abs() <= _bound(gd, wd, n, n * 2.0 ** -38 * rowg * wmax)).all())
+    big = float((rowx * rowg).max())
+    assert bool(((gw.double() - gd.t() @ xd).abs() <= _bound(gd.t(), xd, m, m * 2.0 ** -38 * big)).all())
+
+
+@pytest.mark.gpu
+def test_linear_f32_rows_of_any_magnitude():
+    """Row scales from 2^-100 to 2^100 and zero rows: every row of y and gx
+    keeps its own accuracy; gw that of the largest rows."""
+    from quant_models import ops
+
+    m, n, k = 200, 72, 104
+    x, w, _, gy = _inputs(m, n, k)
+    e = torch.linspace(-100, 60, m, device=DEV).round().reshape(-1, 1)
+    x, gy = x * torch.exp2(e), gy * torch.exp2(-e)
+    x[::7], gy[::5] = 0, 0
+    parts = w.abs().max().reshape(1)
+    y, scale = ops.linear_f32(x, w, None, parts)
+    gx, gw = ops.linear_f32_grad(gy, x, w, parts, scale)
+    xd, wd, gd = x.double(), w.double(), gy.double()
+    wmax = float(wd.abs().max())
+    assert bool(((y.double() - xd @ wd.t()).abs() <= _bound(xd, wd.t(), k, k * 2.0 ** -38 * xd.abs().amax(1, keepdim=True) * wmax)).all())
+    assert bool(((gx.double() - gd @ wd).abs() <= _bound(gd, wd, n, n * 2.0 ** -38 * gd.abs().amax(1, keepdim=True) * wmax)).all())
+    big = float((xd.abs().amax(1) * gd.abs().amax(1)).max())
+    assert bool(((gw.double() - gd.t() @ xd).abs() <= _bound(gd.t(), xd, m, m * 2.0 ** -38 * big)).all())
+    assert not y[::7].any() and not gx[::5].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", ["x", "gy", "w"])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.0e38])
+def test_linear_f32_special_values(where, value):
+    """inf, NaN and the largest floats come out as in a float32 product."""
+    from quant_models import ops
+
+    x, w, b, gy = _inputs(150, 40, 64)
+    t = {"x": x, "gy": gy, "w": w}[where]
+    t[5, 3] = value
+    parts = w.abs().max().reshape(1)
+    y, scale = ops.linear_f32(x, w, b, parts)
+    gx, gw = ops.linear_f32_grad(gy, x, w, parts, scale)
+    xc, wc, gc = x.cpu(), w.cpu(), gy.cpu()
+    for got, ref in ((y, xc @ wc.t() + b.cpu()), (gx, gc @ wc), (gw, gc.t() @ xc)):
+        got = got.cpu()
+        assert torch.equal(torch.isnan(got), torch.isnan(ref))
+        assert torch.equal(torch.isinf(got), torch.isinf(ref))
+        assert torch.equal(got[torch.isinf(got)], ref[torch.isinf(ref)])
+
+
+@pytest.mark.gpu
+def test_linear_f32_empty_gradient():
+    from quant_models import ops
+
+    x, w, _, gy = _inputs(130, 24, 48)
+    parts = w.abs().max().reshape(1)
+    _, scale = ops.linear_f32(x, w, None, parts)
+    gx, gw = ops.linear_f32_grad(torch.zeros_like(gy), x, w, parts, scale)
+    assert not gx.any() and not gw.any()
+
+
+def _layer(method, act, rot, seed=3):
+    from quant_models.quant_i import QATLinearComplexPhase
+
+    torch.manual_seed(seed)
+    return QATLinearComplexPhase(method, method, act > 0, max(2, act), rot, in_features=1024, out_features=1536).cuda()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("method,act,rot", [("complex_phase_v2", 4, False), ("complex_phase_v1", 0, True),
+                                            ("complex_phase_new_v2", 8, True), ("complex_phase_v4", 0, False)])
+def test_training_layer_takes_the_split_product(method, act, rot, monkeypatch):
+    """The layer's float32 training step on the split kernels against the
+    same step on torch's product: float32 rounding, 2^-17 of the largest."""
+    from quant_models import quant_i
+
+    layer = _layer(method, act, rot)
+    x0 = torch.randn(4, 400, 1024, device=DEV)
+    gy = torch.randn(4, 400, 1536, device=DEV)
+    calls, real = [], quant_i._SplitLinearFn.apply
+    monkeypatch.setattr(quant_i._SplitLinearFn, "apply", lambda *a: calls.append(1) or real(*a))
+    out = []
+    for limit in (0, float("inf")):
+        monkeypatch.setattr(quant_i, "SPLIT_LINEAR_MIN", limit)
+        x = x0.clone().requires_grad_(True)
+        layer.zero_grad(set_to_none=True)
+        y = layer(x)
+        y.backward(gy)
+        out.append([y.detach(), x.grad] + [p.grad for p in layer.parameters()])
+    assert len(calls) == 1
+    for a, b in zip(*out):
+        assert a.shape == b.shape
+        # a rotation's gradient sums 1.5 M products of cancelling signs
+        assert float((a - b).abs().max()) <= (2.0 ** -10 if a.numel() == 1 else 2.0 ** -17) * float(b.abs().max())
+
+
+@pytest.mark.gpu
+def test_training_layer_double_backward_and_forward_mode():
+    """create_graph gradients of the split product, and forward-mode
+    differentiation (which keeps F.linear)."""
+    layer = _layer("complex_phase_v2", 0, False)
+    x = torch.randn(2000, 1024, device=DEV, requires_grad=True)
+    gy = torch.randn(2000, 1536, device=DEV, requires_grad=True)
+    (gx,) = torch.autograd.grad(layer(x), x, gy, create_graph=True)
+    (ggy,) = torch.autograd.grad(gx, gy, torch.ones_like(gx))
+    a = layer.quantized_weight().detach()
+    assert torch.allclose(gx.detach(), gy.detach() @ a, rtol=1e-4, atol=1e-4)
+    assert torch.allclose(ggy, torch.ones_like(gx) @ a.t(), rtol=1e-4, atol=1e-4)
+    for p in layer.parameters():
+        p.requires_grad_(False)
+    with torch.autograd.forward_ad.dual_level():
+        t = torch.randn_like(x)
+        y = layer(torch.autograd.forward_ad.make_dual(x.detach(), t))
+        ty = torch.autograd.forward_ad.unpack_dual(y).tangent
+    assert torch.allclose(ty, t @ a.t(), rtol=1e-4, atol=1e-4)
+
+
+def test_linear_f32_argument_errors():
+    """Reported on the host, without a GPU."""
+    from quant_models import _native as N
+
+    lib = N.load()
+    p = ctypes.c_void_p(4096)
+    assert lib.rpfq_linear_f32_workspace_bytes(64, 64, 64, 0) > 64 * 64 * 4
+    for m, n, k in ((0, 64, 64), (64, 60, 64), (64, 64, 4104), (1 << 25, 64, 64)):
+        assert lib.rpfq_linear_f32_workspace_bytes(m, n, k, 1) == 0
+        assert lib.rpfq_linear_f32(p, p, None, m, n, k, p, 1, p, p, p, 1 << 30, None) == 2
+    assert lib.rpfq_linear_f32(p, None, None, 64, 64, 64, p, 1, p, p, p, 1 << 30, None) == 1
+    assert lib.rpfq_linear_f32(p, p, None, 64, 64, 64, p, 0, p, p, p, 1 << 30, None) == 6
+    assert lib.rpfq_linear_f32(p, p, None, 64, 64, 64, p, 1, p, p, p, 1024, None) == 2
+    assert lib.rpfq_linear_f32(ctypes.c_void_p(4100), p, None, 64, 64, 64, p, 1, p, p, p, 1 << 30, None) == 3
+    assert lib.rpfq_linear_f32_grad(p, p, p, 64, 64, 64, p, 1, p, None, None, p, 1 << 30, None) == 1
+
+
+def test_row_and_weight_scales_hold_the_bound():
+    """The float32 A_q of every method stays below the sum of its scales
+    (what scales w in rpfq_linear_f32), also rotated."""
+    from oracle import rpfq_oracle as O
+
+    rng = np.random.default_rng(0)
+    w = rng.standard_normal((64, 48)).astype(np.float32)
+    for kind, steps in (("axis", 1), ("axis", 2), ("axis", 4), ("sign", 2)):
+        for t in (0.0, 0.7, -1.9):
+            cs = (np.float32(np.cos(t)), np.float32(np.sin(t)))
+            a, su, sw = O.quantized_weight(w, kind, steps, kind, steps, (cs, cs) if t else None)
+            total = sum(float(abs(s_re)) + float(abs(s_im)) for _, s_re, s_im in su + sw)
+            assert np.abs(a).max() <= total * (1 + 2.0 ** -20)
