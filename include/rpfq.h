@@ -542,6 +542,17 @@ size_t rpfq_quantize_workspace_bytes(const rpfq_quant_desc* desc);
 int rpfq_quantize_wide(const rpfq_quant_desc* desc, const float* weight, const float* rot, float* a_q,
                        float* scales, uint8_t* codes, void* work, size_t work_bytes, void* stream);
 
+/*
+ * out = softmax(q k^T scale) v per image and head, without mask or dropout:
+ * qkv [B, N, 3, H, D] (the qkv layer's output as it lies), out [B, N, H, D],
+ * both of dtype (RPFQ_F16 or RPFQ_BF16), 16-byte aligned; D = 64, N <= 288.
+ * Scores, softmax and outputs in float32, probabilities rounded to dtype for
+ * their product with v.  Replaces the attention between qkv and proj of a
+ * ViT block (RPFQ-ViTApple/scripts/audit_rpfq_vit_ios_parity.py:523-545).
+ */
+int rpfq_attention(const void* qkv, int dtype, int64_t B, int64_t N, int64_t H, int64_t D, float scale, void* out,
+                   void* stream);
+
 /* Bytes of the device workspace of rpfq_linear_f32 (backward = 0) or
  * rpfq_linear_f32_grad (backward = 1); 0 if the shape is not taken. */
 size_t rpfq_linear_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int backward);

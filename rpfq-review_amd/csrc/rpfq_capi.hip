@@ -597,6 +597,19 @@ int rpfq_quantize_wide_noalloc(const rpfq_quant_desc* desc, const float* weight,
                       "rpfq_quantize_wide_noalloc");
 }
 
+int rpfq_attention(const void* qkv, int dtype, int64_t B, int64_t N, int64_t H, int64_t D, float scale, void* out,
+                   void* stream) {
+    if (!qkv || !out) return fail(RPFQ_ERR_NULL, "qkv/out must not be NULL");
+    if (dtype != RPFQ_F16 && dtype != RPFQ_BF16) return fail(RPFQ_ERR_DTYPE, "unsupported dtype %d", dtype);
+    if (B <= 0 || N <= 0 || H <= 0) return fail(RPFQ_ERR_SHAPE, "B=%lld N=%lld H=%lld must be positive", (long long)B, (long long)N, (long long)H);
+    if (D != 64 || N > rpfq::kAttnMaxN || H > 1024 || B > (1LL << 24) / H)
+        return fail(RPFQ_ERR_SHAPE, "takes heads of 64 values, N <= %d, H <= 1024, B H <= 2^24 (N=%lld H=%lld D=%lld)",
+                    rpfq::kAttnMaxN, (long long)N, (long long)H, (long long)D);
+    if (!aligned(qkv, 16) || !aligned(out, 16)) return fail(RPFQ_ERR_ALIGN, "qkv and out must be 16-byte aligned");
+    return hip_status(rpfq::launch_attention(qkv, dtype, B, N, H, scale, out, reinterpret_cast<hipStream_t>(stream)),
+                      "rpfq_attention");
+}
+
 size_t rpfq_linear_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int backward) {
     if (check_linear_f32(M, N, K) != RPFQ_OK) return 0;
     const rpfq::F32Plan p = rpfq::f32_plan(M, N, K);

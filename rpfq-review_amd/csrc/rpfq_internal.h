@@ -320,6 +320,10 @@ size_t quant_scratch_bytes();
 hipError_t quant_scratch_ptr(void** out);
 hipError_t launch_wide_decode(const rpfq_wide_desc& d, const WideGeom& g, const void* packed,
                               float* a, int round_fp16, hipStream_t s);
+// attention of a qkv tensor (attention.hip): 64 values a head, N <= kAttnMaxN
+constexpr int kAttnMaxN = 288;
+hipError_t launch_attention(const void* qkv, int dt, int64_t B, int64_t N, int64_t H, float scale, void* out,
+                            hipStream_t s);
 // float32 linear layer on split fp16 operands (linear_f32.hip): its workspaces
 struct F32Plan {
     int64_t Mp, Kp, Np;          // padded rows and columns of the operand planes

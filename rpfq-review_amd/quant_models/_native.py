@@ -75,6 +75,7 @@ EXPORTED = (
     "rpfq_wide_linear_scaled",
     "rpfq_wide_mlp",
     "rpfq_layer_norm_wide_mlp",
+    "rpfq_attention",
     "rpfq_linear_f32_workspace_bytes",
     "rpfq_linear_f32",
     "rpfq_linear_f32_grad",
@@ -175,6 +176,7 @@ def load() -> ctypes.CDLL:
         lib.rpfq_wide_mlp.argtypes = [dp, vp, sz, dp, vp, sz, vp, i64, vp, vp, vp, vp, vp]
         lib.rpfq_layer_norm_wide_mlp.argtypes = [dp, vp, sz, dp, vp, sz, vp, i64, vp, vp, ctypes.c_float, vp, vp, vp,
                                                  vp]
+        lib.rpfq_attention.argtypes = [vp, i32, i64, i64, i64, i64, ctypes.c_float, vp, vp]
         lib.rpfq_linear_f32_workspace_bytes.argtypes = [i64, i64, i64, i32]
         lib.rpfq_linear_f32_workspace_bytes.restype = sz
         lib.rpfq_linear_f32.argtypes = [vp, vp, vp, i64, i64, i64, vp, i32, vp, vp, vp, sz, vp]

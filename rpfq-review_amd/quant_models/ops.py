@@ -631,6 +631,24 @@ def quantize_wide(weight: torch.Tensor, kind_u: str, steps_u: int, kind_w: str, 
     return a_q, scales, codes
 
 
+ATTENTION_MAX_TOKENS = 288
+
+
+def attention(qkv: torch.Tensor, num_heads: int, scale: float) -> torch.Tensor:
+    """softmax(q k^T scale) v [B, N, C] of a qkv tensor [B, N, 3 C] (fp16 or
+    bf16, heads of 64 values, N <= ATTENTION_MAX_TOKENS; rpfq_attention)."""
+    N.require_device(qkv)
+    b, n, c3 = qkv.shape
+    c = c3 // 3
+    qkv = _aligned_rows(qkv)
+    out = torch.empty(b, n, c, dtype=qkv.dtype, device=qkv.device)
+    if b and n:
+        N.check("rpfq_attention", N.load().rpfq_attention(
+            qkv.data_ptr(), N.dtype_code(qkv.dtype), b, n, num_heads, c // num_heads, float(scale), out.data_ptr(),
+            N.stream_of(qkv)))
+    return out
+
+
 def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, w_parts: torch.Tensor):
     """(y, x_scale): y = x w^T + bias on contiguous float32 [M, K], [N, K] at
     float32 accuracy (rpfq_linear_f32); w_parts: float32 values whose absolute

@@ -286,11 +286,29 @@ class Attention(nn.Module):
     def _attend(self, qkv):
         b, n, c3 = qkv.shape
         c = c3 // 3
+        if self._attends_on_device(qkv):
+            from . import ops
+
+            return ops.attention(qkv, self.num_heads, self.scale)
         qkv = qkv.reshape(b, n, 3, self.num_heads, self.head_dim)
         qkv = qkv.permute(2, 0, 3, 1, 4)
         q, k, v = qkv.unbind(0)
         x = F.scaled_dot_product_attention(q, k, v, dropout_p=self.attn_drop.p if self.training else 0.0)
         return x.transpose(1, 2).reshape(b, n, c)
+
+    def _attends_on_device(self, qkv) -> bool:
+        """The attention kernel takes qkv, the output of a packed layer: 16-bit
+        heads of 64 values over at most 288 tokens (ops.attention), eval mode,
+        nothing recorded or transformed by autograd.  Longer sequences do not
+        fit the kernel's LDS and keep torch's."""
+        if not (FUSED_BLOCKS and qkv.is_cuda and not self.training and getattr(self.qkv, "use_packed", False)
+                and qkv.dtype in (torch.float16, torch.bfloat16) and self.head_dim == 64):
+            return False
+        if torch.is_grad_enabled() and qkv.requires_grad or torch._C._are_functorch_transforms_active():
+            return False
+        from . import ops
+
+        return qkv.shape[1] <= ops.ATTENTION_MAX_TOKENS and torch.autograd.forward_ad._current_level < 0
 
     def forward(self, x):
         return self.proj_drop(self.proj(self._mix(x)))

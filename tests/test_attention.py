@@ -1,0 +1,110 @@
+"""rpfq_attention against float64 softmax(q k^T scale) v.
+
+Bar: every probability and the output are rounded once to 16 bits (2^-11 or
+2^-8 relative) and the probabilities sum to 1, so an output is within
+2.5 u max|v| of the exact one; the float32 scores add at most
+2^-20 |q| |k| scale in the exponent.
+"""
+import ctypes
+
+import pytest
+import torch
+
+DEV = "cuda"
+
+
+def _exact(qkv, heads, scale):
+    b, n, c3 = qkv.shape
+    q, k, v = (t.contiguous() for t in qkv.double().reshape(b, n, 3, heads, 64).permute(2, 0, 3, 1, 4).unbind(0))
+    p = torch.softmax(q @ k.transpose(-1, -2).contiguous() * scale, -1)
+    return (p @ v).transpose(1, 2).reshape(b, n, c3 // 3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,n,heads", [(1, 1, 1), (2, 31, 2), (1, 32, 3), (3, 33, 1), (2, 64, 2), (2, 65, 1), (2, 128, 1),
+                                       (1, 129, 2), (1, 160, 1), (1, 161, 3), (2, 192, 1), (40, 197, 12), (1, 225, 2),
+                                       (1, 257, 16), (2, 288, 1)])
+def test_attention_matches_float64(b, n, heads, dtype):
+    from quant_models import ops
+
+    g = torch.Generator(device=DEV).manual_seed(n)
+    qkv = (torch.randn(b, n, 3 * heads * 64, device=DEV, generator=g) * 1.5).to(dtype)
+    out = ops.attention(qkv, heads, 0.125)
+    u = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    err = (out.double() - _exact(qkv, heads, 0.125)).abs().max()
+    assert out.shape == (b, n, heads * 64) and out.dtype == dtype
+    assert float(err) <= (2.5 * u + 2.0 ** -13) * float(qkv.abs().max())
+
+
+@pytest.mark.gpu
+def test_attention_extreme_scores_and_special_values():
+    """Scores far apart (one probability near 1), an unaligned view, and inf /
+    NaN in v reach the outputs of their head and image only."""
+    from quant_models import ops
+
+    g = torch.Generator(device=DEV).manual_seed(1)
+    n, heads = 197, 2
+    qkv = torch.randn(2, n, 3 * heads * 64, device=DEV, generator=g).half()
+    qkv[..., : 2 * heads * 64] *= 12
+    ref = _exact(qkv, heads, 0.125)
+    assert float((ops.attention(qkv, heads, 0.125).double() - ref).abs().max()) <= 2.5 * 2.0 ** -11 * float(qkv[..., 2 * heads * 64:].abs().max())
+    flat = torch.zeros(qkv.numel() + 1, device=DEV, dtype=torch.float16)
+    flat[1:] = qkv.reshape(-1)
+    assert torch.equal(ops.attention(flat[1:].view_as(qkv), heads, 0.125), ops.attention(qkv, heads, 0.125))
+    base = torch.randn(2, n, 3 * heads * 64, device=DEV, generator=g).half()
+    for value in (float("inf"), float("-inf"), float("nan")):
+        qkv = base.clone()
+        qkv[1, n - 1, 2 * heads * 64 + 5] = value  # v of the last token, image 1, head 0, value 5
+        out, clean = ops.attention(qkv, heads, 0.125), ops.attention(base, heads, 0.125)
+        hit = torch.zeros_like(out, dtype=torch.bool)
+        hit[1, :, 5] = True
+        assert torch.equal(out[~hit], clean[~hit])
+        got = out[hit]
+        assert bool(torch.isnan(got).all()) if value != value else bool((got == value).all())
+
+
+@pytest.mark.gpu
+def test_block_attention_route():
+    """The block's attention takes the kernel in inference only, and agrees
+    with torch's there."""
+    from quant_models import ops
+    from quant_models.inference import load_synthetic_codes, prepare_inference
+    from quant_models.quant_rpfq_vit import ComplexVisionTransformer
+
+    torch.manual_seed(0)
+    model = ComplexVisionTransformer(img_size=32, embed_dim=192, depth=1, num_heads=3, enable_act_quant=False,
+                                     enable_rotation=False)
+    load_synthetic_codes(model, 1)
+    attn = prepare_inference(model).blocks[0].attn
+    calls, real = [], ops.attention
+    ops.attention = lambda *a: calls.append(1) or real(*a)
+    try:
+        x = torch.randn(2, 50, 192, device=DEV).half()
+        with torch.no_grad():
+            y = attn(x)
+            qkv = attn.qkv(x)
+            q, k, v = qkv.reshape(2, 50, 3, 3, 64).permute(2, 0, 3, 1, 4).unbind(0)
+            ref = torch.nn.functional.scaled_dot_product_attention(q, k, v).transpose(1, 2).reshape(2, 50, 192)
+            assert torch.allclose(attn._attend(qkv), ref, rtol=2.0 ** -9, atol=2.0 ** -9 * float(v.abs().max()))
+            assert len(calls) == 2 and y.shape == x.shape
+            attn(torch.randn(1, 289, 192, device=DEV).half())  # too many tokens
+        for p in attn.parameters():
+            p.requires_grad_(False)
+        xg = x.clone().requires_grad_(True)
+        attn(xg).sum().backward()
+        assert xg.grad is not None and len(calls) == 2
+    finally:
+        ops.attention = real
+
+
+def test_attention_argument_errors():
+    from quant_models import _native as N
+
+    lib = N.load()
+    p = ctypes.c_void_p(4096)
+    assert lib.rpfq_attention(None, N.F16, 1, 8, 1, 64, 0.125, p, None) == 1
+    assert lib.rpfq_attention(p, N.F32, 1, 8, 1, 64, 0.125, p, None) == 5
+    for b, n, h, d in ((0, 8, 1, 64), (1, 289, 1, 64), (1, 8, 1, 32), (1, 8, 2048, 64)):
+        assert lib.rpfq_attention(p, N.F16, b, n, h, d, 0.125, p, None) == 2
+    assert lib.rpfq_attention(ctypes.c_void_p(4098), N.F16, 1, 8, 1, 64, 0.125, p, None) == 3
