@@ -542,6 +542,35 @@ size_t rpfq_quantize_workspace_bytes(const rpfq_quant_desc* desc);
 int rpfq_quantize_wide(const rpfq_quant_desc* desc, const float* weight, const float* rot, float* a_q,
                        float* scales, uint8_t* codes, void* work, size_t work_bytes, void* stream);
 
+/* Bytes of the workspace of rpfq_wide_linear_dense (transpose = 0: K' % 32 ==
+ * 0, N' even) or rpfq_wide_linear_grad_x_dense (transpose = 1: N' % 32 == 0,
+ * K' even); 0 where the layer is not taken. */
+size_t rpfq_wide_dense_bytes(const rpfq_wide_desc* desc, int transpose);
+
+/*
+ * rpfq_wide_linear_scaled on fp16 rows for many rows (M >= 128): the weight is
+ * decoded into `work` (fp16, the coefficients of rpfq_wide_decode with
+ * round_fp16) and contracted without a decode in the loop.  Bit-identical to
+ * the RPFQ_KERNEL_DMA launch of the same rows.  x [M, 2K'] fp16, row_scale as
+ * there (rows already prescaled, undone in the output) or NULL, flags 0 or
+ * RPFQ_FLAG_GELU (not with a residual); x, y, residual, row_scale 16-byte,
+ * packed and work 256-byte aligned.  Replaces F.linear(x, A_q, bias) of
+ * quant_i.py:554 at batch sizes where reading the weight costs nothing.
+ */
+int rpfq_wide_linear_dense(const rpfq_wide_desc* desc, const void* packed, size_t packed_bytes, const void* x, int64_t M,
+                           const float* row_scale, const float* bias, const void* residual, void* y, int y_dtype,
+                           int flags, void* work, size_t work_bytes, void* stream);
+
+/*
+ * rpfq_wide_linear_grad_x on fp16 grad_y rows for many rows (M >= 128), from
+ * the packed blob itself: the same coefficients, decoded into `work` as
+ * columns.  row_scale [M]: powers of two that the rows carry
+ * (rpfq_row_prescale), undone in the output, or NULL.
+ */
+int rpfq_wide_linear_grad_x_dense(const rpfq_wide_desc* desc, const void* packed, size_t packed_bytes, const void* grad_y,
+                                  int64_t M, const float* row_scale, void* grad_x, int grad_x_dtype, void* work,
+                                  size_t work_bytes, void* stream);
+
 /*
  * out = softmax(q k^T scale) v per image and head, without mask or dropout:
  * qkv [B, N, 3, H, D] (the qkv layer's output as it lies), out [B, N, H, D],

@@ -546,24 +546,6 @@ __global__ void __launch_bounds__(256) f32_special_gw_kernel(const float* gy, co
 // ---------------------------------------------------------------------------
 static int64_t up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
-// Rows per tile: 128, 96 or 64, the one whose tiles leave the fullest CU
-// with the least work (a launch of few tiles is as slow as the CU holding
-// one more than the others).
-static int f32_mb(int64_t M, int64_t N) {
-    const int64_t tn = (N + 255) / 256, cus = device_cus();
-    int best = 4;
-    int64_t cost = INT64_MAX;
-    for (int mb = 4; mb >= 2; --mb) {
-        const int64_t tiles = (M + 32 * mb - 1) / (32 * mb) * tn;
-        const int64_t c = (tiles + cus - 1) / cus * (8 * mb + (4 - mb));
-        if (c < cost) {
-            cost = c;
-            best = mb;
-        }
-    }
-    return best;
-}
-
 static int f32_splits(int64_t N, int64_t K, int64_t steps) {
     const int64_t tiles = ((N + 127) / 128) * ((K + 255) / 256), slots = 2 * (int64_t)device_cus();
     int best = 1;
@@ -651,7 +633,7 @@ static hipError_t f32_gemm_go(F32Args& a, hipStream_t s) {
 }
 
 static hipError_t f32_gemm(F32Args& a, hipStream_t s) {
-    const int mb = f32_mb(a.M, a.N);
+    const int mb = rows_per_tile(a.M, a.N);
     if (mb == 2) return f32_gemm_go<2>(a, s);
     if (mb == 3) return f32_gemm_go<3>(a, s);
     return f32_gemm_go<4>(a, s);

@@ -597,6 +597,61 @@ int rpfq_quantize_wide_noalloc(const rpfq_quant_desc* desc, const float* weight,
                       "rpfq_quantize_wide_noalloc");
 }
 
+// Shapes and operands the decoded-fragment kernels take (trans: the input
+// gradient).
+static int check_dense(const rpfq_wide_desc* desc, int trans, const void* packed, size_t packed_bytes, const void* x,
+                       int64_t M, const float* row_scale, const void* residual, const void* y, int y_dtype,
+                       const void* work, size_t work_bytes) {
+    if (!packed || !x || !y || !work) return fail(RPFQ_ERR_NULL, "packed/x/y/work must not be NULL");
+    if (!dtype_ok(y_dtype)) return fail(RPFQ_ERR_DTYPE, "unsupported dtype y=%d", y_dtype);
+    const size_t need = rpfq_wide_dense_bytes(desc, trans);
+    if (need == 0) return fail(RPFQ_ERR_SHAPE, "N'=%lld K'=%lld is not taken", (long long)desc->n_complex, (long long)desc->k_complex);
+    if (M < 128 || M > (int64_t)1 << 30) return fail(RPFQ_ERR_SHAPE, "M=%lld must be 128..2^30", (long long)M);
+    const rpfq::WideGeom g = rpfq::wide_geom(*desc);
+    if (packed_bytes < g.total_bytes)
+        return fail(RPFQ_ERR_SHAPE, "packed buffer holds %zu bytes, need %zu", packed_bytes, g.total_bytes);
+    if (work_bytes < need) return fail(RPFQ_ERR_SHAPE, "workspace holds %zu bytes, need %zu", work_bytes, need);
+    if (!aligned(packed, 256) || !aligned(work, 256) || !aligned(x, 16) || !aligned(y, 16) || !aligned(residual, 16) ||
+        !aligned(row_scale, 16))
+        return fail(RPFQ_ERR_ALIGN, "packed and work must be 256-byte, the other operands 16-byte aligned");
+    return RPFQ_OK;
+}
+
+size_t rpfq_wide_dense_bytes(const rpfq_wide_desc* desc, int transpose) {
+    if (check_desc(desc) != RPFQ_OK) return 0;
+    const rpfq::WideGeom g = rpfq::wide_geom(*desc);
+    // whole steps of the contraction, 4 outputs a store, 31-bit fragment offsets
+    if ((transpose ? g.N : g.K) % 32 != 0 || (transpose ? g.K : g.N) % 2 != 0) return 0;
+    const size_t b = rpfq::wide_dense_bytes(g, transpose ? 1 : 0);
+    return b < ((size_t)1 << 31) ? b : 0;
+}
+
+int rpfq_wide_linear_dense(const rpfq_wide_desc* desc, const void* packed, size_t packed_bytes, const void* x, int64_t M,
+                           const float* row_scale, const float* bias, const void* residual, void* y, int y_dtype,
+                           int flags, void* work, size_t work_bytes, void* stream) {
+    int rc = check_desc(desc);
+    if (rc) return rc;
+    if (flags & ~RPFQ_FLAG_GELU) return fail(RPFQ_ERR_VALUE, "flags=%d: only RPFQ_FLAG_GELU", flags);
+    if (flags && residual) return fail(RPFQ_ERR_VALUE, "RPFQ_FLAG_GELU is not defined with a residual");
+    if ((rc = check_dense(desc, 0, packed, packed_bytes, x, M, row_scale, residual, y, y_dtype, work, work_bytes))) return rc;
+    return hip_status(rpfq::launch_wide_dense(*desc, rpfq::wide_geom(*desc), packed, 0, x, M, row_scale, bias, residual, y,
+                                              y_dtype, flags ? 1 : 0, work, reinterpret_cast<hipStream_t>(stream)),
+                      "rpfq_wide_linear_dense");
+}
+
+int rpfq_wide_linear_grad_x_dense(const rpfq_wide_desc* desc, const void* packed, size_t packed_bytes, const void* grad_y,
+                                  int64_t M, const float* row_scale, void* grad_x, int grad_x_dtype, void* work,
+                                  size_t work_bytes, void* stream) {
+    int rc = check_desc(desc);
+    if (rc) return rc;
+    if ((rc = check_dense(desc, 1, packed, packed_bytes, grad_y, M, row_scale, nullptr, grad_x, grad_x_dtype, work,
+                          work_bytes)))
+        return rc;
+    return hip_status(rpfq::launch_wide_dense(*desc, rpfq::wide_geom(*desc), packed, 1, grad_y, M, row_scale, nullptr, nullptr,
+                                              grad_x, grad_x_dtype, 0, work, reinterpret_cast<hipStream_t>(stream)),
+                      "rpfq_wide_linear_grad_x_dense");
+}
+
 int rpfq_attention(const void* qkv, int dtype, int64_t B, int64_t N, int64_t H, int64_t D, float scale, void* out,
                    void* stream) {
     if (!qkv || !out) return fail(RPFQ_ERR_NULL, "qkv/out must not be NULL");

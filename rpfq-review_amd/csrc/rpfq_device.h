@@ -301,6 +301,15 @@ __device__ __forceinline__ int xcd_tile(int bid, int total) {
     return (xcd < r) ? xcd * (q + 1) + local : r * (q + 1) + (xcd - r) * q + local;
 }
 
+// Tile t of an order that walks `group` column tiles across all row tiles,
+// then the next `group`: a group's weights stay in L2 while the rows pass.
+__device__ __forceinline__ void group_tile(int t, int tiles_m, int tiles_n, int group, int& mt, int& nt) {
+    const int gi = t / (tiles_m * group), rem = t - gi * tiles_m * group;
+    const int wide = min(group, tiles_n - gi * group);
+    mt = rem / wide;
+    nt = gi * group + rem - mt * wide;
+}
+
 // Row i of the 32x32 MFMA accumulator element v held by lane group g (lane/32).
 __device__ __forceinline__ int acc_row(int v, int g) { return 8 * (v >> 2) + 4 * g + (v & 3); }
 // LDS activation row: 32 complex columns as (re, im) fp16 pairs = 128 B,

@@ -320,6 +320,38 @@ size_t quant_scratch_bytes();
 hipError_t quant_scratch_ptr(void** out);
 hipError_t launch_wide_decode(const rpfq_wide_desc& d, const WideGeom& g, const void* packed,
                               float* a, int round_fp16, hipStream_t s);
+// Rows per tile (32 MB, MB = 4, 3 or 2) of a GEMM with 256-column tiles, two
+// workgroups per CU: the one whose fullest CU has the least work.  128 rows
+// reuse each weight fragment most; a launch of few tiles is as slow as the CU
+// that holds one more than the others (12,608 x 768 outputs: 297 tiles of 128
+// rows on 256 CUs, 396 of 96).
+inline int rows_per_tile(int64_t M, int64_t N) {
+    const int64_t tn = (N + 255) / 256, cus = device_cus();
+    int best = 4;
+    int64_t cost = INT64_MAX;
+    for (int mb = 4; mb >= 2; --mb) {
+        const int64_t tiles = (M + 32 * mb - 1) / (32 * mb) * tn;
+        const int64_t c = (tiles + cus - 1) / cus * (8 * mb + (4 - mb));
+        if (c < cost) {
+            cost = c;
+            best = mb;
+        }
+    }
+    return best;
+}
+// Column tiles walked together (group_tile) where one holds `bytes` of
+// weights: about 1.6 MB of an XCD's 4 MB of L2, the rows taking the rest
+// (fp16 ViT-B layers at 50,432 rows: 4 tiles of 384 KB 6-8% faster than all
+// 9 or 12, 2 of them 2-3% slower than 4; all 3 of 1.5 MB 10% faster than 1).
+inline int tile_group(int tiles_n, int64_t bytes) {
+    const int64_t fit = 1600 * 1024 / bytes, g = fit < 3 ? 3 : fit;
+    return (int)(g < tiles_n ? g : tiles_n);
+}
+// the layer or its input gradient on decoded fragments (wide_dense.hip)
+size_t wide_dense_bytes(const WideGeom& g, int trans);
+hipError_t launch_wide_dense(const rpfq_wide_desc& d, const WideGeom& g, const void* packed, int trans, const void* x,
+                             int64_t M, const float* xs, const float* bias, const void* res, void* y, int ydt, int act,
+                             void* work, hipStream_t s);
 // attention of a qkv tensor (attention.hip): 64 values a head, N <= kAttnMaxN
 constexpr int kAttnMaxN = 288;
 hipError_t launch_attention(const void* qkv, int dt, int64_t B, int64_t N, int64_t H, float scale, void* out,

@@ -75,6 +75,9 @@ EXPORTED = (
     "rpfq_wide_linear_scaled",
     "rpfq_wide_mlp",
     "rpfq_layer_norm_wide_mlp",
+    "rpfq_wide_dense_bytes",
+    "rpfq_wide_linear_dense",
+    "rpfq_wide_linear_grad_x_dense",
     "rpfq_attention",
     "rpfq_linear_f32_workspace_bytes",
     "rpfq_linear_f32",
@@ -176,6 +179,10 @@ def load() -> ctypes.CDLL:
         lib.rpfq_wide_mlp.argtypes = [dp, vp, sz, dp, vp, sz, vp, i64, vp, vp, vp, vp, vp]
         lib.rpfq_layer_norm_wide_mlp.argtypes = [dp, vp, sz, dp, vp, sz, vp, i64, vp, vp, ctypes.c_float, vp, vp, vp,
                                                  vp]
+        lib.rpfq_wide_dense_bytes.argtypes = [dp, i32]
+        lib.rpfq_wide_dense_bytes.restype = sz
+        lib.rpfq_wide_linear_dense.argtypes = [dp, vp, sz, vp, i64, vp, vp, vp, vp, i32, i32, vp, sz, vp]
+        lib.rpfq_wide_linear_grad_x_dense.argtypes = [dp, vp, sz, vp, i64, vp, vp, i32, vp, sz, vp]
         lib.rpfq_attention.argtypes = [vp, i32, i64, i64, i64, i64, ctypes.c_float, vp, vp]
         lib.rpfq_linear_f32_workspace_bytes.argtypes = [i64, i64, i64, i32]
         lib.rpfq_linear_f32_workspace_bytes.restype = sz
@@ -183,7 +190,7 @@ def load() -> ctypes.CDLL:
         lib.rpfq_linear_f32_grad.argtypes = [vp, vp, vp, i64, i64, i64, vp, i32, vp, vp, vp, vp, sz, vp]
         for name in EXPORTED[2:]:
             if name not in ("rpfq_wide_packed_bytes", "rpfq_wide_adjoint_bytes", "rpfq_quantize_workspace_bytes",
-                            "rpfq_linear_f32_workspace_bytes"):
+                            "rpfq_linear_f32_workspace_bytes", "rpfq_wide_dense_bytes"):
                 getattr(lib, name).restype = i32
         _lib = lib
         return lib

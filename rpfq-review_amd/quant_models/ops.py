@@ -67,6 +67,10 @@ def prescale_rows(x2: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     return y, s
 
 
+# RPFQ_DENSE=0 keeps every launch on the kernels that decode in their loop.
+DENSE = __import__("os").environ.get("RPFQ_DENSE", "1") != "0"
+
+
 # Optional per-launch timing hook: when set, PackedWide.linear records HIP
 # events around each wide-linear launch on the launch stream and hands
 # (start_event, end_event, flops, algorithmic_bytes, shape) to the recorder.
@@ -322,15 +326,23 @@ class PackedWide:
                 x2, row_scale = prescale_rows(x2)
             else:
                 row_scale = row_scales(x2)
+        nwork = self._dense_bytes(m, x2, out_dtype, flags, r2 is not None)
         rec = _launch_recorder
         if rec is not None:
             ev0 = torch.cuda.Event(enable_timing=True)
             ev1 = torch.cuda.Event(enable_timing=True)
             ev0.record()
-        N.check("rpfq_wide_linear_scaled", lib.rpfq_wide_linear_scaled(
-            ctypes.byref(self.desc), self.blob.data_ptr(), self.blob.numel(), x2.data_ptr(), N.dtype_code(x2.dtype),
-            m, N.ptr(row_scale), N.ptr(bias), N.ptr(r2), y.data_ptr(), N.dtype_code(out_dtype), int(flags),
-            N.stream_of(x2)))
+        if nwork:
+            work = torch.empty(nwork, dtype=torch.uint8, device=x.device)
+            N.check("rpfq_wide_linear_dense", lib.rpfq_wide_linear_dense(
+                ctypes.byref(self.desc), self.blob.data_ptr(), self.blob.numel(), x2.data_ptr(), m, N.ptr(row_scale),
+                N.ptr(bias), N.ptr(r2), y.data_ptr(), N.dtype_code(out_dtype), int(flags), work.data_ptr(), nwork,
+                N.stream_of(x2)))
+        else:
+            N.check("rpfq_wide_linear_scaled", lib.rpfq_wide_linear_scaled(
+                ctypes.byref(self.desc), self.blob.data_ptr(), self.blob.numel(), x2.data_ptr(),
+                N.dtype_code(x2.dtype), m, N.ptr(row_scale), N.ptr(bias), N.ptr(r2), y.data_ptr(),
+                N.dtype_code(out_dtype), int(flags), N.stream_of(x2)))
         if rec is not None:
             ev1.record()
             nbytes = wide_bytes(m, self.n_complex, self.k_complex, x2.element_size(), y.element_size(),
@@ -338,10 +350,41 @@ class PackedWide:
             if residual is not None:
                 nbytes += m * self.out_features * y.element_size()
             # the device kernel (a fused GELU is a separate instantiation)
-            kern = N.KERNEL_NAMES.get(self.kernel_for(m, x2.dtype, out_dtype, flags), "?")
+            kern = "rpfq::wide_dense_kernel" if nwork else \
+                N.KERNEL_NAMES.get(self.kernel_for(m, x2.dtype, out_dtype, flags), "?")
             rec(ev0, ev1, wide_flops(m, self.n_complex, self.k_complex), nbytes,
                 (m, self.n_complex, self.k_complex, kern + ("+gelu" if flags & N.FLAG_GELU else "")))
         return y.reshape(*lead, self.out_features)
+
+    def _dense_bytes(self, m: int, x2: torch.Tensor, out_dtype: torch.dtype, flags: int, residual: bool) -> int:
+        """Workspace of rpfq_wide_linear_dense where linear() takes it, else 0:
+        fp16 rows that the DMA kernel would take (the results are the same
+        bits), where decoding the weight first (~5 us) measured faster.
+        DMA kernel -> decoded, MI355X, us: the fused GELU (its VALU work no
+        longer competes with the decode's) 50,432 rows of ViT-B fc1 360 ->
+        330, 6,304 rows 55 -> 53, but 1,576 rows of ViT-L 30 -> 34; N' % 8 !=
+        0 (16-byte stores instead of single values) 3,152 rows, 500 x 384 27
+        -> 16; float32 outputs (whole-line stores) with a residual 12,608
+        rows of proj 73 -> 42, without 12,608 rows of fc1 96 -> 90 but 3,152
+        of qkv 29 -> 34; long K' on few 128-row tiles (64- and 96-row tiles
+        fill the chip) 12,608 rows of fc2 93 -> 76, 25,216 147 -> 143.
+        Everything else is within 4% either way, power-limited."""
+        ops = wide_flops(m, self.n_complex, self.k_complex)
+        tiles = -(-m // 128) * -(-self.n_complex // 128)
+        if flags & N.FLAG_GELU:
+            least = 2.9e10
+        elif out_dtype == torch.float32:
+            least = 1.5e9 if residual else 4e10
+        else:
+            least = math.inf
+        if self.n_complex % 8:
+            least = min(least, 1.5e9)
+        if self.k_complex >= 1024 and tiles <= 512:
+            least = min(least, 5e9)
+        if (not DENSE or ops < least or m < 128 or x2.dtype != torch.float16 or flags & ~N.FLAG_GELU
+                or self.kernel_for(m, torch.float16, out_dtype, flags) != N.KERNEL_DMA):
+            return 0
+        return N.load().rpfq_wide_dense_bytes(ctypes.byref(self.desc), 0)
 
     def ln_fusable(self, m: int, x_dtype: torch.dtype, y_dtype: torch.dtype | None = None) -> bool:
         """Whether layer_norm_linear() fuses the LayerNorm for m rows
@@ -477,11 +520,41 @@ class PackedWide:
         gx = torch.empty(m, self.in_features, dtype=out_dtype, device=grad_y.device)
         if m == 0:
             return gx.reshape(*lead, self.in_features)
+        nwork = self._grad_dense_bytes(m, g2)
+        if nwork:
+            row_scale = None
+            if g2.dtype != torch.float16:
+                g2, row_scale = prescale_rows(g2)
+            work = torch.empty(nwork, dtype=torch.uint8, device=g2.device)
+            N.check("rpfq_wide_linear_grad_x_dense", N.load().rpfq_wide_linear_grad_x_dense(
+                ctypes.byref(self.desc), self.blob.data_ptr(), self.blob.numel(), g2.data_ptr(), m, N.ptr(row_scale),
+                gx.data_ptr(), N.dtype_code(out_dtype), work.data_ptr(), nwork, N.stream_of(g2)))
+            return gx.reshape(*lead, self.in_features)
         adj = self.adjoint()
         N.check("rpfq_wide_linear_grad_x", N.load().rpfq_wide_linear_grad_x(
             ctypes.byref(self.desc), adj.data_ptr(), adj.numel(), g2.data_ptr(), N.dtype_code(g2.dtype), m,
             gx.data_ptr(), N.dtype_code(out_dtype), N.stream_of(g2)))
         return gx.reshape(*lead, self.in_features)
+
+    def _grad_dense_bytes(self, m: int, g2: torch.Tensor) -> int:
+        """Workspace of rpfq_wide_linear_grad_x_dense where grad_x() takes it,
+        else 0 (the adjoint kernel): contractions long enough to cover the
+        decode and, for bf16 / float32 rows, their prescale pass.  Adjoint
+        kernel -> decoded, MI355X, us: fp16 12,608 rows of fc1 100 -> 69, 512
+        rows 69 -> 38, 12,608 rows of 288 x 96 18 -> 14 but 96 x 96 11 -> 14;
+        bf16 fc1 135 -> 90, 384 x 384 at 512 rows 29 -> 23 but 288 x 96 at
+        12,608 rows 23 -> 26; float32 fc1 156 -> 106, 1152 x 384 at 512 rows
+        50 -> 35, 384 x 384 at 12,608 rows 48 -> 37 but at 3,152 22 -> 23."""
+        n, ops = self.n_complex, wide_flops(m, self.n_complex, self.k_complex)
+        if g2.dtype == torch.float16:
+            pays = n >= 256
+        elif g2.dtype == torch.bfloat16:
+            pays = n >= 384
+        else:
+            pays = n >= 1024 or (n >= 384 and ops >= 5e9)
+        if not DENSE or not pays or ops < 5e8 or m < 128 or (g2.dtype != torch.float16 and 2 * n > 4096):
+            return 0
+        return N.load().rpfq_wide_dense_bytes(ctypes.byref(self.desc), 1)
 
     def decode(self, round_fp16: bool = False) -> torch.Tensor:
         """Fused float32 weight A_q [2N', 2K'] (quant_i.py:534-544 layout)."""
