@@ -174,8 +174,8 @@ struct F32Args {
     float* y;             // [M, N]
     int64_t M;
     int N, KS;            // outputs, 32-column steps
-    int rows32;           // 32-row tiles of wf (a multiple of 8)
-    int tiles_m, tiles_n;
+    int wf_bytes;
+    int tiles_m, tiles_n, group;
 };
 
 // Workgroup = 4 waves, tile = BM rows x 256 outputs, wave w the outputs
@@ -252,7 +252,10 @@ __global__ void __launch_bounds__(256, 2) f32_gemm_kernel(F32Args a) {
     const uint32_t v0 = par ? voff[1] : voff[0], v1 = par ? voff[0] : voff[1];
     const uint32_t lds_x = lds_addr(smem) + RPW * wave * 128;
     const char* xw = nullptr;
-    const uint4* wp[2] = {nullptr, nullptr};
+    // buffer loads: one resource and a scalar offset per load
+    const __amdgpu_buffer_rsrc_t wf = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.wf), 0, a.wf_bytes, 0x00027000);
+    const uint32_t wv = lane * 16;
+    uint32_t wo[2] = {0, 0};
     auto issue_x = [&](int ks, int st) {
         const char* src = xw + ks * 128;
 #pragma unroll
@@ -262,8 +265,8 @@ __global__ void __launch_bounds__(256, 2) f32_gemm_kernel(F32Args a) {
     auto load_w = [&](int t, uint4 (&f)[2][2]) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            f[j][0] = wp[j][(int64_t)t * 128 + lane];
-            f[j][1] = wp[j][(int64_t)t * 128 + 64 + lane];
+            f[j][0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wf, wv, wo[j] + t * 2048, 0));
+            f[j][1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wf, wv, wo[j] + t * 2048 + 1024, 0));
         }
     };
     uint32_t aoff[2][2];  // [h, l][substep]: chunk 4 p + 2 s + g of row r
@@ -273,13 +276,13 @@ __global__ void __launch_bounds__(256, 2) f32_gemm_kernel(F32Args a) {
         for (int s = 0; s < 2; ++s) aoff[p][s] = lds_addr(smem) + r * 128 + (((4 * p + 2 * s + g) ^ ((r >> 1) & 7)) * 16);
 
     const int total = a.tiles_m * a.tiles_n;
+    int mt = 0, ntl = 0;
     auto set_tile = [&](int vb) {
-        const int t = xcd_tile(vb, total);
-        const int mt = t / a.tiles_n, ntl = t - mt * a.tiles_n;
+        group_tile(xcd_tile(vb, total), a.tiles_m, a.tiles_n, a.group, mt, ntl);
         xw = a.xp + ((int64_t)mt * BM + RPW * wave) * ld;
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-            wp[j] = reinterpret_cast<const uint4*>(a.wf) + (int64_t)((ntl * 4 + wave) * 2 + j) * kt * 128;
+            wo[j] = (uint32_t)__builtin_amdgcn_readfirstlane(((ntl * 4 + wave) * 2 + j) * kt * 2048);
     };
     uint4 w0[2][2], w1[2][2], w2[2][2];
     const int we = f32_scale_exp(a.wscale[0]);
@@ -292,8 +295,7 @@ __global__ void __launch_bounds__(256, 2) f32_gemm_kernel(F32Args a) {
         load_w(kt > 2 ? 2 : 1, w2);
     }
     for (int vb = blockIdx.x; vb < total; vb += gridDim.x) {
-        const int tile = xcd_tile(vb, total);
-        const int mt = tile / a.tiles_n, ntl = tile - mt * a.tiles_n;
+        const int64_t mrow = (int64_t)mt * BM, n0 = (int64_t)ntl * 256 + 64 * wave;
         floatx16 acc[2][MB];
 #pragma unroll
         for (int i = 0; i < MB; ++i) acc[0][i] = acc[1][i] = floatx16{0};
@@ -356,10 +358,9 @@ __global__ void __launch_bounds__(256, 2) f32_gemm_kernel(F32Args a) {
             load_w(1, w1);
             load_w(kt > 2 ? 2 : 1, w2);
         }
-        const int64_t n0 = (int64_t)ntl * 256 + 64 * wave;
 #pragma unroll
         for (int i = 0; i < MB; ++i) {
-            const int64_t m = (int64_t)mt * BM + 32 * i;
+            const int64_t m = mrow + 32 * i;
             const float s = a.scale[m + r < a.M ? m + r : a.M - 1];
             f32_store_block(epi, acc[0][i], acc[1][i], -f32_scale_exp(s) - we, a.bias, a.y, m, a.M, n0, a.N, lane);
         }
@@ -627,6 +628,7 @@ static hipError_t f32_gemm_go(F32Args& a, hipStream_t s) {
     if (e != hipSuccess) return e;
     a.tiles_m = (int)((a.M + 32 * MB - 1) / (32 * MB));
     a.tiles_n = (a.N + 255) / 256;
+    a.group = tile_group(a.tiles_n, (int64_t)a.KS * 32768);
     const int total = a.tiles_m * a.tiles_n, slots = 2 * device_cus();
     hipLaunchKernelGGL((f32_gemm_kernel<MB>), dim3(total < slots ? total : slots), dim3(256), f32_lds<MB>(), s, a);
     return hipGetLastError();
@@ -662,6 +664,7 @@ hipError_t launch_linear_f32(const float* x, const float* w, const float* bias, 
     a.M = M;
     a.N = (int)N;
     a.KS = (int)(p.Kp / 32);
+    a.wf_bytes = (int)(p.fwd_bytes - p.w_at);
     RPFQ_TRY(f32_gemm(a, s));
     hipLaunchKernelGGL(f32_special_rows_kernel, dim3(256), dim3(256), 0, s, x, w, bias, y, M, (int)N, (int)K, K,
                        (int64_t)1, xscale, wscale);
@@ -688,6 +691,7 @@ hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* 
         a.M = M;
         a.N = (int)K;
         a.KS = (int)(p.Np / 32);
+        a.wf_bytes = (int)(p.gs_at - p.bw_at);
         RPFQ_TRY(f32_gemm(a, s));
         hipLaunchKernelGGL(f32_special_rows_kernel, dim3(256), dim3(256), 0, s, gy, w, (const float*)nullptr, gx, M,
                            (int)K, (int)N, (int64_t)1, K, gscale, wscale);
