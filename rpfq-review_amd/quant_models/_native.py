@@ -212,9 +212,32 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int | None:
-    """Raw hipStream_t of torch's current stream on t's device."""
+    """Raw hipStream_t of torch's current stream on t's device (without the
+    Stream object around it: 0.1 against 1.8 us)."""
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device()) or None
     return torch.cuda.current_stream(t.device).cuda_stream or None
+
+
+_host = None
+
+
+def host():
+    """The native host path of short launches (csrc/host.cpp), or None where
+    it was not built: callers then go through ctypes."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError:
+            module = False
+        _host = module
+    return _host or None
 
 
 def require_device(*tensors: torch.Tensor) -> None:

@@ -288,11 +288,17 @@ class PackedWide:
         row_scales() computes it, or computed here) so any magnitude keeps
         its relative accuracy through the fp16 operands
         (rpfq_wide_linear_scaled)."""
-        N.require_device(x, bias, residual, row_scale)
         if gelu:
             if residual is not None:
                 raise ValueError("gelu and residual cannot be fused together")
             flags = int(flags) | N.FLAG_GELU
+        host = N.host()
+        if host is not None and row_scale is None and _launch_recorder is None:
+            y = host.linear(ctypes.addressof(self.desc), self.blob, x, bias, residual, out_dtype, int(flags),
+                            int(RANGE_GUARD) + 2 * int(PRESCALE_ROWS))
+            if y is not None:
+                return y
+        N.require_device(x, bias, residual, row_scale)
         if x.shape[-1] != self.in_features:
             raise ValueError(f"expected last dim {self.in_features}, got {x.shape[-1]}")
         lead = x.shape[:-1]
@@ -403,6 +409,12 @@ class PackedWide:
         features runs in the streaming kernel's prologue, its output rounded
         to x's dtype as layer_norm() rounds it.  Only where ln_fusable();
         gelu as in linear()."""
+        host = N.host()
+        if host is not None:
+            y = host.layer_norm_linear(ctypes.addressof(self.desc), self.blob, x, ln_weight, ln_bias, float(eps), bias,
+                                       out_dtype, N.FLAG_GELU if gelu else 0)
+            if y is not None:
+                return y
         N.require_device(x, ln_weight, ln_bias, bias)
         if x.shape[-1] != self.in_features:
             raise ValueError(f"expected last dim {self.in_features}, got {x.shape[-1]}")
@@ -432,6 +444,12 @@ class PackedWide:
         the rows as act_quant() / layer_norm(act_bits=bits) does, bit for bit.
         residual ([..., 2N'] of out_dtype): added in the store.  Only where
         ln_fusable(); gelu as in linear() (not with a residual)."""
+        host = N.host()
+        if host is not None and layer_norm is None:
+            y = host.act_quant_linear(ctypes.addressof(self.desc), self.blob, x, int(bits), bias, residual, out_dtype,
+                                      N.FLAG_GELU if gelu else 0)
+            if y is not None:
+                return y
         N.require_device(x, bias, residual)
         if x.shape[-1] != self.in_features:
             raise ValueError(f"expected last dim {self.in_features}, got {x.shape[-1]}")
@@ -710,6 +728,11 @@ ATTENTION_MAX_TOKENS = 288
 def attention(qkv: torch.Tensor, num_heads: int, scale: float) -> torch.Tensor:
     """softmax(q k^T scale) v [B, N, C] of a qkv tensor [B, N, 3 C] (fp16 or
     bf16, heads of 64 values, N <= ATTENTION_MAX_TOKENS; rpfq_attention)."""
+    host = N.host()
+    if host is not None:
+        out = host.attention(qkv, num_heads, float(scale))
+        if out is not None:
+            return out
     N.require_device(qkv)
     b, n, c3 = qkv.shape
     c = c3 // 3

@@ -740,7 +740,7 @@ class QATLinearComplexPhase(nn.Linear):
             if self.act_quantizer is not None and not prequantized:
                 x = _HipActQuantSTE.apply(x, self.act_quantizer.num_bits)
             return _PackedLinearFn.apply(x, self.bias, pw)
-        bias = None if self.bias is None else self.bias.detach()
+        bias = self.bias  # nothing is recorded here
         if self.act_quantizer is not None and not prequantized:
             if self._aq_fusable(pw, x):  # act quant in the layer's own launch
                 return pw.act_quant_linear(x, self.act_quantizer.num_bits, bias, out_dtype=x.dtype)
@@ -799,7 +799,7 @@ class QATLinearComplexPhase(nn.Linear):
             from . import ops
 
             pw = self.packed(x.device)
-            bias = None if self.bias is None else self.bias.detach()
+            bias = self.bias  # nothing is recorded here
             if self.act_quantizer is not None and not prequantized:
                 if self._aq_fusable(pw, x):  # act quant, layer and GELU in one launch
                     return pw.act_quant_linear(x, self.act_quantizer.num_bits, bias, out_dtype=x.dtype, gelu=True)
@@ -836,7 +836,7 @@ class QATLinearComplexPhase(nn.Linear):
         m = x.numel() // x.shape[-1]
         if not hasattr(pw, "ln_fusable") or m == 0:
             return None
-        bias = None if self.bias is None else self.bias.detach()
+        bias = self.bias  # nothing is recorded here
         if pw.ln_fusable(m, x.dtype):
             return pw.layer_norm_linear(x, ln_weight, ln_bias, eps, bias, out_dtype=x.dtype, gelu=gelu)
         from . import _native as N
@@ -858,7 +858,7 @@ class QATLinearComplexPhase(nn.Linear):
             from . import ops
 
             pw = self.packed(x.device)
-            bias = None if self.bias is None else self.bias.detach()
+            bias = self.bias  # nothing is recorded here
             if self.act_quantizer is not None and not prequantized:
                 if self._aq_fusable(pw, x):  # act quant, layer and residual add in one launch
                     return pw.act_quant_linear(x, self.act_quantizer.num_bits, bias, out_dtype=x.dtype,

@@ -1,0 +1,110 @@
+"""The native host path of short launches (csrc/host.cpp) against the Python
+path it stands in front of: the same bits, and the same calls refused."""
+import pytest
+import torch
+
+DEV = "cuda"
+DTYPES = [torch.float16, torch.bfloat16, torch.float32]
+
+
+def _layer(n, k, seed=0):
+    from quant_models import ops
+
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    planes = [torch.randint(0, 256, (n, k // 4), generator=g, device=DEV, dtype=torch.uint8) for _ in range(4)]
+    scale = [0.01 + 0.03 * torch.rand(n, 1, generator=g, device=DEV) for _ in range(4)]
+    return ops.PackedWide.from_planes(planes, scale, scale, n, k), g
+
+
+def _both(monkeypatch, f):
+    """f() on the native path and on the Python path."""
+    from quant_models import _native as N
+
+    assert N.host() is not None
+    native = f()
+    with monkeypatch.context() as m:
+        m.setattr(N, "_host", False)
+        return native, f()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [(1, 500, 384), (8, 48, 16), (17, 96, 96), (197, 384, 384), (600, 100, 64)])
+def test_native_linear_equals_python_path(m, n, k, dtype, monkeypatch):
+    pw, g = _layer(n, k)
+    bias = torch.randn(2 * n, device=DEV, generator=g)
+    ln = [torch.randn(2 * k, device=DEV, generator=g) for _ in range(2)]
+    x = torch.randn(1, m, 2 * k, device=DEV, generator=g).to(dtype)
+    for out in DTYPES:
+        r = torch.randn(1, m, 2 * n, device=DEV, generator=g).to(out)
+        for kw in ({}, {"residual": r}, {"gelu": True}):
+            for b in (None, bias):
+                a, c = _both(monkeypatch, lambda: pw.linear(x, b, out_dtype=out, **kw))
+                assert a.shape == (1, m, 2 * n) and torch.equal(a, c)
+    if pw.ln_fusable(m, dtype):
+        assert torch.equal(*_both(monkeypatch, lambda: pw.layer_norm_linear(x, *ln, 1e-5, bias)))
+        assert torch.equal(*_both(monkeypatch, lambda: pw.act_quant_linear(x, 4, bias)))
+
+
+@pytest.mark.gpu
+def test_native_path_leaves_other_calls_to_python(monkeypatch):
+    """Strided, offset and other-dtype operands, empty inputs, and errors."""
+    from quant_models import _native as N
+    from quant_models import ops
+
+    pw, g = _layer(48, 32)
+    x = torch.randn(6, 64, device=DEV, generator=g).half()
+    bias = torch.randn(96, device=DEV, generator=g)
+    forms = [x.t().contiguous().t(), torch.cat((x, x), 1)[:, 64:], torch.zeros(385, device=DEV, dtype=torch.half)[1:].view(6, 64).copy_(x)]
+    for f in forms:
+        assert torch.equal(pw.linear(f, bias), pw.linear(x, bias))
+    assert torch.equal(pw.linear(x, bias.double()), pw.linear(x, bias))
+    assert torch.equal(pw.linear(x, bias, residual=torch.ones(6, 96, device=DEV)), pw.linear(x, bias, residual=torch.ones(6, 96, device=DEV).half()))
+    assert pw.linear(x[:0], bias).shape == (0, 96)
+    for bad in (lambda: pw.linear(x[:, :32]), lambda: pw.linear(x.cpu()), lambda: pw.linear(x, residual=x),
+                lambda: pw.linear(x, residual=torch.ones(6, 96, device=DEV).half(), gelu=True)):
+        with pytest.raises(ValueError):
+            bad()
+    with pytest.raises(TypeError):
+        pw.linear(x.double())
+    with pytest.raises(N.RPFQError):
+        pw.linear(x, flags=N.FLAG_STREAM | N.FLAG_NO_STREAM)
+    qkv = torch.randn(2, 20, 3 * 128, device=DEV, generator=g).half()
+    assert torch.equal(*_both(monkeypatch, lambda: ops.attention(qkv, 2, 0.125)))
+    with pytest.raises(N.RPFQError):
+        ops.attention(qkv, 4, 0.125)
+
+
+@pytest.mark.gpu
+def test_native_path_runs_on_the_current_stream():
+    pw, g = _layer(96, 96)
+    x = torch.randn(4, 192, device=DEV, generator=g).half()
+    ref = pw.linear(x)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        z = x.clone()
+        for _ in range(50):
+            z = z + 0
+        y = pw.linear(z)
+    s.synchronize()
+    assert torch.equal(y, ref)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = pw.linear(x)
+    for _ in range(3):
+        x.mul_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, pw.linear(x))
+
+
+def test_native_path_takes_device_tensors_only():
+    from quant_models import _native as N
+
+    host = N.host()
+    assert host is not None, "quant_models/_host.so is not built"
+    t = torch.zeros(4, 64, dtype=torch.half)
+    assert host.linear(0, t, t, None, None, None, 0, 3) is None
+    assert host.linear(t) is None
+    assert host.attention(t, 1, 0.125) is None
