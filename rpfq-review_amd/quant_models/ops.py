@@ -745,6 +745,19 @@ def attention(qkv: torch.Tensor, num_heads: int, scale: float) -> torch.Tensor:
     return out
 
 
+def _require_f32(m: int, n: int, k: int, **operands: torch.Tensor) -> None:
+    """The shapes the float32 kernels index by, contiguous on one device."""
+    shapes = {"x": (m, k), "w": (n, k), "grad_y": (m, n), "bias": (n,), "x_scale": (m,)}
+    device = operands["x"].device
+    for name, t in operands.items():
+        if t is None:
+            continue
+        if t.dtype != torch.float32 or t.device != device or not t.is_contiguous():
+            raise ValueError(f"{name} must be a contiguous float32 tensor on {device}")
+        if name in shapes and tuple(t.shape) != shapes[name]:
+            raise ValueError(f"{name} is {tuple(t.shape)}, expected {shapes[name]}")
+
+
 def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, w_parts: torch.Tensor):
     """(y, x_scale): y = x w^T + bias on contiguous float32 [M, K], [N, K] at
     float32 accuracy (rpfq_linear_f32); w_parts: float32 values whose absolute
@@ -752,6 +765,7 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, w_pa
     N.require_device(x, w, bias, w_parts)
     m, k = x.shape
     n = w.shape[0]
+    _require_f32(m, n, k, x=x, w=w, bias=bias, w_parts=w_parts)
     lib = N.load()
     nbytes = lib.rpfq_linear_f32_workspace_bytes(m, n, k, 0)
     y = torch.empty(m, n, dtype=torch.float32, device=x.device)
@@ -770,6 +784,7 @@ def linear_f32_grad(grad_y: torch.Tensor, x: torch.Tensor, w: torch.Tensor, w_pa
     N.require_device(grad_y, x, w, w_parts, x_scale)
     m, k = x.shape
     n = w.shape[0]
+    _require_f32(m, n, k, grad_y=grad_y, x=x, w=w, w_parts=w_parts, x_scale=x_scale)
     lib = N.load()
     nbytes = lib.rpfq_linear_f32_workspace_bytes(m, n, k, 1)
     gx = torch.empty_like(x) if want_x else None

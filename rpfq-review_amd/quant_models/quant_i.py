@@ -520,6 +520,7 @@ def _split_linear_pays(x: torch.Tensor, w: torch.Tensor, bias) -> bool:
     """Whether float32 x and A_q take _SplitLinearFn: shapes the kernels hold
     (rpfq_linear_f32) and enough work to cover the operand splits, and none of
     the transforms that an autograd function without their rules refuses.
+    Operands that do not fit each other are left to F.linear, which says so.
     MI355X, forward + backward against the float32 library GEMMs, us: 12,608
     rows, 3072 x 768 (59 GFLOP a product) 596 against 1,492; 768 x 768 (15)
     235 against 452; 3,152 rows, 1000 x 768 (4.8) 130 against 190; 1,576 rows,
@@ -527,6 +528,10 @@ def _split_linear_pays(x: torch.Tensor, w: torch.Tensor, bias) -> bool:
     115."""
     n, k = w.shape
     m = x.numel() // k
+    if x.dim() == 0 or x.shape[-1] != k or x.device != w.device:
+        return False
+    if bias is not None and not (bias.shape == (n,) and bias.device == w.device and bias.is_contiguous()):
+        return False
     if not (x.is_cuda and x.dtype == w.dtype == torch.float32 and (bias is None or bias.dtype == torch.float32)
             and n % 8 == 0 and k % 8 == 0 and n <= 4096 and k <= 4096 and m <= 1 << 24
             and w.is_contiguous() and w.data_ptr() % 16 == 0 and m >= 1024 and 2 * m * n * k >= SPLIT_LINEAR_MIN):

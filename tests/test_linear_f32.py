@@ -159,6 +159,29 @@ def test_training_layer_double_backward_and_forward_mode():
     assert torch.allclose(ty, t @ a.t(), rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.gpu
+def test_operands_that_do_not_fit_are_refused():
+    """By F.linear's own error from the layer, by the host checks below it."""
+    from quant_models import ops
+
+    layer = _layer("complex_phase_v2", 0, False)
+    for shape in ((4096, 1016), (4096, 2048)):
+        with pytest.raises(RuntimeError):
+            layer(torch.randn(*shape, device=DEV))
+    layer.bias = torch.nn.Parameter(torch.zeros(1528, device=DEV))
+    with pytest.raises(RuntimeError):
+        layer(torch.randn(4096, 1024, device=DEV))
+    x, w, b, gy = _inputs(64, 40, 48)
+    parts = w.abs().max().reshape(1)
+    y, scale = ops.linear_f32(x, w, b, parts)
+    for args in ((x[:, :40], w, b), (x, w, b[:32]), (x.half(), w, b), (x, w.t().contiguous().t(), b)):
+        with pytest.raises(ValueError):
+            ops.linear_f32(*args, parts)
+    for args in ((gy[:32], x), (gy, x[:, :40]), (gy, x.half()), (gy.t().contiguous().t(), x)):
+        with pytest.raises(ValueError):
+            ops.linear_f32_grad(*args, w, parts, scale)
+
+
 def test_linear_f32_argument_errors():
     """Reported on the host, without a GPU."""
     from quant_models import _native as N
