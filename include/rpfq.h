@@ -576,7 +576,7 @@ int rpfq_wide_linear_grad_x_dense(const rpfq_wide_desc* desc, const void* packed
  * qkv [B, N, 3, H, D] (the qkv layer's output as it lies), out [B, N, H, D],
  * both of dtype (RPFQ_F16 or RPFQ_BF16), 16-byte aligned; D = 64, N <= 288.
  * Scores, softmax and outputs in float32, probabilities rounded to dtype for
- * their product with v.  Replaces the attention between qkv and proj of a
+ * their product with v; scale positive and finite.  Replaces the attention between qkv and proj of a
  * ViT block (RPFQ-ViTApple/scripts/audit_rpfq_vit_ios_parity.py:523-545).
  */
 int rpfq_attention(const void* qkv, int dtype, int64_t B, int64_t N, int64_t H, int64_t D, float scale, void* out,

@@ -657,6 +657,8 @@ int rpfq_attention(const void* qkv, int dtype, int64_t B, int64_t N, int64_t H, 
     if (!qkv || !out) return fail(RPFQ_ERR_NULL, "qkv/out must not be NULL");
     if (dtype != RPFQ_F16 && dtype != RPFQ_BF16) return fail(RPFQ_ERR_DTYPE, "unsupported dtype %d", dtype);
     if (B <= 0 || N <= 0 || H <= 0) return fail(RPFQ_ERR_SHAPE, "B=%lld N=%lld H=%lld must be positive", (long long)B, (long long)N, (long long)H);
+    // the row maximum is taken before the scale
+    if (!(scale > 0.0f && scale < INFINITY)) return fail(RPFQ_ERR_VALUE, "scale=%g must be positive and finite", (double)scale);
     if (D != 64 || N > rpfq::kAttnMaxN || H > 1024 || B > (1LL << 24) / H)
         return fail(RPFQ_ERR_SHAPE, "takes heads of 64 values, N <= %d, H <= 1024, B H <= 2^24 (N=%lld H=%lld D=%lld)",
                     rpfq::kAttnMaxN, (long long)N, (long long)H, (long long)D);

@@ -299,12 +299,14 @@ class Attention(nn.Module):
     def _attends_on_device(self, qkv) -> bool:
         """The attention kernel takes qkv, the output of a packed layer: 16-bit
         heads of 64 values over at most 288 tokens (ops.attention), eval mode,
-        nothing recorded or transformed by autograd.  Longer sequences do not
-        fit the kernel's LDS and keep torch's."""
+        nothing recorded or transformed by autograd, and no autocast to another
+        dtype.  Longer sequences do not fit the kernel's LDS and keep torch's."""
         if not (FUSED_BLOCKS and qkv.is_cuda and not self.training and getattr(self.qkv, "use_packed", False)
                 and qkv.dtype in (torch.float16, torch.bfloat16) and self.head_dim == 64):
             return False
         if torch.is_grad_enabled() and qkv.requires_grad or torch._C._are_functorch_transforms_active():
+            return False
+        if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != qkv.dtype:
             return False
         from . import ops
 

@@ -89,6 +89,9 @@ def test_block_attention_route():
             assert torch.allclose(attn._attend(qkv), ref, rtol=2.0 ** -9, atol=2.0 ** -9 * float(v.abs().max()))
             assert len(calls) == 2 and y.shape == x.shape
             attn(torch.randn(1, 289, 192, device=DEV).half())  # too many tokens
+            with torch.autocast("cuda", dtype=torch.bfloat16):  # torch's runs in the autocast dtype
+                assert attn._attend(qkv).dtype == torch.bfloat16
+            assert len(calls) == 2
         for p in attn.parameters():
             p.requires_grad_(False)
         xg = x.clone().requires_grad_(True)
@@ -108,3 +111,5 @@ def test_attention_argument_errors():
     for b, n, h, d in ((0, 8, 1, 64), (1, 289, 1, 64), (1, 8, 1, 32), (1, 8, 2048, 64)):
         assert lib.rpfq_attention(p, N.F16, b, n, h, d, 0.125, p, None) == 2
     assert lib.rpfq_attention(ctypes.c_void_p(4098), N.F16, 1, 8, 1, 64, 0.125, p, None) == 3
+    for scale in (0.0, -0.125, float("nan"), float("inf")):
+        assert lib.rpfq_attention(p, N.F16, 1, 8, 1, 64, scale, p, None) == 6
