@@ -446,6 +446,15 @@ int rpfq_layer_norm_prescaled(const void* x, int x_dtype, int64_t M, int64_t C, 
 int rpfq_row_prescale(const void* x, int x_dtype, int64_t M, int64_t C, void* y, float* row_scale, void* stream);
 
 /*
+ * rpfq_act_quant (y of x's dtype) followed by rpfq_row_prescale in one pass:
+ * the fp16 rows and scales are the same bits.  bits 2..16; C a multiple of 16
+ * up to 4096; the rest as rpfq_row_prescale.  Replaces the activation
+ * quantization of quant_i.py:438-455 in front of a DMA-kernel launch.
+ */
+int rpfq_act_quant_prescaled(const void* x, int x_dtype, int64_t M, int64_t C, int bits, void* y, float* row_scale,
+                             void* stream);
+
+/*
  * rpfq_layer_norm followed by the activation fake quantization of
  * rpfq_act_quant on its output, in one pass over the rows: the float32
  * LayerNorm output is quantized per row and per half (C/2 columns each;

@@ -485,6 +485,21 @@ int rpfq_row_prescale(const void* x, int x_dtype, int64_t M, int64_t C, void* y,
                       "rpfq_row_prescale");
 }
 
+int rpfq_act_quant_prescaled(const void* x, int x_dtype, int64_t M, int64_t C, int bits, void* y, float* row_scale,
+                             void* stream) {
+    int rc = check_ln(x, x_dtype, M, C, nullptr, nullptr, 0.0f, y, RPFQ_F16);
+    if (rc) return rc;
+    if (x_dtype != RPFQ_BF16 && x_dtype != RPFQ_F32)
+        return fail(RPFQ_ERR_DTYPE, "x must be bf16 or float32 (x_dtype=%d)", x_dtype);
+    if (C % 16 != 0) return fail(RPFQ_ERR_SHAPE, "C=%lld must be a multiple of 16", (long long)C);
+    if (bits < 2 || bits > 16) return fail(RPFQ_ERR_BITS, "bits=%d unsupported (2..16)", bits);
+    if (!row_scale) return fail(RPFQ_ERR_NULL, "row_scale must not be NULL");
+    if (!aligned(row_scale, 16)) return fail(RPFQ_ERR_ALIGN, "row_scale must be 16-byte aligned");
+    return hip_status(rpfq::launch_act_quant_prescaled(x, x_dtype, M, C, bits, y, row_scale,
+                                                       reinterpret_cast<hipStream_t>(stream)),
+                      "rpfq_act_quant_prescaled");
+}
+
 int rpfq_layer_norm_act_quant(const void* x, int x_dtype, int64_t M, int64_t C, const float* gamma,
                               const float* beta, float eps, int bits, void* y, int y_dtype, void* stream) {
     int rc = check_ln(x, x_dtype, M, C, gamma, beta, eps, y, y_dtype);

@@ -67,6 +67,23 @@ def prescale_rows(x2: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     return y, s
 
 
+def act_quant_prescaled(x: torch.Tensor, num_bits: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """(y [..., C] fp16, row_scale): prescale_rows of act_quant(x, num_bits)
+    in one pass, the same bits (rpfq_act_quant_prescaled); bf16 / float32 x,
+    C a multiple of 16 up to 4096."""
+    N.require_device(x)
+    if x.dtype not in (torch.bfloat16, torch.float32):
+        raise ValueError("act_quant_prescaled takes bf16 or float32 rows")
+    x2 = _aligned_rows(x.reshape(-1, x.shape[-1]))
+    m, c = x2.shape
+    y = torch.empty(m, c, dtype=torch.float16, device=x.device)
+    s = torch.empty(m, dtype=torch.float32, device=x.device)
+    if m:
+        N.check("rpfq_act_quant_prescaled", N.load().rpfq_act_quant_prescaled(
+            x2.data_ptr(), N.dtype_code(x2.dtype), m, c, int(num_bits), y.data_ptr(), s.data_ptr(), N.stream_of(x2)))
+    return y.reshape(x.shape), s
+
+
 # RPFQ_DENSE=0 keeps every launch on the kernels that decode in their loop.
 DENSE = __import__("os").environ.get("RPFQ_DENSE", "1") != "0"
 
@@ -326,9 +343,7 @@ class PackedWide:
         # fp16 rows instead (bf16: the same operand bits, no conversion in
         # the kernel; float32: the register-staged kernel's operands).
         if row_scale is None and RANGE_GUARD and x2.dtype != torch.float16:
-            c = x2.shape[1]
-            if (PRESCALE_ROWS and c % 8 == 0 and c <= 4096
-                    and self.kernel_for(m, torch.float16, out_dtype, flags) == N.KERNEL_DMA):
+            if self.prescales(m, x2.dtype, out_dtype, flags):
                 x2, row_scale = prescale_rows(x2)
             else:
                 row_scale = row_scales(x2)
@@ -361,6 +376,21 @@ class PackedWide:
             rec(ev0, ev1, wide_flops(m, self.n_complex, self.k_complex), nbytes,
                 (m, self.n_complex, self.k_complex, kern + ("+gelu" if flags & N.FLAG_GELU else "")))
         return y.reshape(*lead, self.out_features)
+
+    def prescales(self, m: int, x_dtype: torch.dtype, out_dtype: torch.dtype, flags: int = 0) -> bool:
+        """Whether linear() takes m rows of x_dtype as prescaled fp16 rows."""
+        c = self.in_features
+        return (RANGE_GUARD and PRESCALE_ROWS and x_dtype in (torch.bfloat16, torch.float32) and c % 8 == 0
+                and c <= 4096 and self.kernel_for(m, torch.float16, out_dtype, flags) == N.KERNEL_DMA)
+
+    def act_quant_operand(self, x: torch.Tensor, bits: int, out_dtype: torch.dtype, flags: int = 0):
+        """(rows, row_scale) for linear() of act_quant(x, bits): prescaled
+        fp16 rows in one pass where linear() would prescale them in a second
+        one, else the quantized rows and None."""
+        m = x.numel() // x.shape[-1] if x.dim() and x.shape[-1] == self.in_features else 0
+        if m and self.in_features % 16 == 0 and self.prescales(m, x.dtype, out_dtype, flags):
+            return act_quant_prescaled(x, bits)
+        return act_quant(x, bits), None
 
     def _dense_bytes(self, m: int, x2: torch.Tensor, out_dtype: torch.dtype, flags: int, residual: bool) -> int:
         """Workspace of rpfq_wide_linear_dense where linear() takes it, else 0:
@@ -641,12 +671,16 @@ class PackedStages:
 
     def linear(self, x: torch.Tensor, bias: torch.Tensor | None = None,
                out_dtype: torch.dtype | None = None, flags: int = 0,
-               residual: torch.Tensor | None = None) -> torch.Tensor:
+               residual: torch.Tensor | None = None, row_scale: torch.Tensor | None = None) -> torch.Tensor:
         """PackedWide.linear over all stage groups (one launch per group)."""
-        y = self.groups[0].linear(x, bias, out_dtype, flags, residual)
+        y = self.groups[0].linear(x, bias, out_dtype, flags, residual, row_scale=row_scale)
         for g in self.groups[1:]:
-            y = g.linear(x, None, y.dtype, flags, residual=y)
+            y = g.linear(x, None, y.dtype, flags, residual=y, row_scale=row_scale)
         return y
+
+    def act_quant_operand(self, x: torch.Tensor, bits: int, out_dtype: torch.dtype, flags: int = 0):
+        """PackedWide.act_quant_operand: each group prescales its own rows."""
+        return act_quant(x, bits), None
 
     def grad_x(self, grad_y: torch.Tensor, out_dtype: torch.dtype | None = None) -> torch.Tensor:
         """Input gradient over all stage groups: the sum of the groups'

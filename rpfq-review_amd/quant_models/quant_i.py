@@ -749,7 +749,8 @@ class QATLinearComplexPhase(nn.Linear):
         if self.act_quantizer is not None and not prequantized:
             if self._aq_fusable(pw, x):  # act quant in the layer's own launch
                 return pw.act_quant_linear(x, self.act_quantizer.num_bits, bias, out_dtype=x.dtype)
-            x = ops.act_quant(x, self.act_quantizer.num_bits)
+            rows, scale = pw.act_quant_operand(x, self.act_quantizer.num_bits, x.dtype)
+            return pw.linear(rows, bias, out_dtype=x.dtype, row_scale=scale)
         return pw.linear(x, bias, out_dtype=x.dtype)
 
     @staticmethod
@@ -808,12 +809,16 @@ class QATLinearComplexPhase(nn.Linear):
             if self.act_quantizer is not None and not prequantized:
                 if self._aq_fusable(pw, x):  # act quant, layer and GELU in one launch
                     return pw.act_quant_linear(x, self.act_quantizer.num_bits, bias, out_dtype=x.dtype, gelu=True)
-                x = ops.act_quant(x, self.act_quantizer.num_bits)
             m = x.numel() // x.shape[-1]
             kern = pw.kernel_for(m, x.dtype, x.dtype, N.FLAG_GELU) if m else None
-            if kern in N.STREAM_KERNELS or kern == N.KERNEL_RESIDENT or x.dtype == torch.bfloat16 or GELU_ON_TILED:
-                return pw.linear(x, bias, out_dtype=x.dtype, gelu=True)
-            return F.gelu(pw.linear(x, bias, out_dtype=x.dtype))
+            gelu = (kern in N.STREAM_KERNELS or kern == N.KERNEL_RESIDENT or x.dtype == torch.bfloat16
+                    or GELU_ON_TILED)
+            rows, scale = x, None
+            if self.act_quantizer is not None and not prequantized:
+                rows, scale = pw.act_quant_operand(x, self.act_quantizer.num_bits, x.dtype,
+                                                   N.FLAG_GELU if gelu else 0)
+            y = pw.linear(rows, bias, out_dtype=x.dtype, gelu=gelu, row_scale=scale)
+            return y if gelu else F.gelu(y)
         return F.gelu(self.forward_prequantized(x) if prequantized else self.forward(x))
 
     def forward_layer_norm(self, x: torch.Tensor, ln_weight, ln_bias, eps: float, gelu: bool = False):
@@ -868,6 +873,7 @@ class QATLinearComplexPhase(nn.Linear):
                 if self._aq_fusable(pw, x):  # act quant, layer and residual add in one launch
                     return pw.act_quant_linear(x, self.act_quantizer.num_bits, bias, out_dtype=x.dtype,
                                                residual=residual)
-                x = ops.act_quant(x, self.act_quantizer.num_bits)
+                rows, scale = pw.act_quant_operand(x, self.act_quantizer.num_bits, x.dtype)
+                return pw.linear(rows, bias, out_dtype=x.dtype, residual=residual, row_scale=scale)
             return pw.linear(x, bias, out_dtype=x.dtype, residual=residual)
         return residual + (self.forward_prequantized(x) if prequantized else self.forward(x))
