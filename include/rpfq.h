@@ -585,8 +585,8 @@ int rpfq_wide_linear_grad_x_dense(const rpfq_wide_desc* desc, const void* packed
  * qkv [B, N, 3, H, D] (the qkv layer's output as it lies), out [B, N, H, D],
  * both of dtype (RPFQ_F16 or RPFQ_BF16), 16-byte aligned; D = 64, N <= 288.
  * Scores, softmax and outputs in float32, probabilities rounded to dtype for
- * their product with v; scale positive and finite.  Replaces the attention between qkv and proj of a
- * ViT block (RPFQ-ViTApple/scripts/audit_rpfq_vit_ios_parity.py:523-545).
+ * their product with v; scale positive and finite.  Replaces the attention
+ * between qkv and proj of a ViT block (RPFQ-ViTApple/scripts/audit_rpfq_vit_ios_parity.py:523-545).
  */
 int rpfq_attention(const void* qkv, int dtype, int64_t B, int64_t N, int64_t H, int64_t D, float scale, void* out,
                    void* stream);
@@ -618,14 +618,15 @@ int rpfq_linear_f32(const float* x, const float* w, const float* bias, int64_t M
  * grad_w = grad_y^T x (NULL: not wanted), in the same arithmetic; x_scale as
  * the forward wrote it.  grad_w takes row m of x times the scale of grad_y's
  * row, so a row whose gradients lie below 2^-17 of the largest row's loses
- * bits of its (equally smaller) share.  The bias gradient is the column sum
- * of grad_y and is left to the caller.
+ * bits of its (equally smaller) share.  grad_b [N] (NULL: not wanted): the
+ * column sums of grad_y, float32 in a fixed order, at least one of the other
+ * two wanted with it.
  * Replaces the backward of that F.linear (grad_x = grad_output @ weight,
  * grad_weight = grad_output^T @ x; kernel.py:581-588).
  */
 int rpfq_linear_f32_grad(const float* grad_y, const float* x, const float* w, int64_t M, int64_t N, int64_t K,
                          const float* w_parts, int n_parts, const float* x_scale, float* grad_x, float* grad_w,
-                         void* work, size_t work_bytes, void* stream);
+                         float* grad_b, void* work, size_t work_bytes, void* stream);
 
 /*
  * rpfq_quantize_wide without a workspace argument and without any device

@@ -706,7 +706,7 @@ int rpfq_linear_f32(const float* x, const float* w, const float* bias, int64_t M
 
 int rpfq_linear_f32_grad(const float* grad_y, const float* x, const float* w, int64_t M, int64_t N, int64_t K,
                          const float* w_parts, int n_parts, const float* x_scale, float* grad_x, float* grad_w,
-                         void* work, size_t work_bytes, void* stream) {
+                         float* grad_b, void* work, size_t work_bytes, void* stream) {
     int rc = check_linear_f32(M, N, K);
     if (rc) return rc;
     if (!grad_y || !x || !w || !w_parts || !x_scale || !work || (!grad_x && !grad_w))
@@ -718,7 +718,7 @@ int rpfq_linear_f32_grad(const float* grad_y, const float* x, const float* w, in
     const size_t need = rpfq_linear_f32_workspace_bytes(M, N, K, 1);
     if (work_bytes < need) return fail(RPFQ_ERR_SHAPE, "workspace holds %zu bytes, need %zu", work_bytes, need);
     return hip_status(rpfq::launch_linear_f32_grad(grad_y, x, w, M, N, K, w_parts, n_parts, x_scale, grad_x, grad_w,
-                                                   work, reinterpret_cast<hipStream_t>(stream)),
+                                                   grad_b, work, reinterpret_cast<hipStream_t>(stream)),
                       "rpfq_linear_f32_grad");
 }
 

@@ -362,14 +362,14 @@ hipError_t launch_attention(const void* qkv, int dt, int64_t B, int64_t N, int64
 struct F32Plan {
     int64_t Mp, Kp, Np;          // padded rows and columns of the operand planes
     size_t x_at, w_at, fwd_bytes;
-    size_t bx_at, g_at, bw_at, gs_at, part_at, bwd_bytes;
+    size_t bx_at, g_at, bw_at, gs_at, cs_at, part_at, bwd_bytes;
     int steps, splits;           // gw: 16-row steps, row splits
 };
 F32Plan f32_plan(int64_t M, int64_t N, int64_t K);
 hipError_t launch_linear_f32(const float* x, const float* w, const float* bias, int64_t M, int64_t N, int64_t K,
                              const float* parts, int nparts, float* y, float* xscale, void* work, hipStream_t s);
 hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* w, int64_t M, int64_t N, int64_t K,
-                                  const float* parts, int nparts, const float* xscale, float* gx, float* gw,
+                                  const float* parts, int nparts, const float* xscale, float* gx, float* gw, float* gb,
                                   void* work, hipStream_t s);
 // adjoint blob (rpfq_kernels.hip) and the grad_x kernel (wide_adjoint.hip)
 hipError_t launch_wide_pack_adjoint(const rpfq_wide_desc& d, const WideGeom& g, const void* packed, void* adjoint,

@@ -189,7 +189,7 @@ def load() -> ctypes.CDLL:
         lib.rpfq_linear_f32_workspace_bytes.argtypes = [i64, i64, i64, i32]
         lib.rpfq_linear_f32_workspace_bytes.restype = sz
         lib.rpfq_linear_f32.argtypes = [vp, vp, vp, i64, i64, i64, vp, i32, vp, vp, vp, sz, vp]
-        lib.rpfq_linear_f32_grad.argtypes = [vp, vp, vp, i64, i64, i64, vp, i32, vp, vp, vp, vp, sz, vp]
+        lib.rpfq_linear_f32_grad.argtypes = [vp, vp, vp, i64, i64, i64, vp, i32, vp, vp, vp, vp, vp, sz, vp]
         for name in EXPORTED[2:]:
             if name not in ("rpfq_wide_packed_bytes", "rpfq_wide_adjoint_bytes", "rpfq_quantize_workspace_bytes",
                             "rpfq_linear_f32_workspace_bytes", "rpfq_wide_dense_bytes"):

@@ -781,7 +781,7 @@ def attention(qkv: torch.Tensor, num_heads: int, scale: float) -> torch.Tensor:
 
 def _require_f32(m: int, n: int, k: int, **operands: torch.Tensor) -> None:
     """The shapes the float32 kernels index by, contiguous on one device."""
-    shapes = {"x": (m, k), "w": (n, k), "grad_y": (m, n), "bias": (n,), "x_scale": (m,)}
+    shapes = {"x": (m, k), "w": (n, k), "grad_y": (m, n), "bias": (n,), "x_scale": (m,), "grad_b": (n,)}
     device = operands["x"].device
     for name, t in operands.items():
         if t is None:
@@ -812,13 +812,15 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, w_pa
 
 
 def linear_f32_grad(grad_y: torch.Tensor, x: torch.Tensor, w: torch.Tensor, w_parts: torch.Tensor,
-                    x_scale: torch.Tensor, want_x: bool = True, want_w: bool = True):
-    """(grad_x or None, grad_w or None) of linear_f32 (rpfq_linear_f32_grad)
-    for a contiguous float32 grad_y [M, N]."""
+                    x_scale: torch.Tensor, want_x: bool = True, want_w: bool = True,
+                    grad_b: torch.Tensor | None = None):
+    """(grad_x or None, grad_w or None) of linear_f32 (rpfq_linear_f32_grad,
+    one of them at least) for a contiguous float32 grad_y [M, N]; grad_b [N]:
+    where the column sums of grad_y are written."""
     N.require_device(grad_y, x, w, w_parts, x_scale)
     m, k = x.shape
     n = w.shape[0]
-    _require_f32(m, n, k, grad_y=grad_y, x=x, w=w, w_parts=w_parts, x_scale=x_scale)
+    _require_f32(m, n, k, grad_y=grad_y, x=x, w=w, w_parts=w_parts, x_scale=x_scale, grad_b=grad_b)
     lib = N.load()
     nbytes = lib.rpfq_linear_f32_workspace_bytes(m, n, k, 1)
     gx = torch.empty_like(x) if want_x else None
@@ -826,7 +828,7 @@ def linear_f32_grad(grad_y: torch.Tensor, x: torch.Tensor, w: torch.Tensor, w_pa
     work = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     N.check("rpfq_linear_f32_grad", lib.rpfq_linear_f32_grad(
         grad_y.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k, w_parts.data_ptr(), w_parts.numel(),
-        x_scale.data_ptr(), N.ptr(gx), N.ptr(gw), work.data_ptr(), nbytes, N.stream_of(x)))
+        x_scale.data_ptr(), N.ptr(gx), N.ptr(gw), N.ptr(grad_b), work.data_ptr(), nbytes, N.stream_of(x)))
     return gx, gw
 
 

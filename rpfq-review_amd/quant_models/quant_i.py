@@ -485,7 +485,8 @@ def records_grad(module: nn.Module, x: torch.Tensor) -> bool:
 
 class _SplitLinearFn(torch.autograd.Function):
     """F.linear of float32 x and A_q on the split-fp16 matrix-core kernels
-    (rpfq_linear_f32, float32 accuracy); the bias gradient is the column sum.
+    (rpfq_linear_f32, float32 accuracy); the bias gradient is the column sum,
+    taken in the pass that splits grad_y.
     A backward that autograd records (create_graph) runs torch's products."""
 
     @staticmethod
@@ -505,14 +506,18 @@ class _SplitLinearFn(torch.autograd.Function):
         x, w, parts, scale = ctx.saved_tensors
         g2, x2 = grad.reshape(-1, grad.shape[-1]), x.reshape(-1, x.shape[-1])
         want_x, want_w = ctx.needs_input_grad[:2]
+        want_b, gb = ctx.has_bias and ctx.needs_input_grad[2], None
         if torch.is_grad_enabled():
             gx = g2 @ w if want_x else None
             gw = g2.t() @ x2 if want_w else None
         elif want_x or want_w:
-            gx, gw = ops.linear_f32_grad(ops._aligned_rows(g2), ops._aligned_rows(x2), w, parts, scale, want_x, want_w)
+            gb = g2.new_empty(w.shape[0]) if want_b else None
+            gx, gw = ops.linear_f32_grad(ops._aligned_rows(g2), ops._aligned_rows(x2), w, parts, scale, want_x, want_w,
+                                         gb)
         else:
             gx = gw = None
-        gb = g2.sum(0) if ctx.has_bias and ctx.needs_input_grad[2] else None
+        if want_b and gb is None:
+            gb = g2.sum(0)
         return None if gx is None else gx.reshape(x.shape), gw, gb, None
 
 

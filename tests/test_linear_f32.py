@@ -103,6 +103,28 @@ def test_linear_f32_empty_gradient():
     assert not gx.any() and not gw.any()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n", [(1, 8), (5, 40), (96, 520), (1025, 1000), (4099, 2056), (12608, 3072), (130, 4096)])
+def test_bias_gradient_is_the_column_sum(m, n):
+    """Each column within the roundings of its additions: a lane's rows, the
+    block's 4 waves, 16 partial rows and 6 levels of a tree, 2^-24 each."""
+    from quant_models import ops
+
+    x, w, _, gy = _inputs(m, n, 64)
+    gy = gy * torch.exp2(torch.randint(-20, 20, (1, n), device=DEV).float())
+    parts = w.abs().max().reshape(1)
+    _, scale = ops.linear_f32(x, w, None, parts)
+    gb = torch.empty(n, device=DEV)
+    gx, gw = ops.linear_f32_grad(gy, x, w, parts, scale, grad_b=gb)
+    gx0, gw0 = ops.linear_f32_grad(gy, x, w, parts, scale)
+    assert torch.equal(gx, gx0) and torch.equal(gw, gw0)
+    adds = m // 4096 + 2 + 4 + 16 + 6
+    assert bool(((gb.double() - gy.double().sum(0)).abs() <= adds * 2.0 ** -24 * gy.double().abs().sum(0)).all())
+    gy[m // 2, 3], gy[0, 5], gy[m - 1, 7] = float("inf"), float("nan"), float("-inf")
+    ops.linear_f32_grad(gy, x, w, parts, scale, grad_b=gb)
+    assert gb[3] == float("inf") and torch.isnan(gb[5]) and gb[7] == float("-inf")
+
+
 def _layer(method, act, rot, seed=3):
     from quant_models.quant_i import QATLinearComplexPhase
 
@@ -196,7 +218,7 @@ def test_linear_f32_argument_errors():
     assert lib.rpfq_linear_f32(p, p, None, 64, 64, 64, p, 0, p, p, p, 1 << 30, None) == 6
     assert lib.rpfq_linear_f32(p, p, None, 64, 64, 64, p, 1, p, p, p, 1024, None) == 2
     assert lib.rpfq_linear_f32(ctypes.c_void_p(4100), p, None, 64, 64, 64, p, 1, p, p, p, 1 << 30, None) == 3
-    assert lib.rpfq_linear_f32_grad(p, p, p, 64, 64, 64, p, 1, p, None, None, p, 1 << 30, None) == 1
+    assert lib.rpfq_linear_f32_grad(p, p, p, 64, 64, 64, p, 1, p, None, None, p, p, 1 << 30, None) == 1
 
 
 def test_row_and_weight_scales_hold_the_bound():
