@@ -46,19 +46,16 @@ struct QuantArgs {
     int nblocks;       // reduction blocks
 };
 
-// Axis class of (re, im) as the exporter codes it (quant_i.py:36-62,
-// export_rpfq_vit_to_mlx.py:214-218): 1 real_pos, 0 real_neg, 3 imag_pos,
-// 2 imag_neg; 4 = no mask set (only for NaN input), stored as code 0.
-__device__ __forceinline__ int axis_class(float re, float im) {
-    float ar = fabsf(re), ai = fabsf(im);
-    if (ar > ai) return re >= 0.0f ? 1 : 0;
-    if (ai > ar) return im >= 0.0f ? 3 : 2;
-    if (re == 0.0f && im == 0.0f) return 1;  // zero tie -> real_pos
-    if (re > 0.0f && im > 0.0f) return 3;    // quadrant I tie -> imag_pos
-    if (re < 0.0f && im > 0.0f) return 0;    // quadrant II tie -> real_neg
-    if (re < 0.0f && im < 0.0f) return 2;    // quadrant III tie -> imag_neg
-    if (re > 0.0f && im < 0.0f) return 1;    // quadrant IV tie -> real_pos
-    return 4;
+// Masks of the axis class of (re, im) as the exporter codes it (quant_i.py:36-62,
+// export_rpfq_vit_to_mlx.py:214-218): the larger part; of two equal ones the
+// real part for zeros and for unlike signs (quadrants II and IV), the
+// imaginary part for like signs (I and III).  Neither for NaN.  Without
+// branches: the passes are bound by their VALU instructions.
+__device__ __forceinline__ void axis_masks(float re, float im, bool& on_re, bool& on_im) {
+    const float ar = fabsf(re), ai = fabsf(im);
+    const bool tie = ar == ai, tie_re = (ar == 0.0f) | ((re < 0.0f) != (im < 0.0f));
+    on_re = (ar > ai) | (tie & tie_re);
+    on_im = (ai > ar) | (tie & !tie_re);
 }
 
 // One plane's running state: residual r and accumulated q.
@@ -77,20 +74,19 @@ __device__ __forceinline__ uint32_t apply_stage(Plane& p, float s_re, float s_im
         v_im = pi ? s_im : -s_im;
         code = (pr ? 1u : 0u) | (pi ? 2u : 0u);
     } else {  // quant_i.py:65-81
-        int c = axis_class(p.r_re, p.r_im);
-        v_re = c == 1 ? s_re : (c == 0 ? -s_re : 0.0f);
-        v_im = c == 3 ? s_im : (c == 2 ? -s_im : 0.0f);
-        code = c == 4 ? 0u : (uint32_t)c;
+        // codes 1 real_pos, 0 real_neg, 3 imag_pos, 2 imag_neg; 0 for NaN
+        bool on_re, on_im;
+        axis_masks(p.r_re, p.r_im, on_re, on_im);
+        const bool pr = p.r_re >= 0.0f, pi = p.r_im >= 0.0f;
+        v_re = on_re ? (pr ? s_re : -s_re) : 0.0f;
+        v_im = on_im ? (pi ? s_im : -s_im) : 0.0f;
+        code = on_im ? (pi ? 3u : 2u) : (on_re & pr ? 1u : 0u);
     }
     p.q_re = p.q_re + v_re;  // quant_i.py:114-117
     p.q_im = p.q_im + v_im;
     p.r_re = p.r_re - v_re;
     p.r_im = p.r_im - v_im;
     return code;
-}
-
-__device__ __forceinline__ uint32_t apply_stage_k(int kind, Plane& p, float s_re, float s_im) {
-    return kind == RPFQ_QK_SIGN ? apply_stage<RPFQ_QK_SIGN>(p, s_re, s_im) : apply_stage<RPFQ_QK_AXIS>(p, s_re, s_im);
 }
 
 // U and W of element (n, k), rotated for quantization when rot is set
@@ -161,15 +157,38 @@ __device__ __forceinline__ void item_nk(const QuantArgs& a, int64_t it, bool sma
     }
 }
 
-// Masked |r| sums and counts of stage a.stage for U (0..3) and W (4..7):
+// Masked |r| sums and counts of stage ST for U (0..3) and W (4..7):
 // (sum |re| over the real mask, count, sum |im| over the imaginary mask,
-// count); SIGN planes count every element.
-template <int V>
+// count); SIGN planes (KU, KW) count every element.  A kernel per stage and
+// kinds, selects instead of branches and integer counts: with the kinds and
+// stages looked up per element the 9.4 MB of ViT-B fc1 took 12.9 us a stage
+// (9.7 now) and quant_apply_kernel 11.5 (7.9).
+template <int ST, int KIND>
+__device__ __forceinline__ void reduce_element(Plane& q, const float* sc, double& sre, double& sim, int& nre, int& nim) {
+#pragma unroll
+    for (int t = 0; t < ST; ++t) apply_stage<KIND>(q, sc[2 * t], sc[2 * t + 1]);
+    if (KIND == RPFQ_QK_SIGN) {
+        sre += (double)fabsf(q.r_re);
+        sim += (double)fabsf(q.r_im);
+        ++nre;
+        ++nim;
+    } else {
+        bool on_re, on_im;
+        axis_masks(q.r_re, q.r_im, on_re, on_im);
+        sre += (double)(on_re ? fabsf(q.r_re) : 0.0f);
+        sim += (double)(on_im ? fabsf(q.r_im) : 0.0f);
+        nre += on_re;
+        nim += on_im;
+    }
+}
+
+template <int V, int ST, int KU, int KW>
 __global__ void __launch_bounds__(kQThreads) quant_reduce_kernel(QuantArgs a) {
     double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    int cnt[4] = {0, 0, 0, 0};  // of one thread: at most N K / (threads of the grid) + V
     const int64_t items = a.N * (a.K / V);
     const bool small = items < (1LL << 31);
-    const int st = a.stage;
+    const bool do_u = a.steps[0] > ST, do_w = a.steps[1] > ST;
     float sc[16];  // scales of the finished stages (finalized by earlier launches)
 #pragma unroll
     for (int i = 0; i < 16; ++i) sc[i] = a.scales[i];
@@ -181,32 +200,12 @@ __global__ void __launch_bounds__(kQThreads) quant_reduce_kernel(QuantArgs a) {
         load_planes_v<V>(a, n, k0, u, w);
 #pragma unroll
         for (int v = 0; v < V; ++v) {
-            Plane* pl[2] = {&u[v], &w[v]};
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                if (a.steps[p] <= st) continue;
-                Plane& q = *pl[p];
-#pragma unroll
-                for (int t = 0; t < 3; ++t)
-                    if (t < st) apply_stage_k(a.kind[p], q, sc[(p * 4 + t) * 2], sc[(p * 4 + t) * 2 + 1]);
-                if (a.kind[p] == RPFQ_QK_SIGN) {
-                    acc[4 * p + 0] += (double)fabsf(q.r_re);
-                    acc[4 * p + 1] += 1.0;
-                    acc[4 * p + 2] += (double)fabsf(q.r_im);
-                    acc[4 * p + 3] += 1.0;
-                } else {
-                    const int c = axis_class(q.r_re, q.r_im);
-                    if (c == 0 || c == 1) {
-                        acc[4 * p + 0] += (double)fabsf(q.r_re);
-                        acc[4 * p + 1] += 1.0;
-                    } else if (c == 2 || c == 3) {
-                        acc[4 * p + 2] += (double)fabsf(q.r_im);
-                        acc[4 * p + 3] += 1.0;
-                    }
-                }
-            }
+            if (do_u) reduce_element<ST, KU>(u[v], sc, acc[0], acc[2], cnt[0], cnt[1]);
+            if (do_w) reduce_element<ST, KW>(w[v], sc + 8, acc[4], acc[6], cnt[2], cnt[3]);
         }
     }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[2 * j + 1] = (double)cnt[j];
     // fixed-order block reduction: wave butterfly, then the 4 waves in order
     __shared__ double red[kQThreads / 64][8];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -275,7 +274,7 @@ __global__ void __launch_bounds__(kQThreads) quant_finalize_kernel(QuantArgs a) 
 // All stages with the final scales: A_q (rotated back, recombined) and the
 // code planes.  V consecutive columns per thread (V = 4 writes one packed
 // code byte per plane and stage).
-template <int V>
+template <int V, int KU, int KW>
 __global__ void __launch_bounds__(kQThreads) quant_apply_kernel(QuantArgs a) {
     const int64_t items = a.N * (a.K / V);
     const bool small = items < (1LL << 31);
@@ -294,16 +293,11 @@ __global__ void __launch_bounds__(kQThreads) quant_apply_kernel(QuantArgs a) {
         float o11[V], o12[V], o21[V], o22[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) {
-            Plane* pl[2] = {&u[v], &w[v]};
 #pragma unroll
-            for (int p = 0; p < 2; ++p)
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    if (t < a.steps[p]) {
-                        const uint32_t c = apply_stage_k(a.kind[p], *pl[p], sc[(p * 4 + t) * 2],
-                                                         sc[(p * 4 + t) * 2 + 1]);
-                        cbyte[p * 4 + t] |= c << (2 * v);
-                    }
+            for (int t = 0; t < 4; ++t) {
+                if (t < a.steps[0]) cbyte[t] |= apply_stage<KU>(u[v], sc[2 * t], sc[2 * t + 1]) << (2 * v);
+                if (t < a.steps[1]) cbyte[4 + t] |= apply_stage<KW>(w[v], sc[8 + 2 * t], sc[9 + 2 * t]) << (2 * v);
+            }
             float ur = u[v].q_re, ui = u[v].q_im, wr = w[v].q_re, wi = w[v].q_im;
             if (a.rot) {  // quant_i.py:433-434
                 const float cu = a.rot[0], su = a.rot[1], cw = a.rot[2], sw = a.rot[3];
@@ -353,6 +347,36 @@ __global__ void __launch_bounds__(kQThreads) quant_apply_kernel(QuantArgs a) {
 // a kernel (its name is a host-side stand-in there): quant_scratch_ptr() resolves
 // the device address once per device.
 static __device__ __align__(256) double scratch[kQuantMaxBlocks * 8];
+
+template <int V, int ST>
+void reduce_go(const QuantArgs& a, hipStream_t s) {
+    const dim3 grid(a.nblocks), block(kQThreads);
+    const bool su = a.kind[0] == RPFQ_QK_SIGN, sw = a.kind[1] == RPFQ_QK_SIGN;
+    if (su && sw) hipLaunchKernelGGL((quant_reduce_kernel<V, ST, RPFQ_QK_SIGN, RPFQ_QK_SIGN>), grid, block, 0, s, a);
+    else if (su) hipLaunchKernelGGL((quant_reduce_kernel<V, ST, RPFQ_QK_SIGN, RPFQ_QK_AXIS>), grid, block, 0, s, a);
+    else if (sw) hipLaunchKernelGGL((quant_reduce_kernel<V, ST, RPFQ_QK_AXIS, RPFQ_QK_SIGN>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((quant_reduce_kernel<V, ST, RPFQ_QK_AXIS, RPFQ_QK_AXIS>), grid, block, 0, s, a);
+}
+
+template <int V>
+void reduce_stage(const QuantArgs& a, hipStream_t s) {
+    switch (a.stage) {
+        case 0: reduce_go<V, 0>(a, s); break;
+        case 1: reduce_go<V, 1>(a, s); break;
+        case 2: reduce_go<V, 2>(a, s); break;
+        default: reduce_go<V, 3>(a, s); break;
+    }
+}
+
+template <int V>
+void apply_go(const QuantArgs& a, unsigned blocks, hipStream_t s) {
+    const dim3 grid(blocks), block(kQThreads);
+    const bool su = a.kind[0] == RPFQ_QK_SIGN, sw = a.kind[1] == RPFQ_QK_SIGN;
+    if (su && sw) hipLaunchKernelGGL((quant_apply_kernel<V, RPFQ_QK_SIGN, RPFQ_QK_SIGN>), grid, block, 0, s, a);
+    else if (su) hipLaunchKernelGGL((quant_apply_kernel<V, RPFQ_QK_SIGN, RPFQ_QK_AXIS>), grid, block, 0, s, a);
+    else if (sw) hipLaunchKernelGGL((quant_apply_kernel<V, RPFQ_QK_AXIS, RPFQ_QK_SIGN>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((quant_apply_kernel<V, RPFQ_QK_AXIS, RPFQ_QK_AXIS>), grid, block, 0, s, a);
+}
 
 int reduce_blocks(int64_t total) {
     int64_t b = (total + kQThreads - 1) / kQThreads;
@@ -407,9 +431,9 @@ hipError_t launch_quantize_wide(const rpfq_quant_desc& d, const float* weight, c
     for (int st = 0; st < max_steps; ++st) {
         a.stage = st;
         if (v4)
-            hipLaunchKernelGGL(quant_reduce_kernel<4>, dim3(a.nblocks), dim3(kQThreads), 0, s, a);
+            reduce_stage<4>(a, s);
         else
-            hipLaunchKernelGGL(quant_reduce_kernel<1>, dim3(a.nblocks), dim3(kQThreads), 0, s, a);
+            reduce_stage<1>(a, s);
         hipLaunchKernelGGL(quant_finalize_kernel, dim3(1), dim3(kQThreads), 0, s, a);
     }
     if (aq || codes) {
@@ -417,9 +441,9 @@ hipError_t launch_quantize_wide(const rpfq_quant_desc& d, const float* weight, c
         int64_t blocks = (items + kQThreads - 1) / kQThreads;
         if (blocks > 8 * kQuantMaxBlocks) blocks = 8 * kQuantMaxBlocks;
         if (v4)
-            hipLaunchKernelGGL(quant_apply_kernel<4>, dim3((unsigned)blocks), dim3(kQThreads), 0, s, a);
+            apply_go<4>(a, (unsigned)blocks, s);
         else
-            hipLaunchKernelGGL(quant_apply_kernel<1>, dim3((unsigned)blocks), dim3(kQThreads), 0, s, a);
+            apply_go<1>(a, (unsigned)blocks, s);
     }
     return hipGetLastError();
 }
