@@ -97,35 +97,27 @@ PyObject* done(int rc, const at::Tensor& y) {
 }
 
 // linear(desc, blob, x, bias, residual, out_dtype, flags, guard): guard bit 0:
-// float32 / bf16 rows get their prescales, bit 1: as prescaled fp16 rows where
-// the DMA kernel takes those.
+// float32 / bf16 rows get their prescales, bit 1: rows that go to the DMA
+// kernel as prescaled fp16 (many rows) are left to the Python path.
 PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Call c;
     const float* bias;
     if (n != 8 || !layer(a[0], a[1], a[2], a[4], a[5], c) || !vec(a[3], 2 * c.d->n_complex, &bias)) Py_RETURN_NONE;
     const int flags = (int)PyLong_AsLong(a[6]), guard = (int)PyLong_AsLong(a[7]);
-    const void* xp = c.x->data_ptr();
-    int xdt = c.xdt;
     const float* scale = nullptr;
-    at::Tensor s, rows;
-    if (xdt != RPFQ_F16 && (guard & 1)) {
+    at::Tensor s;
+    if (c.xdt != RPFQ_F16 && (guard & 1)) {
         const int64_t in = 2 * c.d->k_complex;
+        int kernel = -1;
+        if ((guard & 2) && in <= 4096 &&
+            rpfq_wide_linear_kernel(c.d, c.m, RPFQ_F16, c.ydt, flags, &kernel) == RPFQ_OK && kernel == RPFQ_KERNEL_DMA)
+            Py_RETURN_NONE;
         s = at::empty({c.m}, c.x->options().dtype(at::kFloat));
         scale = s.const_data_ptr<float>();
-        int kernel = -1, rc;
-        if ((guard & 2) && in <= 4096 &&
-            rpfq_wide_linear_kernel(c.d, c.m, RPFQ_F16, c.ydt, flags, &kernel) == RPFQ_OK && kernel == RPFQ_KERNEL_DMA) {
-            rows = at::empty({c.m, in}, c.x->options().dtype(at::kHalf));
-            rc = rpfq_row_prescale(xp, xdt, c.m, in, rows.data_ptr(), s.data_ptr<float>(), c.stream);
-            xp = rows.data_ptr();
-            xdt = RPFQ_F16;
-        } else {
-            rc = rpfq_row_scales(xp, xdt, c.m, in, s.data_ptr<float>(), c.stream);
-        }
-        if (rc != RPFQ_OK) Py_RETURN_NONE;
+        if (rpfq_row_scales(c.x->data_ptr(), c.xdt, c.m, in, s.data_ptr<float>(), c.stream) != RPFQ_OK) Py_RETURN_NONE;
     }
-    return done(rpfq_wide_linear_scaled(c.d, c.blob->data_ptr(), c.blob->nbytes(), xp, xdt, c.m, scale, bias, c.res,
+    return done(rpfq_wide_linear_scaled(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m, scale, bias, c.res,
                                         c.y.data_ptr(), c.ydt, flags, c.stream),
                 c.y);
     END_HANDLE_TH_ERRORS
