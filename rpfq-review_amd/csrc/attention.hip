@@ -90,10 +90,10 @@ __global__ void __launch_bounds__(256, 2) attention_kernel(AttnArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    {   // V rows past N: a probability of 0 must meet a finite value
-        const int t = a.N + (tid >> 3);
-        if (t < 32 * NB) *reinterpret_cast<uint4*>(smem + KV + t * 128 + (tid & 7) * 16) = make_uint4(0, 0, 0, 0);
-    }
+    // V rows past N (up to 63 of them: N = 1 on 2 blocks): a probability of 0
+    // must meet a finite value
+    for (int t = a.N + (tid >> 3); t < 32 * NB; t += 32)
+        *reinterpret_cast<uint4*>(smem + KV + t * 128 + (tid & 7) * 16) = make_uint4(0, 0, 0, 0);
     __syncthreads();
 
     const int sw = (r >> 1) & 7, i16 = lane & 15, hf = (lane >> 4) & 1;

@@ -65,6 +65,27 @@ def test_attention_extreme_scores_and_special_values():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 20, 31, 32, 33, 63, 64, 65, 82, 95, 96, 97, 127, 129, 161, 193, 225, 288])
+def test_attention_special_values_at_every_padding(n):
+    """inf and NaN in v of the first and last token, 0 to 63 rows of padding
+    behind it: that output column only, and never NaN from an inf."""
+    from quant_models import ops
+
+    heads = 2
+    base = torch.randn(2, n, 3 * heads * 64, device=DEV, generator=torch.Generator(device=DEV).manual_seed(n)).half()
+    clean = ops.attention(base, heads, 0.125)
+    for token in (0, n - 1):
+        for value in (float("inf"), float("-inf"), float("nan")):
+            qkv = base.clone()
+            qkv[1, token, 2 * heads * 64 + 64 + 37] = value  # image 1, head 1, value 37
+            out = ops.attention(qkv, heads, 0.125)
+            got = out[1, :, 64 + 37].clone()
+            assert bool(torch.isnan(got).all()) if value != value else bool((got == value).all())
+            out[1, :, 64 + 37] = clean[1, :, 64 + 37]
+            assert torch.equal(out, clean)
+
+
+@pytest.mark.gpu
 def test_block_attention_route():
     """The block's attention takes the kernel in inference only, and agrees
     with torch's there."""
