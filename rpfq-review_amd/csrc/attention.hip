@@ -17,8 +17,8 @@ namespace rpfq {
 // ds_read_b64_tr_b16 gathers V's rows in that order.  Scores, maxima, sums
 // and outputs are float32.
 // Bound by HBM (q, k, v once, out once) and, next to it, the exponentials:
-// 256 x 12 heads, 197 tokens 92 us (310 MB, 3.4 TB/s; torch's library kernel
-// 172), 64 x 3 heads, 198 tokens 10 us (17).  Without the fences around each
+// 256 x 12 heads, 197 tokens 85 us (310 MB, 3.6 TB/s; torch's library kernel
+// 172), 64 x 3 heads, 198 tokens 9 us (17).  Without the fences around each
 // key block the compiler read every fragment first and spilled (141 us).
 struct AttnArgs {
     const char* qkv;
@@ -130,11 +130,10 @@ __global__ void __launch_bounds__(256, 2) attention_kernel(AttnArgs a) {
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        const int next = qb + 4 * a.parts;
-        load_q(next < blocks ? next : 0, q);
+        // keys past N: in the last block, or the last two of the sizes that NB =
+        // 2 (N = 1 ..) and 4 (N = 65 ..) also serve
 #pragma unroll
-        for (int kb = 0; kb < NB; ++kb) {
-            if (32 * kb + 32 <= a.N) continue;  // keys past N (at most the last blocks)
+        for (int kb = NB <= 4 ? NB - 2 : NB - 1; kb < NB; ++kb) {
 #pragma unroll
             for (int v = 0; v < 16; ++v)
                 if (32 * kb + acc_row(v, g) >= a.N) s[kb][v] = -__builtin_inff();
@@ -145,6 +144,20 @@ __global__ void __launch_bounds__(256, 2) attention_kernel(AttnArgs a) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) mx = fmaxf(mx, s[kb][v]);
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        // Scores far from 0: the product of the largest with scale2 is rounded,
+        // and past 2^20 by enough to carry a probability out of fp16's range
+        // (an inf, and NaN with it).  There the largest is subtracted first.
+        const bool far = fabsf(mx) * a.scale2 > 0x1p20f;
+        if (__any(far)) {
+            const float sub = far ? mx : 0.0f;
+#pragma unroll
+            for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) s[kb][v] -= sub;
+            mx -= sub;
+        }
+        const int next = qb + 4 * a.parts;
+        load_q(next < blocks ? next : 0, q);
         // probabilities times 2^15: fp16 keeps them normal down to 2^-29 of the
         // row's largest (undone by the sum, which carries the same factor)
         const float mc = mx * a.scale2 - 15.0f;

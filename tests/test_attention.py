@@ -86,6 +86,31 @@ def test_attention_special_values_at_every_padding(n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,size", [(torch.float16, 32.0), (torch.bfloat16, 32.0), (torch.bfloat16, 2.0 ** 40)])
+@pytest.mark.parametrize("n", [5, 64, 197, 288])
+def test_attention_scores_past_the_float32_integers(n, dtype, size):
+    """Finite scores of any size: q and k are small integers times `size`, so
+    float32 holds each score exactly, and every row that has its own key wins
+    by far.  The largest scores, times scale and log2(e), pass 2^24 (bf16:
+    2^85), where float32 has no fractions left."""
+    from quant_models import ops
+
+    g = torch.Generator(device=DEV).manual_seed(n)
+    heads = 2
+    qkv = torch.randint(-63, 64, (2, n, 3, heads, 64), device=DEV, generator=g).float() * size
+    far = torch.arange(1, n + 1, device=DEV).reshape(1, n, 1, 1) % 31 + 32.0
+    sign = torch.randint(0, 2, (2, n, heads, 64), device=DEV, generator=g) * 2.0 - 1
+    qkv[:, :, 0] = qkv[:, :, 1] = sign * far * size
+    qkv[:, :, 2] = torch.randn(2, n, heads, 64, device=DEV, generator=g)
+    qkv = qkv.reshape(2, n, -1).to(dtype)
+    ref = _exact(qkv, heads, 0.125)
+    u = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    out = ops.attention(qkv, heads, 0.125).double()
+    assert bool(out.isfinite().all())
+    assert float((out - ref).abs().max()) <= 2.5 * u * float(qkv.reshape(2, n, 3, -1)[:, :, 2].abs().max())
+
+
+@pytest.mark.gpu
 def test_block_attention_route():
     """The block's attention takes the kernel in inference only, and agrees
     with torch's there."""
