@@ -158,9 +158,11 @@ __global__ void __launch_bounds__(256, 2) attention_kernel(AttnArgs a) {
         }
         const int next = qb + 4 * a.parts;
         load_q(next < blocks ? next : 0, q);
-        // probabilities times 2^15: fp16 keeps them normal down to 2^-29 of the
-        // row's largest (undone by the sum, which carries the same factor)
-        const float mc = mx * a.scale2 - 15.0f;
+        // fp16: probabilities times 2^15, normal down to 2^-29 of the row's
+        // largest, in sums below 2^39.  bf16 has float32's range and so have
+        // its values: times 2^-9, so that the sum of 288 of them stays within
+        // the largest value.  Undone by l, which carries the same factor.
+        const float mc = mx * a.scale2 + (BF ? 9.0f : -15.0f);
         float l = 0.0f;
         floatx16 o[2];
         o[0] = o[1] = floatx16{0};

@@ -111,6 +111,22 @@ def test_attention_scores_past_the_float32_integers(n, dtype, size):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 64, 197, 288])
+def test_attention_of_the_largest_bf16_values(n):
+    """v up to bf16's largest: a weighted mean of finite values is finite."""
+    from quant_models import ops
+
+    g = torch.Generator(device=DEV).manual_seed(n)
+    qkv = torch.randn(2, n, 3 * 64, device=DEV, generator=g)
+    qkv[..., 128:] = 1.5 * 2.0 ** 126 + 2.0 ** 125 * torch.rand(2, n, 64, device=DEV, generator=g)
+    qkv[..., 150:] *= -1
+    qkv = qkv.bfloat16()
+    out = ops.attention(qkv, 1, 0.125).double()
+    assert bool(out.isfinite().all())
+    assert float((out - _exact(qkv, 1, 0.125)).abs().max()) <= 2.5 * 2.0 ** -8 * float(qkv.abs().max())
+
+
+@pytest.mark.gpu
 def test_block_attention_route():
     """The block's attention takes the kernel in inference only, and agrees
     with torch's there."""
