@@ -12,6 +12,7 @@ norm1 -> qkv -> SDPA -> proj -> +res -> norm2 -> fc1 -> GELU(erf) -> fc2 -> +res
 """
 from __future__ import annotations
 
+import math
 import os
 
 import torch
@@ -293,14 +294,16 @@ class Attention(nn.Module):
         qkv = qkv.reshape(b, n, 3, self.num_heads, self.head_dim)
         qkv = qkv.permute(2, 0, 3, 1, 4)
         q, k, v = qkv.unbind(0)
-        x = F.scaled_dot_product_attention(q, k, v, dropout_p=self.attn_drop.p if self.training else 0.0)
+        x = F.scaled_dot_product_attention(q, k, v, dropout_p=self.attn_drop.p if self.training else 0.0,
+                                           scale=self.scale)
         return x.transpose(1, 2).reshape(b, n, c)
 
     def _attends_on_device(self, qkv) -> bool:
         """The attention kernel takes qkv, the output of a packed layer: 16-bit
-        heads of 64 values over at most 288 tokens (ops.attention), eval mode,
-        nothing recorded or transformed by autograd, and no autocast to another
-        dtype.  Longer sequences do not fit the kernel's LDS and keep torch's."""
+        heads of 64 values over at most 288 tokens (ops.attention), a scale
+        that is positive and finite, eval mode, nothing recorded
+        or transformed by autograd, and no autocast to another dtype.
+        Longer sequences do not fit the kernel's LDS and keep torch's."""
         if not (FUSED_BLOCKS and qkv.is_cuda and not self.training and getattr(self.qkv, "use_packed", False)
                 and qkv.dtype in (torch.float16, torch.bfloat16) and self.head_dim == 64):
             return False
@@ -310,7 +313,8 @@ class Attention(nn.Module):
             return False
         from . import ops
 
-        return qkv.shape[1] <= ops.ATTENTION_MAX_TOKENS and torch.autograd.forward_ad._current_level < 0
+        return (qkv.shape[1] <= ops.ATTENTION_MAX_TOKENS and 0.0 < self.scale < math.inf
+                and torch.autograd.forward_ad._current_level < 0)
 
     def forward(self, x):
         return self.proj_drop(self.proj(self._mix(x)))

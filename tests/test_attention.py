@@ -163,6 +163,31 @@ def test_block_attention_route():
         ops.attention = real
 
 
+def test_block_attention_keeps_torch_outside_the_kernels_limits():
+    """Every size and scale that torch's attention takes is still taken: the
+    kernel's limits choose the route, and both routes use the same scale."""
+    from types import SimpleNamespace
+
+    from quant_models.vision_transformer import Attention
+
+    def takes(b, n, heads, scale=None):
+        attn = Attention(64 * heads, heads).eval()
+        attn.qkv.use_packed = True
+        attn.scale = attn.scale if scale is None else scale
+        qkv = SimpleNamespace(is_cuda=True, dtype=torch.float16, requires_grad=False, shape=(b, n, 192 * heads))
+        return attn._attends_on_device(qkv)
+
+    assert takes(256, 197, 12) and takes(4, 288, 3, 2.5) and not takes(1, 289, 1)
+    for scale in (0.0, -0.125, float("inf"), float("nan")):
+        assert not takes(1, 8, 1, scale)
+    attn = Attention(128, 2).eval()
+    qkv = torch.randn(2, 9, 384, generator=torch.Generator().manual_seed(0))
+    q, k, v = qkv.reshape(2, 9, 3, 2, 64).permute(2, 0, 3, 1, 4).unbind(0)
+    for attn.scale in (0.125, 0.5, 0.0, -0.25):
+        ref = (torch.softmax(q @ k.transpose(-1, -2) * attn.scale, -1) @ v).transpose(1, 2).reshape(2, 9, 128)
+        assert torch.allclose(attn._attend(qkv), ref, rtol=1e-5, atol=1e-5)
+
+
 def test_attention_argument_errors():
     from quant_models import _native as N
 
