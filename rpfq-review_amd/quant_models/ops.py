@@ -759,6 +759,12 @@ def quantize_wide(weight: torch.Tensor, kind_u: str, steps_u: int, kind_w: str, 
 ATTENTION_MAX_TOKENS = 288
 
 
+def attention_fits(b: int, n: int, heads: int) -> bool:
+    """Whether b images of n tokens and `heads` heads are within
+    rpfq_attention's limits."""
+    return n <= ATTENTION_MAX_TOKENS and heads <= 1024 and b * heads <= 1 << 24
+
+
 def attention(qkv: torch.Tensor, num_heads: int, scale: float) -> torch.Tensor:
     """softmax(q k^T scale) v [B, N, C] of a qkv tensor [B, N, 3 C] (fp16 or
     bf16, heads of 64 values, N <= ATTENTION_MAX_TOKENS; rpfq_attention)."""

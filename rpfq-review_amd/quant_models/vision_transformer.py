@@ -300,8 +300,8 @@ class Attention(nn.Module):
 
     def _attends_on_device(self, qkv) -> bool:
         """The attention kernel takes qkv, the output of a packed layer: 16-bit
-        heads of 64 values over at most 288 tokens (ops.attention), a scale
-        that is positive and finite, eval mode, nothing recorded
+        heads of 64 values, as many tokens and heads as ops.attention_fits
+        and a scale that is positive and finite, eval mode, nothing recorded
         or transformed by autograd, and no autocast to another dtype.
         Longer sequences do not fit the kernel's LDS and keep torch's."""
         if not (FUSED_BLOCKS and qkv.is_cuda and not self.training and getattr(self.qkv, "use_packed", False)
@@ -313,7 +313,7 @@ class Attention(nn.Module):
             return False
         from . import ops
 
-        return (qkv.shape[1] <= ops.ATTENTION_MAX_TOKENS and 0.0 < self.scale < math.inf
+        return (ops.attention_fits(qkv.shape[0], qkv.shape[1], self.num_heads) and 0.0 < self.scale < math.inf
                 and torch.autograd.forward_ad._current_level < 0)
 
     def forward(self, x):

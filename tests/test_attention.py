@@ -177,7 +177,8 @@ def test_block_attention_keeps_torch_outside_the_kernels_limits():
         qkv = SimpleNamespace(is_cuda=True, dtype=torch.float16, requires_grad=False, shape=(b, n, 192 * heads))
         return attn._attends_on_device(qkv)
 
-    assert takes(256, 197, 12) and takes(4, 288, 3, 2.5) and not takes(1, 289, 1)
+    assert takes(256, 197, 12) and takes(1 << 24, 1, 1) and takes(4, 288, 3, 2.5)
+    assert not takes((1 << 24) + 1, 1, 1) and not takes(1 << 23, 2, 3) and not takes(1, 289, 1)
     for scale in (0.0, -0.125, float("inf"), float("nan")):
         assert not takes(1, 8, 1, scale)
     attn = Attention(128, 2).eval()
