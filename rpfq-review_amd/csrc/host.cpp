@@ -51,6 +51,20 @@ bool vec(PyObject* o, int64_t n, const float** p) {
     return true;
 }
 
+// The numbers of a call: false where o is not one (the Python error goes).
+bool number(PyObject* o, int64_t* v) {
+    *v = PyLong_AsLongLong(o);
+    if (!PyErr_Occurred()) return true;
+    PyErr_Clear();
+    return false;
+}
+bool number(PyObject* o, float* v) {
+    *v = (float)PyFloat_AsDouble(o);
+    if (!PyErr_Occurred()) return true;
+    PyErr_Clear();
+    return false;
+}
+
 struct Call {
     const rpfq_wide_desc* d;
     const at::Tensor *blob, *x;
@@ -64,7 +78,9 @@ struct Call {
 // The operands the layer calls share: desc address, blob, x, residual, the
 // output's dtype (None: x's).  Makes y.
 bool layer(PyObject* desc, PyObject* blob, PyObject* x, PyObject* residual, PyObject* out_dtype, Call& c) {
-    c.d = static_cast<const rpfq_wide_desc*>(PyLong_AsVoidPtr(desc));
+    int64_t at;
+    if (!number(desc, &at)) return false;
+    c.d = reinterpret_cast<const rpfq_wide_desc*>(at);
     c.blob = plain(blob);
     c.x = plain(x);
     if (!c.d || !c.blob || !c.x || c.x->dim() < 1) return false;
@@ -103,22 +119,24 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Call c;
     const float* bias;
-    if (n != 8 || !layer(a[0], a[1], a[2], a[4], a[5], c) || !vec(a[3], 2 * c.d->n_complex, &bias)) Py_RETURN_NONE;
-    const int flags = (int)PyLong_AsLong(a[6]), guard = (int)PyLong_AsLong(a[7]);
+    int64_t flags, guard;
+    if (n != 8 || !number(a[6], &flags) || !number(a[7], &guard) || !layer(a[0], a[1], a[2], a[4], a[5], c) ||
+        !vec(a[3], 2 * c.d->n_complex, &bias))
+        Py_RETURN_NONE;
     const float* scale = nullptr;
     at::Tensor s;
     if (c.xdt != RPFQ_F16 && (guard & 1)) {
         const int64_t in = 2 * c.d->k_complex;
         int kernel = -1;
         if ((guard & 2) && in <= 4096 &&
-            rpfq_wide_linear_kernel(c.d, c.m, RPFQ_F16, c.ydt, flags, &kernel) == RPFQ_OK && kernel == RPFQ_KERNEL_DMA)
+            rpfq_wide_linear_kernel(c.d, c.m, RPFQ_F16, c.ydt, (int)flags, &kernel) == RPFQ_OK && kernel == RPFQ_KERNEL_DMA)
             Py_RETURN_NONE;
         s = at::empty({c.m}, c.x->options().dtype(at::kFloat));
         scale = s.const_data_ptr<float>();
         if (rpfq_row_scales(c.x->data_ptr(), c.xdt, c.m, in, s.data_ptr<float>(), c.stream) != RPFQ_OK) Py_RETURN_NONE;
     }
     return done(rpfq_wide_linear_scaled(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m, scale, bias, c.res,
-                                        c.y.data_ptr(), c.ydt, flags, c.stream),
+                                        c.y.data_ptr(), c.ydt, (int)flags, c.stream),
                 c.y);
     END_HANDLE_TH_ERRORS
 }
@@ -129,15 +147,16 @@ PyObject* layer_norm_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Call c;
     const float *w, *b, *bias;
+    float eps;
+    int64_t flags;
     int fusable = 0;
-    if (n != 9 || !layer(a[0], a[1], a[2], Py_None, a[7], c)) Py_RETURN_NONE;
+    if (n != 9 || !number(a[5], &eps) || !number(a[8], &flags) || !layer(a[0], a[1], a[2], Py_None, a[7], c)) Py_RETURN_NONE;
     const int64_t in = 2 * c.d->k_complex;
     if (!vec(a[3], in, &w) || !vec(a[4], in, &b) || !vec(a[6], 2 * c.d->n_complex, &bias) ||
         rpfq_layer_norm_wide_linear_fusable(c.d, c.m, c.xdt, c.ydt, &fusable) != RPFQ_OK || !fusable)
         Py_RETURN_NONE;
     return done(rpfq_layer_norm_wide_linear(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m, w, b,
-                                            (float)PyFloat_AsDouble(a[5]), bias, c.y.data_ptr(), c.ydt,
-                                            (int)PyLong_AsLong(a[8]), c.stream),
+                                            eps, bias, c.y.data_ptr(), c.ydt, (int)flags, c.stream),
                 c.y);
     END_HANDLE_TH_ERRORS
 }
@@ -148,13 +167,14 @@ PyObject* act_quant_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Call c;
     const float* bias;
+    int64_t bits, flags;
     int fusable = 0;
-    if (n != 8 || !layer(a[0], a[1], a[2], a[5], a[6], c) || !vec(a[4], 2 * c.d->n_complex, &bias) ||
+    if (n != 8 || !number(a[3], &bits) || !number(a[7], &flags) || !layer(a[0], a[1], a[2], a[5], a[6], c) || !vec(a[4], 2 * c.d->n_complex, &bias) ||
         rpfq_layer_norm_wide_linear_fusable(c.d, c.m, c.xdt, c.ydt, &fusable) != RPFQ_OK || !fusable)
         Py_RETURN_NONE;
     return done(rpfq_act_quant_wide_linear(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m,
-                                           (int)PyLong_AsLong(a[3]), 0, nullptr, nullptr, 0.0f, bias, c.res,
-                                           c.y.data_ptr(), c.ydt, (int)PyLong_AsLong(a[7]), c.stream),
+                                           (int)bits, 0, nullptr, nullptr, 0.0f, bias, c.res, c.y.data_ptr(), c.ydt,
+                                           (int)flags, c.stream),
                 c.y);
     END_HANDLE_TH_ERRORS
 }
@@ -162,12 +182,16 @@ PyObject* act_quant_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // attention(qkv, heads, scale)
 PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    const at::Tensor* q = n == 3 ? plain(a[0]) : nullptr;
-    const int64_t h = n == 3 ? PyLong_AsLongLong(a[1]) : 0;
-    if (!q || q->dim() != 3 || h < 1 || q->size(2) != 192 * h || q->numel() == 0 || !rows16(*q)) Py_RETURN_NONE;
+    int64_t h;
+    float scale;
+    if (n != 3 || !number(a[1], &h) || !number(a[2], &scale)) Py_RETURN_NONE;
+    const at::Tensor* q = plain(a[0]);
+    if (!q || q->dim() != 3 || h < 1 || q->size(2) != 192 * h ||
+        q->numel() == 0 || !rows16(*q))
+        Py_RETURN_NONE;
     at::Tensor y = at::empty({q->size(0), q->size(1), 64 * h}, q->options());
     return done(rpfq_attention(q->data_ptr(), dtype_code(q->scalar_type()), q->size(0), q->size(1), h, 64,
-                               (float)PyFloat_AsDouble(a[2]), y.data_ptr(),
+                               scale, y.data_ptr(),
                                c10::hip::getCurrentHIPStream(q->device().index()).stream()),
                 y);
     END_HANDLE_TH_ERRORS

@@ -108,3 +108,19 @@ def test_native_path_takes_device_tensors_only():
     assert host.linear(0, t, t, None, None, None, 0, 3) is None
     assert host.linear(t) is None
     assert host.attention(t, 1, 0.125) is None
+
+
+def test_native_path_leaves_other_numbers_to_python():
+    """Numbers of another kind (heads = 2.0) and too large ones are not taken,
+    and leave no Python error behind."""
+    from quant_models import _native as N
+
+    host = N.host()
+    t = torch.zeros(4, 64, dtype=torch.half)
+    assert host.attention(t, 2.0, 0.125) is None
+    assert host.attention(t, 2, "scale") is None
+    assert host.linear(1 << 80, t, t, None, None, None, 0, 3) is None
+    assert host.linear(0, t, t, None, None, None, 0.5, 3) is None
+    assert host.linear(0, t, t, None, None, None, 1 << 80, 3) is None
+    assert host.layer_norm_linear(0, t, t, None, None, None, None, None, 0) is None
+    assert host.act_quant_linear(0, t, t, "4", None, None, None, 0) is None
