@@ -773,6 +773,8 @@ def attention(qkv: torch.Tensor, num_heads: int, scale: float) -> torch.Tensor:
         out = host.attention(qkv, num_heads, float(scale))
         if out is not None:
             return out
+    if qkv.dim() != 3 or num_heads < 1 or qkv.shape[2] % (3 * num_heads):
+        raise ValueError(f"qkv must be [B, N, 3 C] with C a multiple of {num_heads} heads, got {tuple(qkv.shape)}")
     N.require_device(qkv)
     b, n, c3 = qkv.shape
     c = c3 // 3

@@ -201,3 +201,13 @@ def test_attention_argument_errors():
     assert lib.rpfq_attention(ctypes.c_void_p(4098), N.F16, 1, 8, 1, 64, 0.125, p, None) == 3
     for scale in (0.0, -0.125, float("nan"), float("inf")):
         assert lib.rpfq_attention(p, N.F16, 1, 8, 1, 64, scale, p, None) == 6
+
+
+def test_attention_refuses_heads_that_do_not_divide_the_row():
+    """387 values are not 3 x 2 heads of 64: the kernel would walk shorter
+    tokens than there are."""
+    from quant_models import ops
+
+    for shape, heads in (((2, 20, 387), 2), ((2, 20, 384), 0), ((2, 20, 384), 5), ((20, 384), 2)):
+        with pytest.raises(ValueError, match="heads"):
+            ops.attention(torch.zeros(*shape, dtype=torch.half), heads, 0.125)
