@@ -13,6 +13,8 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <cstring>
+
 #include "../../include/rpfq.h"
 
 namespace {
@@ -20,6 +22,26 @@ namespace {
 // Launches of at least this many operations are left to the Python path,
 // which chooses between more kernels; the host is not what bounds them.
 constexpr double kMostOps = 1.5e9;
+
+// The C ABI as the library that _native.load() opened exports it: this module
+// links none, so that another build of the library (RPFQ_LIBRARY) serves these
+// calls too.  Null until bind().
+#define RPFQ_HOST_CALLS(X)                                                                              \
+    X(rpfq_wide_linear_kernel) X(rpfq_row_scales) X(rpfq_wide_linear_scaled)                            \
+    X(rpfq_layer_norm_wide_linear_fusable) X(rpfq_layer_norm_wide_linear) X(rpfq_act_quant_wide_linear) \
+    X(rpfq_attention)
+struct Api {
+#define X(f) decltype(&::f) f;
+    RPFQ_HOST_CALLS(X)
+#undef X
+} api = {};
+constexpr const char* kCalls[] = {
+#define X(f) #f,
+    RPFQ_HOST_CALLS(X)
+#undef X
+};
+constexpr Py_ssize_t kNumCalls = sizeof(kCalls) / sizeof(kCalls[0]);
+static_assert(sizeof(Api) == kNumCalls * sizeof(void*), "one pointer per call");
 
 int dtype_code(at::ScalarType t) {
     switch (t) {
@@ -79,7 +101,7 @@ struct Call {
 // output's dtype (None: x's).  Makes y.
 bool layer(PyObject* desc, PyObject* blob, PyObject* x, PyObject* residual, PyObject* out_dtype, Call& c) {
     int64_t at;
-    if (!number(desc, &at)) return false;
+    if (!api.rpfq_attention || !number(desc, &at)) return false;
     c.d = reinterpret_cast<const rpfq_wide_desc*>(at);
     c.blob = plain(blob);
     c.x = plain(x);
@@ -129,13 +151,13 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t in = 2 * c.d->k_complex;
         int kernel = -1;
         if ((guard & 2) && in <= 4096 &&
-            rpfq_wide_linear_kernel(c.d, c.m, RPFQ_F16, c.ydt, (int)flags, &kernel) == RPFQ_OK && kernel == RPFQ_KERNEL_DMA)
+            api.rpfq_wide_linear_kernel(c.d, c.m, RPFQ_F16, c.ydt, (int)flags, &kernel) == RPFQ_OK && kernel == RPFQ_KERNEL_DMA)
             Py_RETURN_NONE;
         s = at::empty({c.m}, c.x->options().dtype(at::kFloat));
         scale = s.const_data_ptr<float>();
-        if (rpfq_row_scales(c.x->data_ptr(), c.xdt, c.m, in, s.data_ptr<float>(), c.stream) != RPFQ_OK) Py_RETURN_NONE;
+        if (api.rpfq_row_scales(c.x->data_ptr(), c.xdt, c.m, in, s.data_ptr<float>(), c.stream) != RPFQ_OK) Py_RETURN_NONE;
     }
-    return done(rpfq_wide_linear_scaled(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m, scale, bias, c.res,
+    return done(api.rpfq_wide_linear_scaled(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m, scale, bias, c.res,
                                         c.y.data_ptr(), c.ydt, (int)flags, c.stream),
                 c.y);
     END_HANDLE_TH_ERRORS
@@ -153,9 +175,9 @@ PyObject* layer_norm_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 9 || !number(a[5], &eps) || !number(a[8], &flags) || !layer(a[0], a[1], a[2], Py_None, a[7], c)) Py_RETURN_NONE;
     const int64_t in = 2 * c.d->k_complex;
     if (!vec(a[3], in, &w) || !vec(a[4], in, &b) || !vec(a[6], 2 * c.d->n_complex, &bias) ||
-        rpfq_layer_norm_wide_linear_fusable(c.d, c.m, c.xdt, c.ydt, &fusable) != RPFQ_OK || !fusable)
+        api.rpfq_layer_norm_wide_linear_fusable(c.d, c.m, c.xdt, c.ydt, &fusable) != RPFQ_OK || !fusable)
         Py_RETURN_NONE;
-    return done(rpfq_layer_norm_wide_linear(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m, w, b,
+    return done(api.rpfq_layer_norm_wide_linear(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m, w, b,
                                             eps, bias, c.y.data_ptr(), c.ydt, (int)flags, c.stream),
                 c.y);
     END_HANDLE_TH_ERRORS
@@ -170,9 +192,9 @@ PyObject* act_quant_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     int64_t bits, flags;
     int fusable = 0;
     if (n != 8 || !number(a[3], &bits) || !number(a[7], &flags) || !layer(a[0], a[1], a[2], a[5], a[6], c) || !vec(a[4], 2 * c.d->n_complex, &bias) ||
-        rpfq_layer_norm_wide_linear_fusable(c.d, c.m, c.xdt, c.ydt, &fusable) != RPFQ_OK || !fusable)
+        api.rpfq_layer_norm_wide_linear_fusable(c.d, c.m, c.xdt, c.ydt, &fusable) != RPFQ_OK || !fusable)
         Py_RETURN_NONE;
-    return done(rpfq_act_quant_wide_linear(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m,
+    return done(api.rpfq_act_quant_wide_linear(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m,
                                            (int)bits, 0, nullptr, nullptr, 0.0f, bias, c.res, c.y.data_ptr(), c.ydt,
                                            (int)flags, c.stream),
                 c.y);
@@ -185,19 +207,39 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     int64_t h;
     float scale;
     if (n != 3 || !number(a[1], &h) || !number(a[2], &scale)) Py_RETURN_NONE;
-    const at::Tensor* q = plain(a[0]);
+    const at::Tensor* q = api.rpfq_attention ? plain(a[0]) : nullptr;
     if (!q || q->dim() != 3 || h < 1 || q->size(2) != 192 * h ||
         q->numel() == 0 || !rows16(*q))
         Py_RETURN_NONE;
     at::Tensor y = at::empty({q->size(0), q->size(1), 64 * h}, q->options());
-    return done(rpfq_attention(q->data_ptr(), dtype_code(q->scalar_type()), q->size(0), q->size(1), h, 64,
+    return done(api.rpfq_attention(q->data_ptr(), dtype_code(q->scalar_type()), q->size(0), q->size(1), h, 64,
                                scale, y.data_ptr(),
                                c10::hip::getCurrentHIPStream(q->device().index()).stream()),
                 y);
     END_HANDLE_TH_ERRORS
 }
 
+// bind(addresses): the functions named by CALLS, in that order.
+PyObject* bind(PyObject*, PyObject* addresses) {
+    Api next;
+    if (!PyTuple_Check(addresses) || PyTuple_GET_SIZE(addresses) != kNumCalls) {
+        PyErr_SetString(PyExc_ValueError, "bind takes a tuple of one address per name in CALLS");
+        return nullptr;
+    }
+    for (Py_ssize_t i = 0; i < kNumCalls; ++i) {
+        void* f = PyLong_AsVoidPtr(PyTuple_GET_ITEM(addresses, i));
+        if (!f) {
+            if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind: a null address");
+            return nullptr;
+        }
+        std::memcpy(reinterpret_cast<char*>(&next) + i * sizeof(void*), &f, sizeof(f));
+    }
+    api = next;
+    Py_RETURN_NONE;
+}
+
 PyMethodDef methods[] = {
+    {"bind", bind, METH_O, nullptr},
     {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(linear)), METH_FASTCALL, nullptr},
     {"layer_norm_linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(layer_norm_linear)), METH_FASTCALL, nullptr},
     {"act_quant_linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(act_quant_linear)), METH_FASTCALL, nullptr},
@@ -208,4 +250,18 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, null
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host(void) {
+    PyObject* m = PyModule_Create(&module);
+    PyObject* names = m ? PyTuple_New(kNumCalls) : nullptr;
+    for (Py_ssize_t i = 0; names && i < kNumCalls; ++i) {
+        PyObject* name = PyUnicode_FromString(kCalls[i]);
+        if (!name) Py_CLEAR(names);
+        else PyTuple_SET_ITEM(names, i, name);
+    }
+    if (!names || PyModule_AddObject(m, "CALLS", names) < 0) {
+        Py_XDECREF(names);
+        Py_XDECREF(m);
+        return nullptr;
+    }
+    return m;
+}

@@ -230,12 +230,14 @@ _host = None
 
 def host():
     """The native host path of short launches (csrc/host.cpp), or None where
-    it was not built: callers then go through ctypes."""
+    it was not built: callers then go through ctypes.  It calls the library
+    that load() opened."""
     global _host
     if _host is None:
-        load()
+        lib = load()
         try:
             from . import _host as module
+            module.bind(tuple(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in module.CALLS))
         except ImportError:
             module = False
         _host = module

@@ -124,3 +124,27 @@ def test_native_path_leaves_other_numbers_to_python():
     assert host.linear(0, t, t, None, None, None, 1 << 80, 3) is None
     assert host.layer_norm_linear(0, t, t, None, None, None, None, None, 0) is None
     assert host.act_quant_linear(0, t, t, "4", None, None, None, 0) is None
+
+
+def test_native_path_calls_the_library_that_was_loaded(tmp_path):
+    """RPFQ_LIBRARY names another build: the default one is not loaded beside
+    it, so every call of the process runs the named one."""
+    import os
+    import shutil
+    import subprocess
+    import sys
+
+    from quant_models import _native as N
+
+    other = tmp_path / "librpfq_other.so"
+    shutil.copy(N.library_path(), other)
+    code = ("from quant_models import _native as N; host = N.host(); assert host is not None; "
+            "print(*sorted({l.split()[-1] for l in open('/proc/self/maps') if 'librpfq' in l}))")
+    env = dict(os.environ, RPFQ_LIBRARY=str(other), PYTHONPATH=os.path.dirname(os.path.dirname(N.__file__)))
+    out = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stderr
+    assert out.stdout.split() == [str(other)]
+    host = N.host()
+    for bad in ((), (0,) * len(host.CALLS), (1 << 80,) * len(host.CALLS), [1]):
+        with pytest.raises((ValueError, OverflowError)):
+            host.bind(bad)
