@@ -129,6 +129,21 @@ bool layer(PyObject* desc, PyObject* blob, PyObject* x, PyObject* residual, PyOb
     return true;
 }
 
+// Launches run without the interpreter lock, as through ctypes: one that waits
+// for room in the queue must not hold up the other threads, or a host function
+// in that queue that needs the lock.
+struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    Unlocked() = default;
+    Unlocked(const Unlocked&) = delete;
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+template <class F, class... A>
+int launch(F f, A... a) {
+    Unlocked u;
+    return f(a...);
+}
+
 PyObject* done(int rc, const at::Tensor& y) {
     if (rc != RPFQ_OK) Py_RETURN_NONE;
     return THPVariable_Wrap(y);
@@ -155,10 +170,11 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
             Py_RETURN_NONE;
         s = at::empty({c.m}, c.x->options().dtype(at::kFloat));
         scale = s.const_data_ptr<float>();
-        if (api.rpfq_row_scales(c.x->data_ptr(), c.xdt, c.m, in, s.data_ptr<float>(), c.stream) != RPFQ_OK) Py_RETURN_NONE;
+        if (launch(api.rpfq_row_scales, c.x->data_ptr(), c.xdt, c.m, in, s.data_ptr<float>(), c.stream) != RPFQ_OK)
+            Py_RETURN_NONE;
     }
-    return done(api.rpfq_wide_linear_scaled(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m, scale, bias, c.res,
-                                        c.y.data_ptr(), c.ydt, (int)flags, c.stream),
+    return done(launch(api.rpfq_wide_linear_scaled, c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m,
+                       scale, bias, c.res, c.y.data_ptr(), c.ydt, (int)flags, c.stream),
                 c.y);
     END_HANDLE_TH_ERRORS
 }
@@ -177,8 +193,8 @@ PyObject* layer_norm_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!vec(a[3], in, &w) || !vec(a[4], in, &b) || !vec(a[6], 2 * c.d->n_complex, &bias) ||
         api.rpfq_layer_norm_wide_linear_fusable(c.d, c.m, c.xdt, c.ydt, &fusable) != RPFQ_OK || !fusable)
         Py_RETURN_NONE;
-    return done(api.rpfq_layer_norm_wide_linear(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m, w, b,
-                                            eps, bias, c.y.data_ptr(), c.ydt, (int)flags, c.stream),
+    return done(launch(api.rpfq_layer_norm_wide_linear, c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt,
+                       c.m, w, b, eps, bias, c.y.data_ptr(), c.ydt, (int)flags, c.stream),
                 c.y);
     END_HANDLE_TH_ERRORS
 }
@@ -194,9 +210,8 @@ PyObject* act_quant_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 8 || !number(a[3], &bits) || !number(a[7], &flags) || !layer(a[0], a[1], a[2], a[5], a[6], c) || !vec(a[4], 2 * c.d->n_complex, &bias) ||
         api.rpfq_layer_norm_wide_linear_fusable(c.d, c.m, c.xdt, c.ydt, &fusable) != RPFQ_OK || !fusable)
         Py_RETURN_NONE;
-    return done(api.rpfq_act_quant_wide_linear(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m,
-                                           (int)bits, 0, nullptr, nullptr, 0.0f, bias, c.res, c.y.data_ptr(), c.ydt,
-                                           (int)flags, c.stream),
+    return done(launch(api.rpfq_act_quant_wide_linear, c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt,
+                       c.m, (int)bits, 0, nullptr, nullptr, 0.0f, bias, c.res, c.y.data_ptr(), c.ydt, (int)flags, c.stream),
                 c.y);
     END_HANDLE_TH_ERRORS
 }
@@ -212,9 +227,8 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
         q->numel() == 0 || !rows16(*q))
         Py_RETURN_NONE;
     at::Tensor y = at::empty({q->size(0), q->size(1), 64 * h}, q->options());
-    return done(api.rpfq_attention(q->data_ptr(), dtype_code(q->scalar_type()), q->size(0), q->size(1), h, 64,
-                               scale, y.data_ptr(),
-                               c10::hip::getCurrentHIPStream(q->device().index()).stream()),
+    return done(launch(api.rpfq_attention, q->data_ptr(), dtype_code(q->scalar_type()), q->size(0), q->size(1), h, 64,
+                       scale, y.data_ptr(), c10::hip::getCurrentHIPStream(q->device().index()).stream()),
                 y);
     END_HANDLE_TH_ERRORS
 }

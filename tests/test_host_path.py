@@ -99,6 +99,63 @@ def test_native_path_runs_on_the_current_stream():
         assert torch.equal(y, pw.linear(x))
 
 
+@pytest.mark.gpu
+def test_native_path_launches_without_the_interpreter_lock():
+    """Every launch function of the native path replaced by the interpreter's
+    own PyGILState_Check: 0 (the lock is free), read as success, or 1, read as
+    a refused call."""
+    import ctypes
+
+    from quant_models import _native as N
+
+    pw, g = _layer(384, 384)
+    x = torch.randn(20, 768, device=DEV, generator=g).half()
+    host, lib, d = N.host(), N.load(), ctypes.addressof(pw.desc)
+    address = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in host.CALLS}
+    check = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+    # these two choose a kernel and launch nothing
+    chooses = ("rpfq_wide_linear_kernel", "rpfq_layer_norm_wide_linear_fusable")
+    host.bind(tuple(address[name] if name in chooses else check for name in host.CALLS))
+    try:
+        taken = [host.linear(d, pw.blob, x, None, None, None, 0, 3), host.linear(d, pw.blob, x.float(), None, None, None, 0, 1),
+                 host.layer_norm_linear(d, pw.blob, x, None, None, 1e-5, None, None, 0),
+                 host.act_quant_linear(d, pw.blob, x, 4, None, None, None, 0),
+                 host.attention(x.new_zeros(1, 5, 192), 1, 0.125)]
+    finally:
+        host.bind(tuple(address[name] for name in host.CALLS))
+    assert pw.ln_fusable(20, torch.float16)
+    assert all(t is not None for t in taken)
+
+
+@pytest.mark.gpu
+def test_native_path_from_several_threads():
+    """Threads on their own streams get the results of one thread."""
+    import threading
+
+    from quant_models import ops
+
+    pw, g = _layer(96, 96)
+    xs = [torch.randn(1 + 3 * t, 192, device=DEV, generator=g).half() for t in range(4)]
+    qkv = [torch.randn(1, 5 + 40 * t, 384, device=DEV, generator=g).half() for t in range(4)]
+    want = [(pw.linear(x), ops.attention(q, 2, 0.125)) for x, q in zip(xs, qkv)]
+    torch.cuda.synchronize()
+    same = [False] * 4
+
+    def work(t):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            got = [(pw.linear(xs[t]), ops.attention(qkv[t], 2, 0.125)) for _ in range(200)]
+        s.synchronize()
+        same[t] = all(torch.equal(a, b) for pair in got for a, b in zip(pair, want[t]))
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(same)
+
+
 def test_native_path_takes_device_tensors_only():
     from quant_models import _native as N
 
