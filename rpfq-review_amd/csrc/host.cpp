@@ -93,12 +93,19 @@ struct Call {
     const void* res = nullptr;
     int64_t m = 0;
     int xdt = 0, ydt = 0;
+    at::ScalarType yt{};
+    c10::SmallVector<int64_t, 6> shape;
     at::Tensor y;
     void* stream = nullptr;
+    // the output and the stream, once it is known that the call is taken here
+    void take() {
+        y = at::empty(shape, x->options().dtype(yt));
+        stream = c10::hip::getCurrentHIPStream(x->device().index()).stream();
+    }
 };
 
 // The operands the layer calls share: desc address, blob, x, residual, the
-// output's dtype (None: x's).  Makes y.
+// output's dtype (None: x's).
 bool layer(PyObject* desc, PyObject* blob, PyObject* x, PyObject* residual, PyObject* out_dtype, Call& c) {
     int64_t at;
     if (!api.rpfq_attention || !number(desc, &at)) return false;
@@ -109,23 +116,21 @@ bool layer(PyObject* desc, PyObject* blob, PyObject* x, PyObject* residual, PyOb
     const int64_t in = 2 * c.d->k_complex, out = 2 * c.d->n_complex;
     if (c.x->size(-1) != in || !rows16(*c.x)) return false;
     c.m = c.x->numel() / in;
-    at::ScalarType yt = c.x->scalar_type();
+    c.yt = c.x->scalar_type();
     if (out_dtype != Py_None) {
         if (!THPDtype_Check(out_dtype)) return false;
-        yt = reinterpret_cast<THPDtype*>(out_dtype)->scalar_type;
+        c.yt = reinterpret_cast<THPDtype*>(out_dtype)->scalar_type;
     }
     c.xdt = dtype_code(c.x->scalar_type());
-    c.ydt = dtype_code(yt);
+    c.ydt = dtype_code(c.yt);
     if (c.m < 1 || c.xdt < 0 || c.ydt < 0 || 2.0 * (double)c.m * (double)in * (double)out >= kMostOps) return false;
-    c10::SmallVector<int64_t, 6> shape(c.x->sizes().begin(), c.x->sizes().end());
-    shape.back() = out;
+    c.shape.assign(c.x->sizes().begin(), c.x->sizes().end());
+    c.shape.back() = out;
     if (residual != Py_None) {
         const at::Tensor* r = plain(residual);
-        if (!r || r->scalar_type() != yt || r->sizes() != at::IntArrayRef(shape) || !rows16(*r)) return false;
+        if (!r || r->scalar_type() != c.yt || r->sizes() != at::IntArrayRef(c.shape) || !rows16(*r)) return false;
         c.res = r->data_ptr();
     }
-    c.y = at::empty(shape, c.x->options().dtype(yt));
-    c.stream = c10::hip::getCurrentHIPStream(c.x->device().index()).stream();
     return true;
 }
 
@@ -162,12 +167,14 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
         Py_RETURN_NONE;
     const float* scale = nullptr;
     at::Tensor s;
-    if (c.xdt != RPFQ_F16 && (guard & 1)) {
-        const int64_t in = 2 * c.d->k_complex;
-        int kernel = -1;
-        if ((guard & 2) && in <= 4096 &&
-            api.rpfq_wide_linear_kernel(c.d, c.m, RPFQ_F16, c.ydt, (int)flags, &kernel) == RPFQ_OK && kernel == RPFQ_KERNEL_DMA)
-            Py_RETURN_NONE;
+    const int64_t in = 2 * c.d->k_complex;
+    const bool scaled = c.xdt != RPFQ_F16 && (guard & 1);
+    int kernel = -1;
+    if (scaled && (guard & 2) && in <= 4096 &&
+        api.rpfq_wide_linear_kernel(c.d, c.m, RPFQ_F16, c.ydt, (int)flags, &kernel) == RPFQ_OK && kernel == RPFQ_KERNEL_DMA)
+        Py_RETURN_NONE;
+    c.take();
+    if (scaled) {
         s = at::empty({c.m}, c.x->options().dtype(at::kFloat));
         scale = s.const_data_ptr<float>();
         if (launch(api.rpfq_row_scales, c.x->data_ptr(), c.xdt, c.m, in, s.data_ptr<float>(), c.stream) != RPFQ_OK)
@@ -193,6 +200,7 @@ PyObject* layer_norm_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!vec(a[3], in, &w) || !vec(a[4], in, &b) || !vec(a[6], 2 * c.d->n_complex, &bias) ||
         api.rpfq_layer_norm_wide_linear_fusable(c.d, c.m, c.xdt, c.ydt, &fusable) != RPFQ_OK || !fusable)
         Py_RETURN_NONE;
+    c.take();
     return done(launch(api.rpfq_layer_norm_wide_linear, c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt,
                        c.m, w, b, eps, bias, c.y.data_ptr(), c.ydt, (int)flags, c.stream),
                 c.y);
@@ -210,6 +218,7 @@ PyObject* act_quant_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 8 || !number(a[3], &bits) || !number(a[7], &flags) || !layer(a[0], a[1], a[2], a[5], a[6], c) || !vec(a[4], 2 * c.d->n_complex, &bias) ||
         api.rpfq_layer_norm_wide_linear_fusable(c.d, c.m, c.xdt, c.ydt, &fusable) != RPFQ_OK || !fusable)
         Py_RETURN_NONE;
+    c.take();
     return done(launch(api.rpfq_act_quant_wide_linear, c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt,
                        c.m, (int)bits, 0, nullptr, nullptr, 0.0f, bias, c.res, c.y.data_ptr(), c.ydt, (int)flags, c.stream),
                 c.y);

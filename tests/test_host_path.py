@@ -100,6 +100,31 @@ def test_native_path_runs_on_the_current_stream():
 
 
 @pytest.mark.gpu
+def test_native_path_allocates_nothing_for_calls_it_leaves(monkeypatch):
+    """A call that goes on to the Python path allocates what it allocates there."""
+    from quant_models import _native as N
+
+    pw, g = _layer(384, 384)
+    x = torch.randn(1576, 768, device=DEV, generator=g).bfloat16()  # prescaled rows, the DMA kernel
+    half = torch.randn(8, 768, device=DEV, generator=g).half()
+    calls = [lambda: pw.linear(x), lambda: pw.linear(half, torch.ones(768, device=DEV).double()),
+             lambda: pw.layer_norm_linear(half.expand(4, 8, 768).contiguous(), torch.ones(768, device=DEV).double(), None, 1e-5)]
+    assert pw.kernel_for(1576, torch.float16, torch.bfloat16) == N.KERNEL_DMA
+
+    def count(f):
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        f()
+        return torch.cuda.memory_stats()["allocation.all.allocated"] - before
+
+    for f in calls:
+        f()
+        native = count(f)
+        with monkeypatch.context() as m:
+            m.setattr(N, "_host", False)
+            assert native == count(f)
+
+
+@pytest.mark.gpu
 def test_native_path_launches_without_the_interpreter_lock():
     """Every launch function of the native path replaced by the interpreter's
     own PyGILState_Check: 0 (the lock is free), read as success, or 1, read as
