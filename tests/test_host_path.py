@@ -230,3 +230,23 @@ def test_native_path_calls_the_library_that_was_loaded(tmp_path):
     for bad in ((), (0,) * len(host.CALLS), (1 << 80,) * len(host.CALLS), [1]):
         with pytest.raises((ValueError, OverflowError)):
             host.bind(bad)
+
+
+def test_native_path_is_built_for_the_installed_torch():
+    """Another torch rebuilds it; without torch's headers the library is built
+    and the native path left out."""
+    import os
+    import subprocess
+
+    from quant_models import _native as N
+
+    csrc = os.path.join(os.path.dirname(N.library_path()), "csrc")
+
+    def plan(*args):
+        out = subprocess.run(["make", "-n", "-C", csrc, *args], capture_output=True, text=True, timeout=120)
+        assert out.returncode == 0, out.stderr
+        return out.stdout
+
+    assert "host.cpp" in plan("TORCH_VERSION=0.0.other")
+    without = plan("-B", "TORCH=/nonexistent")
+    assert "host.cpp" not in without and "librpfq.so" in without
