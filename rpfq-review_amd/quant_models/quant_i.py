@@ -483,11 +483,20 @@ def records_grad(module: nn.Module, x: torch.Tensor) -> bool:
     return torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in module.parameters()))
 
 
+def _transformed(t: torch.Tensor) -> bool:
+    """t stands for other tensors (a batch of vmap, a dual number): its values
+    are reached by torch's operators only."""
+    functorch = torch._C._functorch
+    return (functorch.is_functorch_wrapped_tensor(t) or functorch.is_legacy_batchedtensor(t)
+            or torch.autograd.forward_ad.unpack_dual(t).tangent is not None)
+
+
 class _SplitLinearFn(torch.autograd.Function):
     """F.linear of float32 x and A_q on the split-fp16 matrix-core kernels
     (rpfq_linear_f32, float32 accuracy); the bias gradient is the column sum,
     taken in the pass that splits grad_y.
-    A backward that autograd records (create_graph) runs torch's products."""
+    A backward that autograd records (create_graph), batches (vmap,
+    is_grads_batched) or differentiates forward runs torch's products."""
 
     @staticmethod
     def forward(ctx, x, w, bias, parts):
@@ -507,7 +516,7 @@ class _SplitLinearFn(torch.autograd.Function):
         g2, x2 = grad.reshape(-1, grad.shape[-1]), x.reshape(-1, x.shape[-1])
         want_x, want_w = ctx.needs_input_grad[:2]
         want_b, gb = ctx.has_bias and ctx.needs_input_grad[2], None
-        if torch.is_grad_enabled():
+        if torch.is_grad_enabled() or _transformed(grad):
             gx = g2 @ w if want_x else None
             gw = g2.t() @ x2 if want_w else None
         elif want_x or want_w:

@@ -181,6 +181,31 @@ def test_training_layer_double_backward_and_forward_mode():
     assert torch.allclose(ty, t @ a.t(), rtol=1e-4, atol=1e-4)
 
 
+def test_transformed_gradients_take_torch_products(monkeypatch):
+    """Batched gradients (is_grads_batched, vmap) and dual ones reach the
+    backward as tensors without memory of their own: torch's products, as
+    behind F.linear."""
+    from quant_models import ops
+    from quant_models.quant_i import _SplitLinearFn
+
+    monkeypatch.setattr(ops, "linear_f32", lambda x, w, b, parts: (torch.nn.functional.linear(x, w, b), x.new_ones(len(x))))
+    monkeypatch.setattr(ops, "linear_f32_grad", lambda *a: pytest.fail("the kernels were given a transformed gradient"))
+    x, w, b, _ = (t.requires_grad_(True) for t in _inputs(6, 4, 8, dev="cpu"))
+    gys = torch.randn(3, 6, 4)
+    y = _SplitLinearFn.apply(x, w, b, torch.ones(1))
+    ref = torch.nn.functional.linear(x, w, b)
+    want = torch.autograd.grad(ref, (x, w, b), gys, is_grads_batched=True, retain_graph=True)
+    got = torch.autograd.grad(y, (x, w, b), gys, is_grads_batched=True, retain_graph=True)
+    mapped = torch.func.vmap(lambda g: torch.autograd.grad(y, (x, w, b), g, retain_graph=True))(gys)
+    for a, c, d in zip(want, got, mapped):
+        assert torch.allclose(a, c) and torch.allclose(a, d)
+    with torch.autograd.forward_ad.dual_level():
+        g = torch.autograd.forward_ad.make_dual(gys[0], gys[1])
+        for a, c in zip(torch.autograd.grad(y, (x, w, b), g), torch.autograd.grad(ref, (x, w, b), g)):
+            a, c = torch.autograd.forward_ad.unpack_dual(a), torch.autograd.forward_ad.unpack_dual(c)
+            assert torch.allclose(a.primal, c.primal) and torch.allclose(a.tangent, c.tangent)
+
+
 @pytest.mark.gpu
 def test_operands_that_do_not_fit_are_refused():
     """By F.linear's own error from the layer, by the host checks below it."""
