@@ -381,11 +381,12 @@ class _HipWideQuantSTE(torch.autograd.Function):
         if ctx.rotated:
             ctx.save_for_backward(weight, a_q)
         ctx.mark_non_differentiable(scales)
+        ctx.set_materialize_grads(False)  # else every backward fills zeros for the scales
         return a_q, scales
 
     @staticmethod
     def backward(ctx, grad, _):
-        if not ctx.rotated:
+        if grad is None or not ctx.rotated:
             return grad, None, None, None
         weight, a_q = ctx.saved_tensors
         th_u, th_w = rotation_grad(grad.float(), weight.detach(), a_q)

@@ -33,6 +33,32 @@ def _rot_cos_sin(tu, tw):
     return tuple(out)
 
 
+@pytest.mark.parametrize("rotated", [False, True])
+def test_quantizer_backward_fills_nothing_for_its_scales(rotated, monkeypatch):
+    """The scales carry no gradient, and none is made for them: the backward
+    allocates and fills no zeros."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from quant_models import ops, quant_i
+
+    monkeypatch.setattr(ops, "quantize_wide", lambda w, *spec, rot=None: (w * 1.0, w.new_ones(16), None))
+    made = []
+
+    class Record(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if "zeros" in str(func) or "fill" in str(func):
+                made.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    w = torch.randn(8, 12, requires_grad=True)
+    theta = [torch.zeros(1, requires_grad=True) if rotated else None for _ in range(2)]
+    a_q, _ = quant_i._HipWideQuantSTE.apply(w, *theta, ("axis", 2, "axis", 2))
+    g = torch.randn(8, 12)
+    with Record():
+        a_q.backward(g)
+    assert torch.equal(w.grad, g) and not made
+
+
 # ---------------------------------------------------------------------------
 # CPU: straight-through gradients of the rotation
 # ---------------------------------------------------------------------------
