@@ -24,6 +24,12 @@ namespace rpfq {
 // the step's 32 h values, then its 32 l values, so a step's tile row is one
 // 128-byte line.  Rows and columns past the matrix are zero.
 constexpr int kF32NoRow = -100000;
+// What the passes of a call leave for the ones behind them, in its workspace.
+struct F32Words {
+    int emax;   // gw: largest exponent of a row's product of maxima, or kF32NoRow
+    int bad;    // gw: a row of x or gy has inf or NaN
+    int rows;   // rows of y / gx that f32_exact_rows_kernel writes
+};
 // Most blocks of the gy pass where it also sums columns: 4 a CU.
 constexpr int kColBlocks = 1024;
 
@@ -33,10 +39,11 @@ __device__ __forceinline__ int f32_scale_exp(float s) {  // s = 2^e
 
 // One wave per row, the row in registers (K <= 4096).  MODE 0: the row's own
 // scale 2^e (largest magnitude in [2^14, 2^15)), written to scale[m]; +inf
-// for a zero row, 0 for one with inf or NaN (its planes are zeroed).
+// for a zero row, 0 for one with inf or NaN (its planes are zeroed, and it goes
+// to the list of exact rows).
 // MODE 1 (gy): also collects over the rows the largest exponent of x's rows
-// over r (word[0]) and whether any row of x or gy is non-finite (word[1]).
-// MODE 2 (x of gw): times 1 / r[m], r = gscale, and 2^-word[0].
+// over r (emax) and whether any row of x or gy is non-finite (bad).
+// MODE 2 (x of gw): times 1 / r[m], r = gscale, and 2^-emax.
 // COLS (gy): also the column sums of the block's rows, colsum[block][K], for
 // the bias gradient: each lane adds the values it holds anyway (a separate
 // reduction over 12,608 x 3,072 reads 155 MB again, 40.6 us; here 7.5 us and
@@ -44,11 +51,11 @@ __device__ __forceinline__ int f32_scale_exp(float s) {  // s = 2^e
 // HBM bound: 8 bytes per element.
 template <int NC, int MODE, bool COLS = false>
 __global__ void __launch_bounds__(256) f32_split_rows_kernel(const float* x, int64_t M, int64_t Mp, int K, int Kp,
-                                                            const float* xscale, const float* gscale, int* word,
-                                                            char* planes, float* scale, float* colsum) {
+                                                            const float* xscale, const float* gscale, F32Words* word,
+                                                            int* list, char* planes, float* scale, float* colsum) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int emax = kF32NoRow, bad = 0;
-    const int e2 = MODE == 2 ? word[0] : 0;
+    const int e2 = MODE == 2 ? word->emax : 0;
     f32x4 cs[NC][2];
     if (COLS) {
 #pragma unroll
@@ -86,7 +93,10 @@ __global__ void __launch_bounds__(256) f32_split_rows_kernel(const float* x, int
             zero = !in || mx == 0 || !fin;
             const float s = !fin ? 0.0f : mx == 0 ? __builtin_inff() : row_prescale(__uint_as_float(mx));
             k = zero ? 0 : f32_scale_exp(s);
-            if (in && lane == 0) scale[m] = s;
+            if (in && lane == 0) {
+                scale[m] = s;
+                if (!fin) list[atomicAdd(&word->rows, 1)] = (int)m;
+            }
             if (MODE == 1 && in) {
                 const float sx = xscale[m];
                 if (!fin || sx == 0.0f) bad = 1;
@@ -126,8 +136,8 @@ __global__ void __launch_bounds__(256) f32_split_rows_kernel(const float* x, int
         }
         __syncthreads();
         if (threadIdx.x == 0) {
-            atomicMax(word, max(max(sm[0], sm[1]), max(sm[2], sm[3])));
-            if (sm[4] | sm[5] | sm[6] | sm[7]) atomicOr(word + 1, 1);
+            atomicMax(&word->emax, max(max(sm[0], sm[1]), max(sm[2], sm[3])));
+            if (sm[4] | sm[5] | sm[6] | sm[7]) atomicOr(&word->bad, 1);
         }
     }
     if (COLS) {  // the four waves one after another, then one coalesced row
@@ -169,12 +179,12 @@ __global__ void __launch_bounds__(1024) f32_colsum_kernel(const float* parts, in
 // row r, contraction 8 g .. 8 g + 7.  TRANS = 0: rows = N, contraction = K;
 // 1: rows = K, contraction = N.  One thread per 16 bytes of h and l; zero
 // past the matrix.  The scale 2^e of w from the bound sum |parts| >= |w|
-// goes to wscale[0] (0 if that is not finite: every row is then recomputed);
-// block 0 also initialises gw's words.
+// goes to wscale[0] (0 if that is not finite: every row is then an exact one);
+// block 0 also initialises the words.
 template <int TRANS>
 __global__ void __launch_bounds__(256) f32_split_w_kernel(const float* w, int N, int K, int rows32, int kt,
                                                          const float* parts, int nparts, char* wf, float* wscale,
-                                                         int* word) {
+                                                         F32Words* word) {
     float bound = 0.0f;
     for (int i = 0; i < nparts; ++i) bound += fabsf(parts[i]);
     const bool fin = bound <= 3.40282347e38f;
@@ -182,10 +192,7 @@ __global__ void __launch_bounds__(256) f32_split_w_kernel(const float* w, int N,
     const int k = f32_scale_exp(s);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         wscale[0] = fin ? s : 0.0f;
-        if (word) {
-            word[0] = kF32NoRow;
-            word[1] = 0;
-        }
+        *word = {kF32NoRow, 0, 0};
     }
     const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (id >= (int64_t)rows32 * kt * 64) return;
@@ -280,6 +287,7 @@ __device__ __forceinline__ void f32_store_block(char* epi, const floatx16& acc0,
 
 template <int MB>
 __global__ void __launch_bounds__(256, 2) f32_gemm_kernel(F32Args a) {
+    if (a.wscale[0] == 0.0f) return;  // every row is an exact one
     extern __shared__ __align__(16) char smem[];
     constexpr int BM = 32 * MB, RPW = BM / 4, XL = RPW / 8;  // rows and DMA loads per wave and step
     constexpr int STAGE = f32_stage<MB>();
@@ -426,19 +434,21 @@ __global__ void __launch_bounds__(256, 2) f32_gemm_kernel(F32Args a) {
 struct F32GwArgs {
     const char* gp;   // planes of gy
     const char* xp;   // planes of x
-    const int* word;
+    const F32Words* word;
     float* part;
     int64_t ldg, ldx;  // plane row bytes
     int N, K;
     int steps, per;    // 16-row steps in all, and per split
     int tiles_n, tiles_k, splits;
 };
+__device__ __forceinline__ bool gw_exact(const F32Words& w) { return w.bad != 0; }
 constexpr int kGwG = 16 * 512, kGwStage = kGwG + 16 * 1024;
 constexpr int kGwLds = 3 * kGwStage + 256;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* lds_s4_t;
 
 __global__ void __launch_bounds__(256, 2) f32_gw_kernel(F32GwArgs a) {
+    if (gw_exact(*a.word)) return;  // f32_exact_gw_kernel writes the partial sums
     extern __shared__ __align__(16) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -532,7 +542,7 @@ __global__ void __launch_bounds__(256, 2) f32_gw_kernel(F32GwArgs a) {
     }
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    const int e = a.splits == 1 && a.word[0] != kF32NoRow ? a.word[0] : 0;
+    const int e = a.splits == 1 && a.word->emax != kF32NoRow ? a.word->emax : 0;
     const int64_t k0 = (int64_t)tk * 256 + 64 * wave;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -541,10 +551,10 @@ __global__ void __launch_bounds__(256, 2) f32_gw_kernel(F32GwArgs a) {
     }
 }
 
-// gw = 2^word[0] times the sum of the splits' partials, in their order.
-__global__ void __launch_bounds__(256) f32_gw_reduce_kernel(const float* part, int64_t n4, int splits, const int* word,
+// gw = 2^emax times the sum of the splits' partials, in their order.
+__global__ void __launch_bounds__(256) f32_gw_reduce_kernel(const float* part, int64_t n4, int splits, const F32Words* word,
                                                            float* gw) {
-    const int e = word[0] == kF32NoRow ? 0 : word[0];
+    const int e = word->emax == kF32NoRow || gw_exact(*word) ? 0 : word->emax;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)gridDim.x * 256) {
         f32x4 v = reinterpret_cast<const f32x4*>(part)[i];
         for (int s = 1; s < splits; ++s) v += reinterpret_cast<const f32x4*>(part)[i + s * n4];
@@ -555,38 +565,150 @@ __global__ void __launch_bounds__(256) f32_gw_reduce_kernel(const float* part, i
     }
 }
 
-// Rows with inf or NaN (scale 0), and every row when w's bound is not
-// finite: plain float32 sums, so that the special values come out as a
-// float32 GEMM's.  out[m, n] = sum_c a[m, c] b[n bn + c bc] + bias[n].
-__global__ void __launch_bounds__(256) f32_special_rows_kernel(const float* in, const float* b, const float* bias,
-                                                              float* out, int64_t M, int N, int C, int64_t bn,
-                                                              int64_t bc, const float* scale, const float* wscale) {
-    const bool all = wscale[0] == 0.0f;
-    for (int64_t base = (int64_t)blockIdx.x * 64; base < M; base += (int64_t)gridDim.x * 64) {
-        const int lane = threadIdx.x & 63;
-        const bool mine = base + lane < M && (all || scale[base + lane] == 0.0f);
-        uint64_t todo = __ballot(mine);
-        while (todo) {
-            const int64_t m = base + __builtin_ctzll(todo);
-            todo &= todo - 1;
-            for (int n = threadIdx.x; n < N; n += 256) {
-                float s = 0.0f;
-                for (int c = 0; c < C; ++c) s = fmaf(in[m * C + c], b[n * bn + c * bc], s);
-                out[m * N + n] = s + (bias ? bias[n] : 0.0f);
-            }
+// ---------------------------------------------------------------------------
+// exact rows: plain float32 sums
+// ---------------------------------------------------------------------------
+// Where split operands do not stand for their values (inf, NaN) the products
+// run on v_mfma_f32_32x32x2_f32, so that special values come out as a float32
+// GEMM's: the listed rows of y and gx, and all of gw.  1/16 of the fp16 rate;
+// with every row listed 12,608 x 3,072 x 768 takes 640 us a product (the
+// float32 library GEMM: 541), and an empty list one short launch.
+//
+// Tile: 128 rows i x 128 outputs j, 4 waves of 64 x 64, 16 of the contraction
+// c a step through two LDS buffers of odd row stride (17 floats: 32 rows of a
+// column on distinct banks), the next step's loads in registers meanwhile.
+// AC / BC: operand a / b lies with c contiguous (rows of lda), else with i / j
+// contiguous.  Sums of 512 products, then the sum of those.
+struct F32Exact {
+    const float* a;
+    const float* b;
+    const float* bias;  // of the outputs j, or NULL
+    float* out;         // [.., J]
+    const int* list;    // rows i of a and out, or NULL: as they are
+    int64_t lda, ldb;
+    int64_t I;
+    int J;
+};
+constexpr int kExLd = 17, kExHalf = 128 * kExLd;
+
+template <bool AC, bool BC>
+__device__ __forceinline__ void f32_exact_tile(const F32Exact& x, float* lds, int64_t i0, int j0, int64_t c0, int64_t c1) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r = lane & 31, g = lane >> 5, wi = (wave & 1) * 64, wj = (wave >> 1) * 64;
+    // two 4-float loads of each operand: (row q4, columns 4 qc ..) of the tile,
+    // or (contraction q, rows 4 qr ..)
+    const int q4 = tid >> 2, qc = 4 * (tid & 3), q = tid >> 5, qr = 4 * (tid & 31);
+    const float* ap[2];
+    const float* bp[2];
+    bool aok[2], bok[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const int64_t i = AC ? i0 + q4 + 64 * p : i0 + qr;
+        aok[p] = i < x.I;
+        const int64_t row = !aok[p] ? 0 : AC && x.list ? x.list[i] : i;
+        ap[p] = AC ? x.a + row * x.lda + qc : x.a + row;
+        const int j = BC ? j0 + q4 + 64 * p : j0 + qr;
+        bok[p] = j < x.J;
+        bp[p] = BC ? x.b + (int64_t)(bok[p] ? j : 0) * x.ldb + qc : x.b + (bok[p] ? j : 0);
+    }
+    f32x4 ra[2], rb[2];
+    auto load = [&](int64_t c) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            ra[p] = rb[p] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+            const int64_t ca = AC ? c + qc : c + q + 8 * p, cb = BC ? c + qc : c + q + 8 * p;
+            if (aok[p] && ca < c1) ra[p] = *reinterpret_cast<const f32x4*>(AC ? ap[p] + c : ap[p] + ca * x.lda);
+            if (bok[p] && cb < c1) rb[p] = *reinterpret_cast<const f32x4*>(BC ? bp[p] + c : bp[p] + cb * x.ldb);
         }
+    };
+    auto store = [&](float* d) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                d[AC ? (q4 + 64 * p) * kExLd + qc + e : (qr + e) * kExLd + q + 8 * p] = ra[p][e];
+                d[kExHalf + (BC ? (q4 + 64 * p) * kExLd + qc + e : (qr + e) * kExLd + q + 8 * p)] = rb[p][e];
+            }
+    };
+    floatx16 acc[2][2], sum[2][2];  // [j block][i block]
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[j][i] = sum[j][i] = floatx16{0};
+    __syncthreads();  // the tile before this one is read
+    load(c0);
+    store(lds);
+    __syncthreads();
+    int buf = 0, steps = 0;
+    for (int64_t c = c0; c < c1; c += 16) {
+        const bool more = c + 16 < c1;
+        if (more) load(c + 16);
+        const float* la = lds + buf * 2 * kExHalf + (wi + r) * kExLd + g;
+        const float* lb = lds + buf * 2 * kExHalf + kExHalf + (wj + r) * kExLd + g;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float a0 = la[2 * k], a1 = la[32 * kExLd + 2 * k], b0 = lb[2 * k], b1 = lb[32 * kExLd + 2 * k];
+            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(b0, a0, acc[0][0], 0, 0, 0);
+            acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(b0, a1, acc[0][1], 0, 0, 0);
+            acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(b1, a0, acc[1][0], 0, 0, 0);
+            acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(b1, a1, acc[1][1], 0, 0, 0);
+        }
+        if (++steps % 32 == 0) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    sum[j][i] += acc[j][i];
+                    acc[j][i] = floatx16{0};
+                }
+        }
+        if (more) store(lds + (buf ^ 1) * 2 * kExHalf);
+        __syncthreads();
+        buf ^= 1;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int64_t at = i0 + wi + 32 * i + r;
+        if (at >= x.I) continue;
+        float* out = x.out + (x.list ? (int64_t)x.list[at] : at) * x.J;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {  // a lane holds 4 consecutive outputs
+                const int n = j0 + wj + 32 * j + 8 * t + 4 * g;
+                if (n >= x.J) continue;
+                f32x4 v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = sum[j][i][4 * t + e] + acc[j][i][4 * t + e] + (x.bias ? x.bias[n + e] : 0.0f);
+                *reinterpret_cast<f32x4*>(out + n) = v;
+            }
     }
 }
 
-__global__ void __launch_bounds__(256) f32_special_gw_kernel(const float* gy, const float* x, float* gw, int64_t M, int N,
-                                                            int K, const int* word) {
-    if (word[1] == 0) return;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < (int64_t)N * K; i += (int64_t)gridDim.x * 256) {
-        const int64_t n = i / K, k = i - n * K;
-        float s = 0.0f;
-        for (int64_t m = 0; m < M; ++m) s = fmaf(gy[m * N + n], x[m * K + k], s);
-        gw[i] = s;
-    }
+// The listed rows of y = x w^T + bias (BC) or gx = gy w, or every row where w
+// has no scale.  C: the contraction.
+template <bool BC>
+__global__ void __launch_bounds__(256, 2) f32_exact_rows_kernel(F32Exact x, int C, const F32Words* word, const float* wscale) {
+    __shared__ float lds[4 * kExHalf];
+    if (wscale[0] == 0.0f)
+        x.list = nullptr;
+    else
+        x.I = word->rows;
+    const int tj = (x.J + 127) / 128;
+    const int64_t tiles = (x.I + 127) / 128 * tj;
+    for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x)
+        f32_exact_tile<true, BC>(x, lds, t / tj * 128, (int)(t % tj) * 128, 0, C);
+}
+
+// gw (or its partial sums) where gw_exact, over the row splits of f32_gw_kernel.
+__global__ void __launch_bounds__(256, 2) f32_exact_gw_kernel(F32Exact x, int64_t M, int64_t per, const F32Words* word) {
+    __shared__ float lds[4 * kExHalf];
+    if (!gw_exact(*word)) return;
+    const int64_t c0 = (int64_t)blockIdx.y * per;
+    const int tj = (x.J + 127) / 128;
+    x.out += (int64_t)blockIdx.y * x.I * x.J;
+    f32_exact_tile<false, false>(x, lds, (int64_t)(blockIdx.x / tj) * 128, (int)(blockIdx.x % tj) * 128, c0,
+                                 c0 + per < M ? c0 + per : M);
 }
 
 // ---------------------------------------------------------------------------
@@ -622,6 +744,9 @@ F32Plan f32_plan(int64_t M, int64_t N, int64_t K) {
     at += (size_t)up(p.Mp * p.Kp * 4 + slack, 256);
     p.w_at = at;
     at += (size_t)(up(N, 256) / 32 * (p.Kp / 16) * 2048);
+    p.wf_bytes = at - p.w_at;
+    p.list_at = at;
+    at += (size_t)up(M * 4, 256);
     p.fwd_bytes = at;
     at = 256;
     p.bx_at = at;
@@ -630,8 +755,11 @@ F32Plan f32_plan(int64_t M, int64_t N, int64_t K) {
     at += (size_t)up(p.Mp * p.Np * 4 + slack, 256);
     p.bw_at = at;
     at += (size_t)(up(K, 256) / 32 * (p.Np / 16) * 2048);
+    p.bwf_bytes = at - p.bw_at;
     p.gs_at = at;
     at += (size_t)up(p.Mp * 4, 256);
+    p.blist_at = at;
+    at += (size_t)up(M * 4, 256);
     p.steps = (int)(up(M, 16) / 16);
     p.splits = f32_splits(N, K, p.steps);
     p.cs_at = at;
@@ -644,14 +772,14 @@ F32Plan f32_plan(int64_t M, int64_t N, int64_t K) {
 
 template <int MODE, bool COLS = false>
 static hipError_t split_rows(const float* x, int64_t M, int64_t Mp, int64_t K, int64_t Kp, const float* xscale,
-                             const float* gscale, int* word, char* planes, float* scale, hipStream_t s,
+                             const float* gscale, F32Words* word, int* list, char* planes, float* scale, hipStream_t s,
                              float* colsum = nullptr, float* colout = nullptr) {
     const int nc = (int)((Kp + 511) / 512);
     const int64_t rows4 = (Mp + 3) / 4, most = COLS ? kColBlocks : 2048;
     const int grid = (int)(rows4 < most ? rows4 : most);
 #define RPFQ_SPLIT(NC)                                                                                              \
     hipLaunchKernelGGL((f32_split_rows_kernel<NC, MODE, COLS>), dim3(grid), dim3(256), 0, s, x, M, Mp, (int)K,    \
-                       (int)Kp, xscale, gscale, word, planes, scale, colsum)
+                       (int)Kp, xscale, gscale, word, list, planes, scale, colsum)
     if (nc <= 1) RPFQ_SPLIT(1);
     else if (nc <= 2) RPFQ_SPLIT(2);
     else if (nc <= 4) RPFQ_SPLIT(4);
@@ -666,7 +794,7 @@ static hipError_t split_rows(const float* x, int64_t M, int64_t Mp, int64_t K, i
 
 template <int TRANS>
 static hipError_t split_w(const float* w, int64_t N, int64_t K, const float* parts, int nparts, char* wf,
-                          float* wscale, int* word, hipStream_t s) {
+                          float* wscale, F32Words* word, hipStream_t s) {
     const int64_t rows = TRANS ? K : N, con = TRANS ? N : K;
     const int rows32 = (int)(up(rows, 256) / 32), kt = (int)(up(con, 32) / 16);
     hipLaunchKernelGGL((f32_split_w_kernel<TRANS>), dim3((rows32 * kt + 3) / 4), dim3(256), 0, s, w, (int)N, (int)K,
@@ -694,6 +822,26 @@ static hipError_t f32_gemm(F32Args& a, hipStream_t s) {
     return f32_gemm_go<4>(a, s);
 }
 
+// a [M, C], out [M, J], b [J, C] (BC) or [C, J].
+template <bool BC>
+static hipError_t exact_rows(const float* a, const float* b, const float* bias, float* out, const int* list, int64_t M,
+                             int64_t J, int64_t C, const F32Words* word, const float* wscale, hipStream_t s) {
+    F32Exact x = {};
+    x.a = a;
+    x.b = b;
+    x.bias = bias;
+    x.out = out;
+    x.list = list;
+    x.lda = C;
+    x.ldb = BC ? C : J;
+    x.I = M;
+    x.J = (int)J;
+    const int64_t tiles = (M + 127) / 128 * ((J + 127) / 128), most = 2 * (int64_t)device_cus();
+    hipLaunchKernelGGL((f32_exact_rows_kernel<BC>), dim3((unsigned)(tiles < most ? tiles : most)), dim3(256), 0, s, x, (int)C,
+                       word, wscale);
+    return hipGetLastError();
+}
+
 #define RPFQ_TRY(e)                           \
     do {                                      \
         const hipError_t e_ = (e);            \
@@ -705,8 +853,10 @@ hipError_t launch_linear_f32(const float* x, const float* w, const float* bias, 
     const F32Plan p = f32_plan(M, N, K);
     char* base = reinterpret_cast<char*>(work);
     float* wscale = reinterpret_cast<float*>(base);
-    RPFQ_TRY(split_w<0>(w, N, K, parts, nparts, base + p.w_at, wscale, nullptr, s));
-    RPFQ_TRY(split_rows<0>(x, M, p.Mp, K, p.Kp, nullptr, nullptr, nullptr, base + p.x_at, xscale, s));
+    F32Words* word = reinterpret_cast<F32Words*>(base + 64);
+    int* list = reinterpret_cast<int*>(base + p.list_at);
+    RPFQ_TRY(split_w<0>(w, N, K, parts, nparts, base + p.w_at, wscale, word, s));
+    RPFQ_TRY(split_rows<0>(x, M, p.Mp, K, p.Kp, nullptr, nullptr, word, list, base + p.x_at, xscale, s));
     F32Args a = {};
     a.xp = base + p.x_at;
     a.wf = base + p.w_at;
@@ -717,11 +867,9 @@ hipError_t launch_linear_f32(const float* x, const float* w, const float* bias, 
     a.M = M;
     a.N = (int)N;
     a.KS = (int)(p.Kp / 32);
-    a.wf_bytes = (int)(p.fwd_bytes - p.w_at);
+    a.wf_bytes = (int)p.wf_bytes;
     RPFQ_TRY(f32_gemm(a, s));
-    hipLaunchKernelGGL(f32_special_rows_kernel, dim3(256), dim3(256), 0, s, x, w, bias, y, M, (int)N, (int)K, K,
-                       (int64_t)1, xscale, wscale);
-    return hipGetLastError();
+    return exact_rows<true>(x, w, bias, y, list, M, N, K, word, wscale, s);
 }
 
 hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* w, int64_t M, int64_t N, int64_t K,
@@ -730,14 +878,15 @@ hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* 
     const F32Plan p = f32_plan(M, N, K);
     char* base = reinterpret_cast<char*>(work);
     float* wscale = reinterpret_cast<float*>(base);
-    int* word = reinterpret_cast<int*>(base + 64);
+    F32Words* word = reinterpret_cast<F32Words*>(base + 64);
+    int* list = reinterpret_cast<int*>(base + p.blist_at);
     float* gscale = reinterpret_cast<float*>(base + p.gs_at);
     RPFQ_TRY(split_w<1>(w, N, K, parts, nparts, base + p.bw_at, wscale, word, s));
     if (gb)
-        RPFQ_TRY((split_rows<1, true>(gy, M, p.Mp, N, p.Np, xscale, nullptr, word, base + p.g_at, gscale, s,
+        RPFQ_TRY((split_rows<1, true>(gy, M, p.Mp, N, p.Np, xscale, nullptr, word, list, base + p.g_at, gscale, s,
                                       reinterpret_cast<float*>(base + p.cs_at), gb)));
     else
-        RPFQ_TRY(split_rows<1>(gy, M, p.Mp, N, p.Np, xscale, nullptr, word, base + p.g_at, gscale, s));
+        RPFQ_TRY(split_rows<1>(gy, M, p.Mp, N, p.Np, xscale, nullptr, word, list, base + p.g_at, gscale, s));
     if (gx) {
         F32Args a = {};
         a.xp = base + p.g_at;
@@ -748,14 +897,12 @@ hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* 
         a.M = M;
         a.N = (int)K;
         a.KS = (int)(p.Np / 32);
-        a.wf_bytes = (int)(p.gs_at - p.bw_at);
+        a.wf_bytes = (int)p.bwf_bytes;
         RPFQ_TRY(f32_gemm(a, s));
-        hipLaunchKernelGGL(f32_special_rows_kernel, dim3(256), dim3(256), 0, s, gy, w, (const float*)nullptr, gx, M,
-                           (int)K, (int)N, (int64_t)1, K, gscale, wscale);
-        RPFQ_TRY(hipGetLastError());
+        RPFQ_TRY(exact_rows<false>(gy, w, nullptr, gx, list, M, K, N, word, wscale, s));
     }
     if (gw) {
-        RPFQ_TRY(split_rows<2>(x, M, p.Mp, K, p.Kp, nullptr, gscale, word, base + p.bx_at, nullptr, s));
+        RPFQ_TRY(split_rows<2>(x, M, p.Mp, K, p.Kp, nullptr, gscale, word, nullptr, base + p.bx_at, nullptr, s));
         static std::atomic<uint64_t> attr_done{0};
         RPFQ_TRY(set_lds_attr_once(reinterpret_cast<const void*>(&f32_gw_kernel), kGwLds, attr_done));
         F32GwArgs g = {};
@@ -774,16 +921,24 @@ hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* 
         g.splits = p.splits;
         hipLaunchKernelGGL(f32_gw_kernel, dim3(g.tiles_n * g.tiles_k * g.splits), dim3(256), kGwLds, s, g);
         RPFQ_TRY(hipGetLastError());
+        F32Exact x2 = {};
+        x2.a = gy;
+        x2.b = x;
+        x2.out = g.part;
+        x2.lda = N;
+        x2.ldb = K;
+        x2.I = N;
+        x2.J = (int)K;
+        hipLaunchKernelGGL(f32_exact_gw_kernel, dim3((unsigned)(((N + 127) / 128) * ((K + 127) / 128)), p.splits), dim3(256), 0,
+                           s, x2, M, (int64_t)g.per * 16, (const F32Words*)word);
+        RPFQ_TRY(hipGetLastError());
         if (p.splits > 1) {
             const int64_t n4 = N * K / 4;
             const int grid = (int)((n4 + 255) / 256 < 2048 ? (n4 + 255) / 256 : 2048);
             hipLaunchKernelGGL(f32_gw_reduce_kernel, dim3(grid), dim3(256), 0, s, (const float*)g.part, n4, p.splits,
-                               (const int*)word, gw);
+                               (const F32Words*)word, gw);
             RPFQ_TRY(hipGetLastError());
         }
-        hipLaunchKernelGGL(f32_special_gw_kernel, dim3(1024), dim3(256), 0, s, gy, x, gw, M, (int)N, (int)K,
-                           (const int*)word);
-        RPFQ_TRY(hipGetLastError());
     }
     return hipSuccess;
 }

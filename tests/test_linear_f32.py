@@ -93,6 +93,59 @@ def test_linear_f32_special_values(where, value):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(1, 8, 8), (127, 120, 24), (129, 136, 40), (700, 264, 776), (1300, 1000, 128),
+                                   (3000, 16, 4096)])
+def test_exact_rows_match_float64(m, n, k):
+    """The plain float32 products, at the edges of their 128 x 128 tiles: every
+    row where w has no finite bound, single rows with an inf, and all of gw
+    beside one.  Each of the con additions of an output rounds once."""
+    from quant_models import ops
+
+    x, w, b, gy = _inputs(m, n, k)
+    xd, wd, gd = x.double(), w.double(), gy.double()
+    none = torch.full((1,), float("inf"), device=DEV)
+    y, scale = ops.linear_f32(x, w, b, none)
+    gx, _ = ops.linear_f32_grad(gy, x, w, none, scale)
+    for got, ref, con, mag in ((y, xd @ wd.t() + b.double(), k, xd.abs() @ wd.abs().t() + b.abs()),
+                               (gx, gd @ wd, n, gd.abs() @ wd.abs())):
+        assert bool(((got.double() - ref).abs() <= (con + 2) * 2.0 ** -24 * mag).all())
+    some = torch.unique(torch.linspace(0, m - 1, 5).long())
+    x[some, 3] = float("inf")
+    y, scale = ops.linear_f32(x, w, b, w.abs().max().reshape(1))
+    _, gw = ops.linear_f32_grad(gy, x, w, w.abs().max().reshape(1), scale)
+    assert torch.equal(y[some.cuda()].isinf(), (x[some] @ w.t()).isinf()) and bool(y[some.cuda()].isinf().any())
+    keep = [i for i in range(k) if i != 3]
+    assert not gw[:, 3].isfinite().any()
+    ref = gd.t() @ xd
+    assert bool(((gw.double() - ref).abs() <= (m + 2) * 2.0 ** -24 * (gd.abs().t() @ xd.abs()))[:, keep].all())
+
+
+@pytest.mark.gpu
+def test_a_step_of_nan_costs_a_few_ordinary_steps():
+    """NaN in every row: all three products in plain float32, 16 times the
+    matrix work, which must not become a serial sum per output."""
+    from quant_models import ops
+
+    x, w, b, gy = _inputs(12608, 3072, 768)
+    parts = w.abs().max().reshape(1)
+
+    def step():
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        y, scale = ops.linear_f32(x, w, b, parts)
+        grads = ops.linear_f32_grad(gy, x, w, parts, scale)
+        end.record()
+        torch.cuda.synchronize()
+        return start.elapsed_time(end), (y, *grads)
+
+    usual = min(step()[0] for _ in range(5))
+    x[:, 0] = gy[:, 0] = float("nan")
+    times, outs = zip(*(step() for _ in range(2)))
+    assert all(bool(t.isnan().any()) for t in outs[0])
+    assert min(times) <= 16 * usual
+
+
+@pytest.mark.gpu
 def test_linear_f32_empty_gradient():
     from quant_models import ops
 
