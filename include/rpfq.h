@@ -619,8 +619,8 @@ int rpfq_linear_f32(const float* x, const float* w, const float* bias, int64_t M
  * grad_w = grad_y^T x (NULL: not wanted), in the same arithmetic; x_scale as
  * the forward wrote it.  grad_w takes row m of x times the scale of grad_y's
  * row, so a row whose gradients lie below 2^-17 of the largest row's loses
- * bits of its (equally smaller) share.  With inf or NaN in a row of x or
- * grad_y all of grad_w is summed in plain float32.  grad_b [N] (NULL: not wanted): the
+ * bits of its (equally smaller) share.  A row with inf or NaN in x or
+ * grad_y takes part in grad_w in plain float32.  grad_b [N] (NULL: not wanted): the
  * column sums of grad_y, float32 in a fixed order, at least one of the other
  * two wanted with it.
  * Replaces the backward of that F.linear (grad_x = grad_output @ weight,

@@ -27,7 +27,7 @@ constexpr int kF32NoRow = -100000;
 // What the passes of a call leave for the ones behind them, in its workspace.
 struct F32Words {
     int emax;   // gw: largest exponent of a row's product of maxima, or kF32NoRow
-    int bad;    // gw: a row of x or gy has inf or NaN
+    int gw;     // gw has rows that f32_exact_gw_kernel adds
     int rows;   // rows of y / gx that f32_exact_rows_kernel writes
 };
 // Most blocks of the gy pass where it also sums columns: 4 a CU.
@@ -37,13 +37,18 @@ __device__ __forceinline__ int f32_scale_exp(float s) {  // s = 2^e
     return (int)((__float_as_uint(s) >> 23) & 0xffu) - 127;
 }
 
+// Rows of gw that f32_exact_gw_kernel sums: inf or NaN in x or gy (scale 0).
+__device__ __forceinline__ bool gw_listed(float r, float sx, int emax) {
+    return r == 0.0f || sx == 0.0f;
+}
+
 // One wave per row, the row in registers (K <= 4096).  MODE 0: the row's own
 // scale 2^e (largest magnitude in [2^14, 2^15)), written to scale[m]; +inf
 // for a zero row, 0 for one with inf or NaN (its planes are zeroed, and it goes
 // to the list of exact rows).
-// MODE 1 (gy): also collects over the rows the largest exponent of x's rows
-// over r (emax) and whether any row of x or gy is non-finite (bad).
-// MODE 2 (x of gw): times 1 / r[m], r = gscale, and 2^-emax.
+// MODE 1 (gy): also collects the largest exponent of x's rows over r (emax).
+// MODE 2 (x of gw): times 1 / r[m], r = gscale, and 2^-emax; rows that are not
+// part of the split sum (gw_listed) are zero.
 // COLS (gy): also the column sums of the block's rows, colsum[block][K], for
 // the bias gradient: each lane adds the values it holds anyway (a separate
 // reduction over 12,608 x 3,072 reads 155 MB again, 40.6 us; here 7.5 us and
@@ -54,7 +59,7 @@ __global__ void __launch_bounds__(256) f32_split_rows_kernel(const float* x, int
                                                             const float* xscale, const float* gscale, F32Words* word,
                                                             int* list, char* planes, float* scale, float* colsum) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int emax = kF32NoRow, bad = 0;
+    int emax = kF32NoRow, listed = 0;
     const int e2 = MODE == 2 ? word->emax : 0;
     f32x4 cs[NC][2];
     if (COLS) {
@@ -99,12 +104,13 @@ __global__ void __launch_bounds__(256) f32_split_rows_kernel(const float* x, int
             }
             if (MODE == 1 && in) {
                 const float sx = xscale[m];
-                if (!fin || sx == 0.0f) bad = 1;
-                if (!zero && sx != 0.0f && sx < __builtin_inff()) emax = max(emax, -k - f32_scale_exp(sx));
+                if (!zero && sx > 0.0f && sx < __builtin_inff()) emax = max(emax, -k - f32_scale_exp(sx));
             }
         } else if (in) {
-            const float r = gscale[m];
-            zero = r == 0.0f || r == __builtin_inff() || e2 == kF32NoRow;
+            const float r = gscale[m], sx = xscale[m];
+            const bool apart = gw_listed(r, sx, e2);
+            if (apart) listed = 1;
+            zero = apart || r == __builtin_inff() || sx == __builtin_inff();
             k = zero ? 0 : -f32_scale_exp(r) - e2;
         }
         char* dst = planes + m * (int64_t)Kp * 4;
@@ -129,17 +135,12 @@ __global__ void __launch_bounds__(256) f32_split_rows_kernel(const float* x, int
         }
     }
     if (MODE == 1) {
-        __shared__ int sm[8];
-        if (lane == 0) {
-            sm[wave] = emax;
-            sm[4 + wave] = bad;
-        }
+        __shared__ int sm[4];
+        if (lane == 0) sm[wave] = emax;
         __syncthreads();
-        if (threadIdx.x == 0) {
-            atomicMax(&word->emax, max(max(sm[0], sm[1]), max(sm[2], sm[3])));
-            if (sm[4] | sm[5] | sm[6] | sm[7]) atomicOr(&word->bad, 1);
-        }
+        if (threadIdx.x == 0) atomicMax(&word->emax, max(max(sm[0], sm[1]), max(sm[2], sm[3])));
     }
+    if (MODE == 2 && listed && lane == 0) atomicOr(&word->gw, 1);
     if (COLS) {  // the four waves one after another, then one coalesced row
         __shared__ __align__(16) float sum[NC * 512];
         for (int w = 0; w < 4; ++w) {
@@ -441,14 +442,12 @@ struct F32GwArgs {
     int steps, per;    // 16-row steps in all, and per split
     int tiles_n, tiles_k, splits;
 };
-__device__ __forceinline__ bool gw_exact(const F32Words& w) { return w.bad != 0; }
 constexpr int kGwG = 16 * 512, kGwStage = kGwG + 16 * 1024;
 constexpr int kGwLds = 3 * kGwStage + 256;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* lds_s4_t;
 
 __global__ void __launch_bounds__(256, 2) f32_gw_kernel(F32GwArgs a) {
-    if (gw_exact(*a.word)) return;  // f32_exact_gw_kernel writes the partial sums
     extern __shared__ __align__(16) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -551,10 +550,11 @@ __global__ void __launch_bounds__(256, 2) f32_gw_kernel(F32GwArgs a) {
     }
 }
 
-// gw = 2^emax times the sum of the splits' partials, in their order.
+// gw = 2^emax (1 after f32_exact_gw_kernel) times the sum of the splits'
+// partials, in their order.
 __global__ void __launch_bounds__(256) f32_gw_reduce_kernel(const float* part, int64_t n4, int splits, const F32Words* word,
                                                            float* gw) {
-    const int e = word->emax == kF32NoRow || gw_exact(*word) ? 0 : word->emax;
+    const int e = word->emax == kF32NoRow || word->gw ? 0 : word->emax;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)gridDim.x * 256) {
         f32x4 v = reinterpret_cast<const f32x4*>(part)[i];
         for (int s = 1; s < splits; ++s) v += reinterpret_cast<const f32x4*>(part)[i + s * n4];
@@ -570,9 +570,9 @@ __global__ void __launch_bounds__(256) f32_gw_reduce_kernel(const float* part, i
 // ---------------------------------------------------------------------------
 // Where split operands do not stand for their values (inf, NaN) the products
 // run on v_mfma_f32_32x32x2_f32, so that special values come out as a float32
-// GEMM's: the listed rows of y and gx, and all of gw.  1/16 of the fp16 rate;
-// with every row listed 12,608 x 3,072 x 768 takes 640 us a product (the
-// float32 library GEMM: 541), and an empty list one short launch.
+// GEMM's: the listed rows of y and gx, and the listed rows' share of gw.  1/16
+// of the fp16 rate; with every row listed 12,608 x 3,072 x 768 takes 640 us a
+// product (the float32 library GEMM: 541), and an empty list one short launch.
 //
 // Tile: 128 rows i x 128 outputs j, 4 waves of 64 x 64, 16 of the contraction
 // c a step through two LDS buffers of odd row stride (17 floats: 32 rows of a
@@ -590,9 +590,23 @@ struct F32Exact {
     int J;
 };
 constexpr int kExLd = 17, kExHalf = 128 * kExLd;
+struct F32ExactSum {
+    floatx16 acc[2][2], sum[2][2];  // [j block][i block]
+    int steps;
+    __device__ __forceinline__ void zero() {
+        steps = 0;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) acc[j][i] = sum[j][i] = floatx16{0};
+    }
+};
 
+// Adds c0 .. c1 - 1 of the contraction to the tile at (i0, j0); rows: where c
+// is a row number of a and b, these (in LDS) instead of c itself.
 template <bool AC, bool BC>
-__device__ __forceinline__ void f32_exact_tile(const F32Exact& x, float* lds, int64_t i0, int j0, int64_t c0, int64_t c1) {
+__device__ __forceinline__ void f32_exact_add(const F32Exact& x, float* lds, int64_t i0, int j0, int64_t c0, int64_t c1,
+                                              const int* rows, F32ExactSum& s) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 31, g = lane >> 5, wi = (wave & 1) * 64, wj = (wave >> 1) * 64;
     // two 4-float loads of each operand: (row q4, columns 4 qc ..) of the tile,
@@ -617,8 +631,9 @@ __device__ __forceinline__ void f32_exact_tile(const F32Exact& x, float* lds, in
         for (int p = 0; p < 2; ++p) {
             ra[p] = rb[p] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
             const int64_t ca = AC ? c + qc : c + q + 8 * p, cb = BC ? c + qc : c + q + 8 * p;
-            if (aok[p] && ca < c1) ra[p] = *reinterpret_cast<const f32x4*>(AC ? ap[p] + c : ap[p] + ca * x.lda);
-            if (bok[p] && cb < c1) rb[p] = *reinterpret_cast<const f32x4*>(BC ? bp[p] + c : bp[p] + cb * x.ldb);
+            const int64_t at = !AC && rows && ca < c1 ? rows[ca] : ca, bt = !BC && rows && cb < c1 ? rows[cb] : cb;
+            if (aok[p] && ca < c1) ra[p] = *reinterpret_cast<const f32x4*>(AC ? ap[p] + c : ap[p] + at * x.lda);
+            if (bok[p] && cb < c1) rb[p] = *reinterpret_cast<const f32x4*>(BC ? bp[p] + c : bp[p] + bt * x.ldb);
         }
     };
     auto store = [&](float* d) {
@@ -630,16 +645,11 @@ __device__ __forceinline__ void f32_exact_tile(const F32Exact& x, float* lds, in
                 d[kExHalf + (BC ? (q4 + 64 * p) * kExLd + qc + e : (qr + e) * kExLd + q + 8 * p)] = rb[p][e];
             }
     };
-    floatx16 acc[2][2], sum[2][2];  // [j block][i block]
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) acc[j][i] = sum[j][i] = floatx16{0};
-    __syncthreads();  // the tile before this one is read
+    __syncthreads();  // rows is written, the step before this one is read
     load(c0);
     store(lds);
     __syncthreads();
-    int buf = 0, steps = 0;
+    int buf = 0;
     for (int64_t c = c0; c < c1; c += 16) {
         const bool more = c + 16 < c1;
         if (more) load(c + 16);
@@ -648,24 +658,31 @@ __device__ __forceinline__ void f32_exact_tile(const F32Exact& x, float* lds, in
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const float a0 = la[2 * k], a1 = la[32 * kExLd + 2 * k], b0 = lb[2 * k], b1 = lb[32 * kExLd + 2 * k];
-            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(b0, a0, acc[0][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(b0, a1, acc[0][1], 0, 0, 0);
-            acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(b1, a0, acc[1][0], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(b1, a1, acc[1][1], 0, 0, 0);
+            s.acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(b0, a0, s.acc[0][0], 0, 0, 0);
+            s.acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(b0, a1, s.acc[0][1], 0, 0, 0);
+            s.acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(b1, a0, s.acc[1][0], 0, 0, 0);
+            s.acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(b1, a1, s.acc[1][1], 0, 0, 0);
         }
-        if (++steps % 32 == 0) {
+        if (++s.steps % 32 == 0) {
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    sum[j][i] += acc[j][i];
-                    acc[j][i] = floatx16{0};
+                    s.sum[j][i] += s.acc[j][i];
+                    s.acc[j][i] = floatx16{0};
                 }
         }
         if (more) store(lds + (buf ^ 1) * 2 * kExHalf);
         __syncthreads();
         buf ^= 1;
     }
+}
+
+// out = the tile plus bias, or (ADD) out times 2^e plus the tile.
+template <bool ADD>
+__device__ __forceinline__ void f32_exact_store(const F32Exact& x, int64_t i0, int j0, const F32ExactSum& s, int e) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane & 31, g = lane >> 5, wi = (wave & 1) * 64, wj = (wave >> 1) * 64;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int64_t at = i0 + wi + 32 * i + r;
@@ -677,10 +694,16 @@ __device__ __forceinline__ void f32_exact_tile(const F32Exact& x, float* lds, in
             for (int t = 0; t < 4; ++t) {  // a lane holds 4 consecutive outputs
                 const int n = j0 + wj + 32 * j + 8 * t + 4 * g;
                 if (n >= x.J) continue;
-                f32x4 v;
+                f32x4* o = reinterpret_cast<f32x4*>(out + n);
+                f32x4 v, b = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+                if (ADD) v = *o;
+                else if (x.bias) b = (f32x4){x.bias[n], x.bias[n + 1], x.bias[n + 2], x.bias[n + 3]};
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = sum[j][i][4 * t + e] + acc[j][i][4 * t + e] + (x.bias ? x.bias[n + e] : 0.0f);
-                *reinterpret_cast<f32x4*>(out + n) = v;
+                for (int k = 0; k < 4; ++k) {
+                    const float w = s.sum[j][i][4 * t + k] + s.acc[j][i][4 * t + k];
+                    v[k] = ADD ? __builtin_amdgcn_ldexpf(v[k], e) + w : w + b[k];
+                }
+                *o = v;
             }
     }
 }
@@ -696,19 +719,59 @@ __global__ void __launch_bounds__(256, 2) f32_exact_rows_kernel(F32Exact x, int 
         x.I = word->rows;
     const int tj = (x.J + 127) / 128;
     const int64_t tiles = (x.I + 127) / 128 * tj;
-    for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x)
-        f32_exact_tile<true, BC>(x, lds, t / tj * 128, (int)(t % tj) * 128, 0, C);
+    for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+        F32ExactSum s;
+        s.zero();
+        f32_exact_add<true, BC>(x, lds, t / tj * 128, (int)(t % tj) * 128, 0, C, nullptr, s);
+        f32_exact_store<false>(x, t / tj * 128, (int)(t % tj) * 128, s, 0);
+    }
 }
 
-// gw (or its partial sums) where gw_exact, over the row splits of f32_gw_kernel.
-__global__ void __launch_bounds__(256, 2) f32_exact_gw_kernel(F32Exact x, int64_t M, int64_t per, const F32Words* word) {
+// Adds the listed rows' share to gw (splits = 1) or to the partial sums, which
+// leave their unit 2^emax with it (the listed rows may lie far above).  Split sp takes the listed ones of the rows of split sp of
+// f32_gw_kernel, in their order, 1,024 rows at a time through LDS.
+__global__ void __launch_bounds__(256, 2) f32_exact_gw_kernel(F32Exact x, int64_t M, int64_t per, int splits,
+                                                             const float* gscale, const float* xscale, const F32Words* word) {
     __shared__ float lds[4 * kExHalf];
-    if (!gw_exact(*word)) return;
-    const int64_t c0 = (int64_t)blockIdx.y * per;
-    const int tj = (x.J + 127) / 128;
+    __shared__ int rows[1024], total[4];
+    if (word->gw == 0) return;
+    const int emax = word->emax, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int tj = (x.J + 127) / 128, j0 = (int)(blockIdx.x % tj) * 128;
+    const int64_t i0 = (int64_t)(blockIdx.x / tj) * 128;
+    const int64_t m1 = min(M, ((int64_t)blockIdx.y + 1) * per);
     x.out += (int64_t)blockIdx.y * x.I * x.J;
-    f32_exact_tile<false, false>(x, lds, (int64_t)(blockIdx.x / tj) * 128, (int)(blockIdx.x % tj) * 128, c0,
-                                 c0 + per < M ? c0 + per : M);
+    F32ExactSum s;
+    s.zero();
+    for (int64_t m0 = (int64_t)blockIdx.y * per; m0 < m1; m0 += 1024) {
+        bool on[4];
+        int n = 0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int64_t m = m0 + 4 * threadIdx.x + t;
+            on[t] = m < m1 && gw_listed(gscale[m], xscale[m], emax);
+            n += on[t];
+        }
+        int before = n;  // of the lanes up to this one
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(before, o, 64);
+            if (lane >= o) before += v;
+        }
+        if (lane == 63) total[wave] = before;
+        __syncthreads();
+        int at = before - n, count = 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            if (w < wave) at += total[w];
+            count += total[w];
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            if (on[t]) rows[at++] = (int)(m0 + 4 * threadIdx.x + t);
+        if (count) f32_exact_add<false, false>(x, lds, i0, j0, 0, count, rows, s);
+        __syncthreads();  // total and rows are read
+    }
+    f32_exact_store<true>(x, i0, j0, s, splits > 1 && emax != kF32NoRow ? emax : 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -902,7 +965,7 @@ hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* 
         RPFQ_TRY(exact_rows<false>(gy, w, nullptr, gx, list, M, K, N, word, wscale, s));
     }
     if (gw) {
-        RPFQ_TRY(split_rows<2>(x, M, p.Mp, K, p.Kp, nullptr, gscale, word, nullptr, base + p.bx_at, nullptr, s));
+        RPFQ_TRY(split_rows<2>(x, M, p.Mp, K, p.Kp, xscale, gscale, word, nullptr, base + p.bx_at, nullptr, s));
         static std::atomic<uint64_t> attr_done{0};
         RPFQ_TRY(set_lds_attr_once(reinterpret_cast<const void*>(&f32_gw_kernel), kGwLds, attr_done));
         F32GwArgs g = {};
@@ -930,7 +993,7 @@ hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* 
         x2.I = N;
         x2.J = (int)K;
         hipLaunchKernelGGL(f32_exact_gw_kernel, dim3((unsigned)(((N + 127) / 128) * ((K + 127) / 128)), p.splits), dim3(256), 0,
-                           s, x2, M, (int64_t)g.per * 16, (const F32Words*)word);
+                           s, x2, M, (int64_t)g.per * 16, p.splits, (const float*)gscale, xscale, (const F32Words*)word);
         RPFQ_TRY(hipGetLastError());
         if (p.splits > 1) {
             const int64_t n4 = N * K / 4;
