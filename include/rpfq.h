@@ -601,8 +601,12 @@ size_t rpfq_linear_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int back
  * Runs on the fp16 matrix cores with every operand split into two fp16
  * terms (22 bits) under power-of-two scales, three products per pair summed
  * in float32: its distance to the exact sum is no larger than a float32
- * GEMM's.  Rows with inf or NaN (every row, where w_parts has one) are summed
- * in plain float32 on the matrix cores, at a float32 GEMM's speed.
+ * GEMM's.  An element keeps 2^-39 of its row's largest magnitude (w: of the
+ * bound).  Summed in plain float32 on the matrix cores instead, at a float32
+ * GEMM's speed: rows with inf or NaN; rows of which one half of the columns
+ * has fewer than 32 elements within 2^-4 of the largest and its others average
+ * below 2^-15 of it; every row where a nonzero part is below 2^-15 of the sum,
+ * or the sum is not finite.
  * w_parts[n_parts] (device): values whose absolute sum bounds every |w|
  * (the scales rpfq_quantize_wide wrote for w; 0 only if w is all 0).
  * x_scale [M] (out): the power-of-two scale of each row of x, read by
@@ -617,10 +621,10 @@ int rpfq_linear_f32(const float* x, const float* w, const float* bias, int64_t M
 /*
  * Gradients of rpfq_linear_f32: grad_x = grad_y w (NULL: not wanted) and
  * grad_w = grad_y^T x (NULL: not wanted), in the same arithmetic; x_scale as
- * the forward wrote it.  grad_w takes row m of x times the scale of grad_y's
- * row, so a row whose gradients lie below 2^-17 of the largest row's loses
- * bits of its (equally smaller) share.  A row with inf or NaN in x or
- * grad_y takes part in grad_w in plain float32.  grad_b [N] (NULL: not wanted): the
+ * the forward wrote it.  grad_w: a row takes part in split operands under the
+ * product of its two scales, in plain float32 where x's or grad_y's row is one
+ * that y or grad_x sums so, or where the product of the two rows' largest
+ * magnitudes is below 2^-14 of the largest such product.  grad_b [N] (NULL: not wanted): the
  * column sums of grad_y, float32 in a fixed order, at least one of the other
  * two wanted with it.
  * Replaces the backward of that F.linear (grad_x = grad_output @ weight,

@@ -11,6 +11,12 @@
 // once l is subnormal), and the dropped l l' is below 2^-22 of h h'; the
 // accumulator takes 3 K / 16 roundings where a float32 GEMM takes K.
 //
+// A value more than 2^15 below the largest of its scale keeps fewer bits than
+// a float32's.  Next to sums that hold the largest values that is lost in
+// their rounding; it shows where a weight, or another row, takes those out.
+// Such rows are summed in plain float32 instead: f32_wide_row (y, gx),
+// gw_listed (gw), and all rows of a w whose parts differ that much.
+//
 // Scales: y and gx scale each row of x / gy by its own largest magnitude and
 // w by one bound (the sum of its quantizer's scales), undone exactly on the
 // output.  gw contracts over the rows, so a row's scale cannot be undone
@@ -37,15 +43,62 @@ __device__ __forceinline__ int f32_scale_exp(float s) {  // s = 2^e
     return (int)((__float_as_uint(s) >> 23) & 0xffu) - 127;
 }
 
-// Rows of gw that f32_exact_gw_kernel sums: inf or NaN in x or gy (scale 0).
+// Rows of gw that f32_exact_gw_kernel sums, by the scales of gy's and x's row:
+// inf or NaN (0), a wide row (negative), or a product of maxima more than 2^14
+// below the largest such product.
 __device__ __forceinline__ bool gw_listed(float r, float sx, int emax) {
-    return r == 0.0f || sx == 0.0f;
+    if (r <= 0.0f || sx <= 0.0f) return true;
+    return r < __builtin_inff() && sx < __builtin_inff() && emax + f32_scale_exp(r) + f32_scale_exp(sx) > 14;
+}
+
+// Whether a row (mx: its largest magnitude, finite and not 0) holds values
+// that the split loses beside the others and a sum may still depend on: in one
+// half of its columns (a complex layer's weight can be 0 on one) fewer than 32
+// values reach mx / 16, and the rest average below 2^-15 mx -- split operands
+// keep 2^-39 mx, float32 2^-24 of the rest.  Also rows that row_prescale cannot
+// lift to the top of fp16's range.  Ordinary rows are told by the count alone.
+template <int NC>
+__device__ __forceinline__ bool f32_wide_row(const f32x4 (&v)[NC][2], float mx, int K, int lane) {
+    if (mx < 0x1p-112f) return true;
+    const float thr = mx * 0.0625f;
+    const int cut = (K / 2 + 7) / 8;  // of the 8-column pieces, those of the first half
+    uint32_t count = 0;               // first half, second half << 16
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        uint32_t c = 0;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) c += fabsf(v[i][t >> 2][t & 3]) >= thr;
+        count += lane + 64 * i < cut ? c : c << 16;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) count += __shfl_xor((int)count, o, 64);
+    const uint32_t big[2] = {count & 0xffffu, count >> 16};
+    if (big[0] >= 32 && big[1] >= 32) return false;
+    bool wide = false;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        float sum = 0.0f, n = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            if ((lane + 64 * i < cut) != (h == 0)) continue;
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const float a = fabsf(v[i][t >> 2][t & 3]);
+                sum += a < thr ? a : 0.0f;
+                n += a < thr && a > 0.0f ? 1.0f : 0.0f;
+            }
+        }
+        sum = group_sum<64>(sum);
+        n = group_sum<64>(n);
+        wide |= big[h] < 32 && sum < 0x1p-15f * mx * n;
+    }
+    return wide;
 }
 
 // One wave per row, the row in registers (K <= 4096).  MODE 0: the row's own
 // scale 2^e (largest magnitude in [2^14, 2^15)), written to scale[m]; +inf
-// for a zero row, 0 for one with inf or NaN (its planes are zeroed, and it goes
-// to the list of exact rows).
+// for a zero row, 0 for one with inf or NaN (its planes are zeroed), negative
+// for a wide one; these two go to the list of exact rows.
 // MODE 1 (gy): also collects the largest exponent of x's rows over r (emax).
 // MODE 2 (x of gw): times 1 / r[m], r = gscale, and 2^-emax; rows that are not
 // part of the split sum (gw_listed) are zero.
@@ -98,13 +151,14 @@ __global__ void __launch_bounds__(256) f32_split_rows_kernel(const float* x, int
             zero = !in || mx == 0 || !fin;
             const float s = !fin ? 0.0f : mx == 0 ? __builtin_inff() : row_prescale(__uint_as_float(mx));
             k = zero ? 0 : f32_scale_exp(s);
+            const bool wide = !zero && f32_wide_row<NC>(v, __uint_as_float(mx), K, lane);
             if (in && lane == 0) {
-                scale[m] = s;
-                if (!fin) list[atomicAdd(&word->rows, 1)] = (int)m;
+                scale[m] = wide ? -s : s;
+                if (!fin || wide) list[atomicAdd(&word->rows, 1)] = (int)m;
             }
             if (MODE == 1 && in) {
                 const float sx = xscale[m];
-                if (!zero && sx > 0.0f && sx < __builtin_inff()) emax = max(emax, -k - f32_scale_exp(sx));
+                if (!zero && !wide && sx > 0.0f && sx < __builtin_inff()) emax = max(emax, -k - f32_scale_exp(sx));
             }
         } else if (in) {
             const float r = gscale[m], sx = xscale[m];
@@ -180,15 +234,19 @@ __global__ void __launch_bounds__(1024) f32_colsum_kernel(const float* parts, in
 // row r, contraction 8 g .. 8 g + 7.  TRANS = 0: rows = N, contraction = K;
 // 1: rows = K, contraction = N.  One thread per 16 bytes of h and l; zero
 // past the matrix.  The scale 2^e of w from the bound sum |parts| >= |w|
-// goes to wscale[0] (0 if that is not finite: every row is then an exact one);
+// goes to wscale[0] (0 if that is not finite, below 2^-112 or 2^15 times the
+// smallest part: every row is then an exact one);
 // block 0 also initialises the words.
 template <int TRANS>
 __global__ void __launch_bounds__(256) f32_split_w_kernel(const float* w, int N, int K, int rows32, int kt,
                                                          const float* parts, int nparts, char* wf, float* wscale,
                                                          F32Words* word) {
-    float bound = 0.0f;
-    for (int i = 0; i < nparts; ++i) bound += fabsf(parts[i]);
-    const bool fin = bound <= 3.40282347e38f;
+    float bound = 0.0f, least = __builtin_inff();
+    for (int i = 0; i < nparts; ++i) {
+        bound += fabsf(parts[i]);
+        if (parts[i] != 0.0f) least = fminf(least, fabsf(parts[i]));
+    }
+    const bool fin = bound <= 3.40282347e38f && !(least < 0x1p-15f * bound) && !(bound > 0.0f && bound < 0x1p-112f);
     const float s = bound > 0.0f ? row_prescale(bound) : 1.0f;
     const int k = f32_scale_exp(s);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -568,7 +626,7 @@ __global__ void __launch_bounds__(256) f32_gw_reduce_kernel(const float* part, i
 // ---------------------------------------------------------------------------
 // exact rows: plain float32 sums
 // ---------------------------------------------------------------------------
-// Where split operands do not stand for their values (inf, NaN) the products
+// Where split operands do not stand for their values the products
 // run on v_mfma_f32_32x32x2_f32, so that special values come out as a float32
 // GEMM's: the listed rows of y and gx, and the listed rows' share of gw.  1/16
 // of the fp16 rate; with every row listed 12,608 x 3,072 x 768 takes 640 us a

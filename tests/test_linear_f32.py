@@ -72,6 +72,83 @@ def test_linear_f32_rows_of_any_magnitude():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("what", ["feature", "half", "weight"])
+def test_linear_f32_values_far_below_a_scale(what):
+    """Values 2^0 .. 2^70 below the largest of their scale, in outputs whose
+    weights take the largest out: the bar of a float32 product, without a
+    floor.  feature: one column of x and gy; half: the first half of their
+    columns; weight: columns of w below another part."""
+    from quant_models import ops
+
+    m, n, k = 213, 264, 520
+    x, w, b, gy = _inputs(m, n, k)
+    e = torch.exp2((torch.arange(m, device=DEV) % 71).float()).reshape(-1, 1)
+    parts = w.abs().max().reshape(1)
+    if what == "feature":
+        x[:, 7:8] *= e
+        gy[:, 5:6] *= e
+        w[:, 7] = w[5] = 0
+    elif what == "half":
+        x[:, : k // 2] *= e
+        gy[:, : n // 2] *= e
+        w[: n // 2, : k // 2] = w[: n // 2, k // 4 :] = 0
+        w[n // 2 :, : k // 2] = 0
+    else:
+        x[:, ::2], gy[:, ::2] = 0, 0
+        w[:, 1::2] *= 2.0 ** -33
+        w[1::2] *= 2.0 ** -33
+        parts = torch.stack((w.abs().max(), w[1::2, 1::2].abs().max()))
+    y, scale = ops.linear_f32(x, w, None, parts)
+    gx, _ = ops.linear_f32_grad(gy, x, w, parts, scale)
+    xd, wd, gd = x.double(), w.double(), gy.double()
+    assert bool(((y.double() - xd @ wd.t()).abs() <= _bound(xd, wd.t(), k, 0)).all())
+    assert bool(((gx.double() - gd @ wd).abs() <= _bound(gd, wd, n, 0)).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(40, 8, 16), (1037, 136, 264), (9000, 72, 104)])
+def test_weight_gradient_of_rows_of_any_magnitude(m, n, k):
+    """x and grad_y rows of independent magnitudes, products of maxima over
+    2^0 .. 2^-80, and columns of x that only the lesser half of the rows have:
+    the bar of a float32 product in every column, the same bits each time."""
+    from quant_models import ops
+
+    x, w, _, gy = _inputs(m, n, k)
+    g = torch.Generator(device=DEV).manual_seed(m)
+    ex, eg = (torch.randint(-40, 1, (m, 1), device=DEV, generator=g).float() for _ in range(2))
+    x, gy = x * torch.exp2(ex), gy * torch.exp2(eg)
+    x[(ex + eg > -40).reshape(-1), : k // 4] = 0
+    parts = w.abs().max().reshape(1)
+    _, scale = ops.linear_f32(x, w, None, parts)
+    _, gw = ops.linear_f32_grad(gy, x, w, parts, scale, want_x=False)
+    xd, gd = x.double(), gy.double()
+    assert bool(((gw.double() - gd.t() @ xd).abs() <= _bound(gd.t(), xd, m, 0)).all())
+    for _ in range(3):
+        assert torch.equal(gw, ops.linear_f32_grad(gy, x, w, parts, scale, want_x=False)[1])
+
+
+@pytest.mark.gpu
+def test_ordinary_rows_take_the_split_product():
+    """Activations, GELU outputs, quantized rows with few levels left, softmax
+    gradients and rows with some outliers are not summed apart: the scales of
+    such rows stay positive."""
+    from quant_models import ops
+
+    g = torch.Generator(device=DEV).manual_seed(0)
+    k = 768
+    z = torch.randn(2000, k, device=DEV, generator=g)
+    outlier = z.clone()
+    outlier[:, 11] *= 1000
+    quantized = torch.round(z / z.abs().amax(1, keepdim=True) * 7) * (z.abs().amax(1, keepdim=True) / 7)
+    quantized[:, ::2] *= z[:, ::2].abs() > 2.5
+    p = torch.softmax(2 * z, 1)
+    p[:, 5] -= 1
+    for x in (z, torch.nn.functional.gelu(2 * z - 2), outlier, quantized, p, z * (z > 1), z[:, :1].expand(-1, k).contiguous()):
+        _, scale = ops.linear_f32(x, z[:8].contiguous(), None, z[:8].abs().max().reshape(1))
+        assert bool((scale > 0).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("where", ["x", "gy", "w"])
 @pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.0e38])
 def test_linear_f32_special_values(where, value):
