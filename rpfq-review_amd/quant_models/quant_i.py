@@ -326,8 +326,8 @@ PRESCALED_LN = os.environ.get("RPFQ_PRESCALED_LN", "1") != "0"
 # which is slower than the library's fp16 GEMM on the decoded weight).
 QAT_PACKED_GRAD = os.environ.get("RPFQ_QAT_PACKED_GRAD", "0")
 # float32 training products of at least this many operations (2 M N K) run on
-# split fp16 operands (_split_linear_pays)
-SPLIT_LINEAR_MIN = 4.5e9
+# split fp16 operands (_split_linear_pays); RPFQ_SPLIT_LINEAR=0 keeps F.linear
+SPLIT_LINEAR_MIN = 4.5e9 if os.environ.get("RPFQ_SPLIT_LINEAR", "1") != "0" else float("inf")
 
 _HIP_KINDS = {
     "complex_phase_v1": ("axis", 1),

@@ -359,6 +359,21 @@ def test_operands_that_do_not_fit_are_refused():
             ops.linear_f32_grad(*args, w, parts, scale)
 
 
+def test_split_product_switch():
+    """RPFQ_SPLIT_LINEAR=0 leaves every training product to F.linear."""
+    import os
+    import subprocess
+    import sys
+
+    from quant_models import _native as N
+
+    for value, limit in (("0", "inf"), ("1", "4500000000.0")):
+        env = dict(os.environ, RPFQ_SPLIT_LINEAR=value, PYTHONPATH=os.path.dirname(os.path.dirname(N.__file__)))
+        out = subprocess.run([sys.executable, "-c", "from quant_models import quant_i; print(quant_i.SPLIT_LINEAR_MIN)"],
+                             env=env, capture_output=True, text=True, timeout=300)
+        assert out.stdout.strip() == limit, out.stderr
+
+
 def test_linear_f32_argument_errors():
     """Reported on the host, without a GPU."""
     from quant_models import _native as N
