@@ -591,8 +591,10 @@ int rpfq_wide_linear_grad_x_dense(const rpfq_wide_desc* desc, const void* packed
 int rpfq_attention(const void* qkv, int dtype, int64_t B, int64_t N, int64_t H, int64_t D, float scale, void* out,
                    void* stream);
 
-/* Bytes of the device workspace of rpfq_linear_f32 (backward = 0) or
- * rpfq_linear_f32_grad (backward = 1); 0 if the shape is not taken. */
+/* Bytes of the device workspace of rpfq_linear_f32 (backward = 0: about 4 M K
+ * and 4 N K) or rpfq_linear_f32_grad (backward = 1: about 4 M (N + K) and up to
+ * 64 partial grad_w of 4 N K, as many as keep the chip busy); 0 if the shape is
+ * not taken. */
 size_t rpfq_linear_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int backward);
 
 /*

@@ -22,6 +22,8 @@
 // output.  gw contracts over the rows, so a row's scale cannot be undone
 // after the sum: gy keeps its row scales r[m], and row m of x is taken times
 // 1 / r[m] times one power of two for the whole tensor.
+#include <algorithm>
+
 #include "rpfq_device.h"
 
 namespace rpfq {
@@ -870,8 +872,10 @@ F32Plan f32_plan(int64_t M, int64_t N, int64_t K) {
     at += (size_t)up(M * 4, 256);
     p.fwd_bytes = at;
     at = 256;
+    // x's planes; before they are written, the column sums of gy's blocks
     p.bx_at = at;
-    at += (size_t)up(p.Mp * p.Kp * 4 + slack, 256);
+    const int64_t xb = p.Mp * p.Kp * 4 + slack, cb = std::min<int64_t>(p.Mp / 4, kColBlocks) * N * 4;
+    at += (size_t)up(xb > cb ? xb : cb, 256);
     p.g_at = at;
     at += (size_t)up(p.Mp * p.Np * 4 + slack, 256);
     p.bw_at = at;
@@ -883,8 +887,6 @@ F32Plan f32_plan(int64_t M, int64_t N, int64_t K) {
     at += (size_t)up(M * 4, 256);
     p.steps = (int)(up(M, 16) / 16);
     p.splits = f32_splits(N, K, p.steps);
-    p.cs_at = at;
-    at += (size_t)up((int64_t)kColBlocks * N * 4, 256);
     p.part_at = at;
     if (p.splits > 1) at += (size_t)p.splits * N * K * 4;
     p.bwd_bytes = at;
@@ -1005,7 +1007,7 @@ hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* 
     RPFQ_TRY(split_w<1>(w, N, K, parts, nparts, base + p.bw_at, wscale, word, s));
     if (gb)
         RPFQ_TRY((split_rows<1, true>(gy, M, p.Mp, N, p.Np, xscale, nullptr, word, list, base + p.g_at, gscale, s,
-                                      reinterpret_cast<float*>(base + p.cs_at), gb)));
+                                      reinterpret_cast<float*>(base + p.bx_at), gb)));
     else
         RPFQ_TRY(split_rows<1>(gy, M, p.Mp, N, p.Np, xscale, nullptr, word, list, base + p.g_at, gscale, s));
     if (gx) {

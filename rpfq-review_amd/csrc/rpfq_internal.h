@@ -362,7 +362,7 @@ hipError_t launch_attention(const void* qkv, int dt, int64_t B, int64_t N, int64
 struct F32Plan {
     int64_t Mp, Kp, Np;          // padded rows and columns of the operand planes
     size_t x_at, w_at, wf_bytes, list_at, fwd_bytes;
-    size_t bx_at, g_at, bw_at, bwf_bytes, gs_at, blist_at, cs_at, part_at, bwd_bytes;
+    size_t bx_at, g_at, bw_at, bwf_bytes, gs_at, blist_at, part_at, bwd_bytes;
     int steps, splits;           // gw: 16-row steps, row splits
 };
 F32Plan f32_plan(int64_t M, int64_t N, int64_t K);

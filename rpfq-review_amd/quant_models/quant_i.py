@@ -329,6 +329,11 @@ QAT_PACKED_GRAD = os.environ.get("RPFQ_QAT_PACKED_GRAD", "0")
 # split fp16 operands (_split_linear_pays); RPFQ_SPLIT_LINEAR=0 keeps F.linear
 SPLIT_LINEAR_MIN = 4.5e9 if os.environ.get("RPFQ_SPLIT_LINEAR", "1") != "0" else float("inf")
 
+# ... and their planes of x and grad_y, 4 (K + N) bytes a row that a call holds
+# until it returns, stay below this; F.linear needs none (1.5% of the card, five
+# times ViT-B/16 fc1 at batch 256)
+SPLIT_LINEAR_SCRATCH = 4 << 30
+
 _HIP_KINDS = {
     "complex_phase_v1": ("axis", 1),
     "complex_phase_v2": ("axis", 2),
@@ -533,8 +538,8 @@ class _SplitLinearFn(torch.autograd.Function):
 
 def _split_linear_pays(x: torch.Tensor, w: torch.Tensor, bias) -> bool:
     """Whether float32 x and A_q take _SplitLinearFn: shapes the kernels hold
-    (rpfq_linear_f32) and enough work to cover the operand splits, and none of
-    the transforms that an autograd function without their rules refuses.
+    (rpfq_linear_f32), enough work to cover the operand splits, planes within
+    SPLIT_LINEAR_SCRATCH, and none of the transforms that an autograd function without their rules refuses.
     Operands that do not fit each other are left to F.linear, which says so.
     MI355X, forward + backward against the float32 library GEMMs, us: 12,608
     rows, 3072 x 768 (59 GFLOP a product) 596 against 1,492; 768 x 768 (15)
@@ -542,14 +547,15 @@ def _split_linear_pays(x: torch.Tensor, w: torch.Tensor, bias) -> bool:
     768 x 768 (1.9) 97 against 75; 512 rows, 4096 x 1024 (4.3) 163 against
     115."""
     n, k = w.shape
-    m = x.numel() // k
-    if x.dim() == 0 or x.shape[-1] != k or x.device != w.device:
+    if k == 0 or x.dim() == 0 or x.shape[-1] != k or x.device != w.device:
         return False
+    m = x.numel() // k
     if bias is not None and not (bias.shape == (n,) and bias.device == w.device and bias.is_contiguous()):
         return False
     if not (x.is_cuda and x.dtype == w.dtype == torch.float32 and (bias is None or bias.dtype == torch.float32)
             and n % 8 == 0 and k % 8 == 0 and n <= 4096 and k <= 4096 and m <= 1 << 24
-            and w.is_contiguous() and w.data_ptr() % 16 == 0 and m >= 1024 and 2 * m * n * k >= SPLIT_LINEAR_MIN):
+            and w.is_contiguous() and w.data_ptr() % 16 == 0 and m >= 1024 and 2 * m * n * k >= SPLIT_LINEAR_MIN
+            and 4 * m * (n + k) <= SPLIT_LINEAR_SCRATCH):
         return False
     if torch.is_autocast_enabled(x.device.type) or torch._C._are_functorch_transforms_active():
         return False

@@ -359,6 +359,32 @@ def test_operands_that_do_not_fit_are_refused():
             ops.linear_f32_grad(*args, w, parts, scale)
 
 
+def test_split_product_scratch():
+    """The workspace is the operands' planes and little else, and a layer whose
+    planes pass the limit keeps F.linear, which needs none."""
+    from types import SimpleNamespace
+
+    from quant_models import _native as N
+    from quant_models import quant_i
+
+    lib, m, n, k = N.load(), 496, 4096, 4096  # one split of grad_w
+    planes = 4 * 768 * (n + k) + 4 * n * k  # x, grad_y (768 padded rows), w
+    assert planes <= lib.rpfq_linear_f32_workspace_bytes(m, n, k, 1) <= planes + (1 << 20)
+    assert lib.rpfq_linear_f32_workspace_bytes(m, n, k, 0) <= planes
+    # the column sums of the bias gradient fit where x's planes go
+    assert lib.rpfq_linear_f32_workspace_bytes(4096, 4096, 8, 1) >= 1024 * 4096 * 4 + 4096 * 4096 * 4
+
+    def pays(m, n, k):
+        x = SimpleNamespace(dim=lambda: 2, shape=(m, k), numel=lambda: m * k, device=SimpleNamespace(type="cuda"),
+                            is_cuda=True, dtype=torch.float32)
+        w = SimpleNamespace(shape=(n, k), device=x.device, dtype=torch.float32, is_contiguous=lambda: True, data_ptr=lambda: 256)
+        return quant_i._split_linear_pays(x, w, None)
+
+    assert pays(12608, 3072, 768) and pays(1 << 18, 3072, 768)
+    assert not pays(12608, 4104, 768) and not pays(12608, 768, 4104)  # past the kernels' columns
+    assert not pays(1 << 19, 3072, 768) and not pays(1 << 24, 4096, 4096) and not pays(4096, 3072, 0)
+
+
 def test_split_product_switch():
     """RPFQ_SPLIT_LINEAR=0 leaves every training product to F.linear."""
     import os
