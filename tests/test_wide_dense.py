@@ -126,6 +126,34 @@ def test_dense_grad_x_matches_float64(m, n, k, cb, block, rot):
         assert bool(((gx.double() - exact).abs() <= bound).all())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_dense_grad_x_special_values(value, dt, monkeypatch):
+    """inf and NaN in a row of grad_y come out as in a float32 product and, also
+    beside values past fp16, as from the adjoint kernel; other rows keep theirs."""
+    from quant_models import ops
+
+    pw, g = _layer(1024, 136, 0, 0, None)
+    gy = torch.randn(600, 2048, device=DEV, generator=g).to(dt)
+    clean = pw.grad_x(gy)
+    assert pw._grad_dense_bytes(600, gy) > 0
+    gy[3, 70] = value
+    gy[599, 1500] = value
+    if dt != torch.float16:
+        gy[599, 1501] = 1e30  # finite, and past fp16
+    gx = pw.grad_x(gy, out_dtype=torch.float32)
+    ref = gy.float().cpu() @ pw.decode(round_fp16=True).cpu()
+    keep = [i for i in range(600) if i not in (3, 599)]
+    assert torch.equal(pw.grad_x(gy)[keep], clean[keep])
+    monkeypatch.setattr(ops, "DENSE", False)
+    adjoint = pw.grad_x(gy, out_dtype=torch.float32).cpu()
+    for r, other in ((3, adjoint), (599, adjoint), (3, ref)):
+        got, want = gx[r].cpu(), other[r]
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+        assert torch.equal(got[got.isinf()], want[want.isinf()])
+
+
 def test_dense_argument_errors():
     from quant_models import _native as N
     from quant_models import ops
