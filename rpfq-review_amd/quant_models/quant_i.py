@@ -367,14 +367,14 @@ def _blocks(a: torch.Tensor):
 
 
 class _HipWideQuantSTE(torch.autograd.Function):
-    """A_q from the float32 master weight by rpfq_quantize_wide, and its
-    scales (whose sum bounds |A_q|); backward:
+    """A_q from the float32 master weight by rpfq_quantize_wide; backward:
     the weight gets the A_q gradient unchanged (split and recombination are
     inverse linear maps and the quantizer is straight-through), the rotation
-    angles get rotation_grad."""
+    angles get rotation_grad.  parts (a list): takes the scales, whose sum
+    bounds |A_q|; as a second output they would cost every step a gradient."""
 
     @staticmethod
-    def forward(ctx, weight, theta_u, theta_w, spec):
+    def forward(ctx, weight, theta_u, theta_w, spec, parts=None):
         from . import ops
 
         rot = None
@@ -385,17 +385,17 @@ class _HipWideQuantSTE(torch.autograd.Function):
         ctx.rotated = theta_u is not None
         if ctx.rotated:
             ctx.save_for_backward(weight, a_q)
-        ctx.mark_non_differentiable(scales)
-        ctx.set_materialize_grads(False)  # else every backward fills zeros for the scales
-        return a_q, scales
+        if parts is not None:
+            parts.append(scales)
+        return a_q
 
     @staticmethod
-    def backward(ctx, grad, _):
-        if grad is None or not ctx.rotated:
-            return grad, None, None, None
+    def backward(ctx, grad):
+        if not ctx.rotated:
+            return grad, None, None, None, None
         weight, a_q = ctx.saved_tensors
         th_u, th_w = rotation_grad(grad.float(), weight.detach(), a_q)
-        return grad, th_u.reshape(1), th_w.reshape(1), None
+        return grad, th_u.reshape(1), th_w.reshape(1), None, None
 
 
 class _GivenWeightSTE(torch.autograd.Function):
@@ -656,15 +656,17 @@ class QATLinearComplexPhase(nn.Linear):
         if spec is not None and spec[0] == spec[2] and spec[1] == spec[3] and self._packed_grad():
             return self._qat_forward_packed_grad(x, spec)
         if spec is not None:
-            q_weight, scales = _HipWideQuantSTE.apply(self.weight, self.quantizer_u.rotation_angle,
-                                                      self.quantizer_w.rotation_angle, spec)
+            large = x.dtype == torch.float32 and 2 * x.numel() * self.out_features >= SPLIT_LINEAR_MIN
+            parts = [] if large else None  # _linear may take the split product
+            q_weight = _HipWideQuantSTE.apply(self.weight, self.quantizer_u.rotation_angle,
+                                              self.quantizer_w.rotation_angle, spec, parts)
             if self.act_quantizer is not None:
                 if x.dtype == torch.float32:
                     x = _HipActQuantSTE.apply(x, self.act_quantizer.num_bits)
                 else:  # reduced-precision activations: the reference's per-op rounding
                     h = self.in_features // 2
                     x = torch.cat(self.act_quantizer(x[..., :h], x[..., h:]), dim=-1)
-            return _linear(x, q_weight, self.bias, scales)
+            return _linear(x, q_weight, self.bias, parts[0] if parts else None)
         q_weight = self.quantized_weight()
         if self.act_quantizer is not None:
             h = self.in_features // 2

@@ -35,8 +35,8 @@ def _rot_cos_sin(tu, tw):
 
 @pytest.mark.parametrize("rotated", [False, True])
 def test_quantizer_backward_fills_nothing_for_its_scales(rotated, monkeypatch):
-    """The scales carry no gradient, and none is made for them: the backward
-    allocates and fills no zeros."""
+    """The scales are no output that carries a gradient: the backward allocates
+    and fills no zeros."""
     from torch.utils._python_dispatch import TorchDispatchMode
 
     from quant_models import ops, quant_i
@@ -52,7 +52,9 @@ def test_quantizer_backward_fills_nothing_for_its_scales(rotated, monkeypatch):
 
     w = torch.randn(8, 12, requires_grad=True)
     theta = [torch.zeros(1, requires_grad=True) if rotated else None for _ in range(2)]
-    a_q, _ = quant_i._HipWideQuantSTE.apply(w, *theta, ("axis", 2, "axis", 2))
+    parts = []
+    a_q = quant_i._HipWideQuantSTE.apply(w, *theta, ("axis", 2, "axis", 2), parts)
+    assert not parts[0].requires_grad and len(parts) == 1
     g = torch.randn(8, 12)
     with Record():
         a_q.backward(g)
