@@ -55,11 +55,16 @@ __device__ __forceinline__ float sum2(uint32_t v, float c) {
     }
 }
 
-// NB: 32-key blocks (N <= 32 NB)
+// NB: 32-key blocks (N <= 32 NB).  One block of keys is one block of queries
+// too: a workgroup of one wave, so that no wave waits beside it.  49,152 heads
+// of 5 tokens 39 us and of 32 tokens 189 us (on two blocks and four waves: 104
+// and 225; torch's: 60 bf16, 176 fp16, and 215).
+constexpr int attn_waves(int nb) { return nb == 1 ? 1 : 4; }
 template <int NB, bool BF>
-__global__ void __launch_bounds__(256, 2) attention_kernel(AttnArgs a) {
+__global__ void __launch_bounds__(64 * attn_waves(NB), 2) attention_kernel(AttnArgs a) {
     extern __shared__ __align__(16) char smem[];
     constexpr int KV = NB * 32 * 128;  // bytes of K, then of V
+    constexpr int W = attn_waves(NB);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
@@ -71,7 +76,7 @@ __global__ void __launch_bounds__(256, 2) attention_kernel(AttnArgs a) {
     // DMA of 8 rows per load: lane l fills row l >> 3, slot l & 7.  K: chunk c
     // at slot c ^ ((row >> 1) & 7); V: c ^ (((row >> 1) & 1) << 2).
     // Rows past N repeat row N - 1 (K: masked below; V: zeroed below).
-    for (int i = wave; i < 4 * NB; i += 4) {
+    for (int i = wave; i < 4 * NB; i += W) {
         const int t = 8 * i + (lane >> 3);
         const int64_t at = (int64_t)min(t, a.N - 1) * row;
         const uint32_t kc = (uint32_t)((lane & 7) ^ ((t >> 1) & 7)) * 16, vc = (uint32_t)((lane & 7) ^ (((t >> 1) & 1) << 2)) * 16;
@@ -79,7 +84,7 @@ __global__ void __launch_bounds__(256, 2) attention_kernel(AttnArgs a) {
         dma_dwordx4(base + a.H * 256, (uint32_t)at + vc, lds_addr(smem) + KV + i * 1024);
     }
     const int blocks = (a.N + 31) / 32;
-    int qb = part * 4 + wave;
+    int qb = part * W + wave;
     auto load_q = [&](int blk, uint4 (&q)[4]) {  // lane (r, g): d 16 s + 8 g .. + 7 of query 32 blk + r
         const char* src = base + (int64_t)min(32 * blk + r, a.N - 1) * row + 16 * g;
 #pragma unroll
@@ -90,9 +95,9 @@ __global__ void __launch_bounds__(256, 2) attention_kernel(AttnArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    // V rows past N (up to 63 of them: N = 1 on 2 blocks): a probability of 0
+    // V rows past N (up to 63 of them: 65 tokens on 4 blocks): a probability of 0
     // must meet a finite value
-    for (int t = a.N + (tid >> 3); t < 32 * NB; t += 32)
+    for (int t = a.N + (tid >> 3); t < 32 * NB; t += 8 * W)
         *reinterpret_cast<uint4*>(smem + KV + t * 128 + (tid & 7) * 16) = make_uint4(0, 0, 0, 0);
     __syncthreads();
 
@@ -108,7 +113,7 @@ __global__ void __launch_bounds__(256, 2) attention_kernel(AttnArgs a) {
     for (int j = 0; j < 2; ++j)
         voff[j] = lds_addr(smem) + KV + vr * 128 + (((4 * j + 2 * hf + ((i16 & 3) >> 1)) ^ (((vr >> 1) & 1) << 2)) * 16) + (i16 & 1) * 8;
 
-    for (; qb < blocks; qb += 4 * a.parts) {
+    for (; qb < blocks; qb += W * a.parts) {
         floatx16 s[NB];
         auto read_k = [&](int kb, u32x4 (&f)[4]) {
 #pragma unroll
@@ -130,10 +135,10 @@ __global__ void __launch_bounds__(256, 2) attention_kernel(AttnArgs a) {
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        // keys past N: in the last block, or the last two of the sizes that NB =
-        // 2 (N = 1 ..) and 4 (N = 65 ..) also serve
+        // keys past N: in the last block, or the last two where NB = 4 also
+        // serves N = 65 .. 96
 #pragma unroll
-        for (int kb = NB <= 4 ? NB - 2 : NB - 1; kb < NB; ++kb) {
+        for (int kb = NB == 4 ? NB - 2 : NB - 1; kb < NB; ++kb) {
 #pragma unroll
             for (int v = 0; v < 16; ++v)
                 if (32 * kb + acc_row(v, g) >= a.N) s[kb][v] = -__builtin_inff();
@@ -156,7 +161,7 @@ __global__ void __launch_bounds__(256, 2) attention_kernel(AttnArgs a) {
                 for (int v = 0; v < 16; ++v) s[kb][v] -= sub;
             mx -= sub;
         }
-        const int next = qb + 4 * a.parts;
+        const int next = qb + W * a.parts;
         load_q(next < blocks ? next : 0, q);
         // fp16: probabilities times 2^15, normal down to 2^-29 of the row's
         // largest, in sums below 2^39.  bf16 has float32's range and so have
@@ -224,14 +229,16 @@ static hipError_t attention_go(const AttnArgs& a, int64_t heads, hipStream_t s) 
     constexpr int lds = 2 * NB * 32 * 128;
     const hipError_t e = set_lds_attr_once(reinterpret_cast<const void*>(&attention_kernel<NB, BF>), lds, attr_done);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((attention_kernel<NB, BF>), dim3((unsigned)(heads * a.parts)), dim3(256), lds, s, a);
+    hipLaunchKernelGGL((attention_kernel<NB, BF>), dim3((unsigned)(heads * a.parts)), dim3(64 * attn_waves(NB)),
+                       lds, s, a);
     return hipGetLastError();
 }
 
 template <bool BF>
 static hipError_t attention_nb(const AttnArgs& a, int64_t heads, hipStream_t s) {
     switch ((a.N + 31) / 32) {
-        case 1: case 2: return attention_go<2, BF>(a, heads, s);
+        case 1: return attention_go<1, BF>(a, heads, s);
+        case 2: return attention_go<2, BF>(a, heads, s);
         case 3: case 4: return attention_go<4, BF>(a, heads, s);
         case 5: return attention_go<5, BF>(a, heads, s);
         case 6: return attention_go<6, BF>(a, heads, s);
