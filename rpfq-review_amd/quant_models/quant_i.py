@@ -539,13 +539,18 @@ class _SplitLinearFn(torch.autograd.Function):
 def _split_linear_pays(x: torch.Tensor, w: torch.Tensor, bias) -> bool:
     """Whether float32 x and A_q take _SplitLinearFn: shapes the kernels hold
     (rpfq_linear_f32), enough work to cover the operand splits, planes within
-    SPLIT_LINEAR_SCRATCH, and none of the transforms that an autograd function without their rules refuses.
-    Operands that do not fit each other are left to F.linear, which says so.
+    SPLIT_LINEAR_SCRATCH, and none of the transforms that an autograd function
+    without their rules refuses.  Operands that do not fit each other are left
+    to F.linear, which says so.
     MI355X, forward + backward against the float32 library GEMMs, us: 12,608
     rows, 3072 x 768 (59 GFLOP a product) 596 against 1,492; 768 x 768 (15)
-    235 against 452; 3,152 rows, 1000 x 768 (4.8) 130 against 190; 1,576 rows,
+    231 against 508; 4,096 rows, 1000 x 768 (6.3) 160 against 204; 1,576 rows,
     768 x 768 (1.9) 97 against 75; 512 rows, 4096 x 1024 (4.3) 163 against
-    115."""
+    115.  Narrow layers move more bytes in the splits than the products save:
+    401,408 rows of 96 x 96 949 against 1,209, but 1,048,576 of 64 x 64 2,599
+    against 1,914 and 524,288 of 384 x 32 level; a forward alone of 401,408
+    rows of 96 x 384 478 against 321, of 100,352 rows of 192 x 768 250 against
+    309."""
     n, k = w.shape
     if k == 0 or x.dim() == 0 or x.shape[-1] != k or x.device != w.device:
         return False
@@ -555,7 +560,8 @@ def _split_linear_pays(x: torch.Tensor, w: torch.Tensor, bias) -> bool:
     if not (x.is_cuda and x.dtype == w.dtype == torch.float32 and (bias is None or bias.dtype == torch.float32)
             and n % 8 == 0 and k % 8 == 0 and n <= 4096 and k <= 4096 and m <= 1 << 24
             and w.is_contiguous() and w.data_ptr() % 16 == 0 and m >= 1024 and 2 * m * n * k >= SPLIT_LINEAR_MIN
-            and 4 * m * (n + k) <= SPLIT_LINEAR_SCRATCH):
+            and 4 * m * (n + k) <= SPLIT_LINEAR_SCRATCH
+            and min(n, k) >= (96 if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad) else 192)):
         return False
     if torch.is_autocast_enabled(x.device.type) or torch._C._are_functorch_transforms_active():
         return False

@@ -359,13 +359,32 @@ def test_operands_that_do_not_fit_are_refused():
             ops.linear_f32_grad(*args, w, parts, scale)
 
 
+def _pays(m, n, k, grad=True):
+    from types import SimpleNamespace
+
+    from quant_models import quant_i
+
+    x = SimpleNamespace(dim=lambda: 2, shape=(m, k), numel=lambda: m * k, device=SimpleNamespace(type="cuda"), is_cuda=True,
+                        dtype=torch.float32, requires_grad=False)
+    w = SimpleNamespace(shape=(n, k), device=x.device, dtype=torch.float32, is_contiguous=lambda: True, data_ptr=lambda: 256,
+                        requires_grad=grad)
+    return quant_i._split_linear_pays(x, w, None)
+
+
+def test_split_product_leaves_narrow_layers_to_the_library():
+    """Layers whose splits move more than the products save."""
+    assert _pays(401408, 288, 96) and _pays(100352, 192, 192) and _pays(100352, 192, 768, grad=False)
+    for m, n, k in ((1 << 20, 64, 64), (1 << 19, 384, 32), (1 << 19, 32, 384), (150000, 1024, 16), (1 << 17, 8, 4096)):
+        assert 2 * m * n * k > 4.5e9 and not _pays(m, n, k)
+    assert not _pays(401408, 96, 384, grad=False)
+    with torch.no_grad():
+        assert not _pays(401408, 96, 384) and _pays(12608, 3072, 768)
+
+
 def test_split_product_scratch():
     """The workspace is the operands' planes and little else, and a layer whose
     planes pass the limit keeps F.linear, which needs none."""
-    from types import SimpleNamespace
-
     from quant_models import _native as N
-    from quant_models import quant_i
 
     lib, m, n, k = N.load(), 496, 4096, 4096  # one split of grad_w
     planes = 4 * 768 * (n + k) + 4 * n * k  # x, grad_y (768 padded rows), w
@@ -374,15 +393,9 @@ def test_split_product_scratch():
     # the column sums of the bias gradient fit where x's planes go
     assert lib.rpfq_linear_f32_workspace_bytes(4096, 4096, 8, 1) >= 1024 * 4096 * 4 + 4096 * 4096 * 4
 
-    def pays(m, n, k):
-        x = SimpleNamespace(dim=lambda: 2, shape=(m, k), numel=lambda: m * k, device=SimpleNamespace(type="cuda"),
-                            is_cuda=True, dtype=torch.float32)
-        w = SimpleNamespace(shape=(n, k), device=x.device, dtype=torch.float32, is_contiguous=lambda: True, data_ptr=lambda: 256)
-        return quant_i._split_linear_pays(x, w, None)
-
-    assert pays(12608, 3072, 768) and pays(1 << 18, 3072, 768)
-    assert not pays(12608, 4104, 768) and not pays(12608, 768, 4104)  # past the kernels' columns
-    assert not pays(1 << 19, 3072, 768) and not pays(1 << 24, 4096, 4096) and not pays(4096, 3072, 0)
+    assert _pays(12608, 3072, 768) and _pays(1 << 18, 3072, 768)
+    assert not _pays(12608, 4104, 768) and not _pays(12608, 768, 4104)  # past the kernels' columns
+    assert not _pays(1 << 19, 3072, 768) and not _pays(1 << 24, 4096, 4096) and not _pays(4096, 3072, 0)
 
 
 def test_split_product_switch():
