@@ -403,8 +403,9 @@ class PackedWide:
         -> 16; float32 outputs (whole-line stores) with a residual 12,608
         rows of proj 73 -> 42, without 12,608 rows of fc1 96 -> 90 but 3,152
         of qkv 29 -> 34; long K' on few 128-row tiles (64- and 96-row tiles
-        fill the chip) 12,608 rows of fc2 93 -> 76, 25,216 147 -> 143.
-        Everything else is within 4% either way, power-limited."""
+        fill the chip) 12,608 rows of fc2 93 -> 76, 25,216 147 -> 143, but one
+        or two column tiles from a whole round of the chip on 1.0-1.2x the
+        time (31,379 rows of 48 x 2048 float32 222 -> 255).  Everything else is within 4% either way, power-limited."""
         ops = wide_flops(m, self.n_complex, self.k_complex)
         tiles = -(-m // 128) * -(-self.n_complex // 128)
         if flags & N.FLAG_GELU:
@@ -415,7 +416,7 @@ class PackedWide:
             least = math.inf
         if self.n_complex % 8:
             least = min(least, 1.5e9)
-        if self.k_complex >= 1024 and tiles <= 512:
+        if self.k_complex >= 1024 and (tiles <= 512 if self.n_complex > 256 else tiles < 256):
             least = min(least, 5e9)
         if (not DENSE or ops < least or m < 128 or x2.dtype != torch.float16 or flags & ~N.FLAG_GELU
                 or self.kernel_for(m, torch.float16, out_dtype, flags) != N.KERNEL_DMA):
@@ -592,14 +593,19 @@ class PackedWide:
         rows 69 -> 38, 12,608 rows of 288 x 96 18 -> 14 but 96 x 96 11 -> 14;
         bf16 fc1 135 -> 90, 384 x 384 at 512 rows 29 -> 23 but 288 x 96 at
         12,608 rows 23 -> 26; float32 fc1 156 -> 106, 1152 x 384 at 512 rows
-        50 -> 35, 384 x 384 at 12,608 rows 48 -> 37 but at 3,152 22 -> 23."""
+        50 -> 35, 384 x 384 at 12,608 rows 48 -> 37 but at 3,152 22 -> 23, 384
+        x 160 at 16,384 1.12x.  Short rows of the gradient cannot cover that
+        pass once there are many: 52,399 rows of 1024 x 64 bf16 117 -> 148,
+        24,893 of 1024 x 96 float32 83 -> 94; 8,192 of 1536 x 96 0.77x."""
         n, ops = self.n_complex, wide_flops(m, self.n_complex, self.k_complex)
         if g2.dtype == torch.float16:
             pays = n >= 256
         elif g2.dtype == torch.bfloat16:
             pays = n >= 384
         else:
-            pays = n >= 1024 or (n >= 384 and ops >= 5e9)
+            pays = n >= 1024 or (n >= 384 and ops >= (5e9 if n >= 768 else 1e10))
+        if g2.dtype != torch.float16 and self.k_complex <= 128 and m > 16384:
+            pays = False
         if not DENSE or not pays or ops < 5e8 or m < 128 or (g2.dtype != torch.float16 and 2 * n > 4096):
             return 0
         return N.load().rpfq_wide_dense_bytes(ctypes.byref(self.desc), 1)

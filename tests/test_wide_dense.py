@@ -154,6 +154,27 @@ def test_dense_grad_x_special_values(value, dt, monkeypatch):
         assert torch.equal(got[got.isinf()], want[want.isinf()])
 
 
+def test_decoded_weight_routes():
+    """Where the decoded weight is left to the kernels that decode in their
+    loop: few columns over many rows, and gradients of short rows that their
+    prescale pass outweighs."""
+    from types import SimpleNamespace
+
+    from quant_models import _native as N
+    from quant_models import ops
+
+    def routes(m, n, k, dt):
+        pw = ops.PackedWide(n, k, N.CB_AXIS, 2, 0, torch.empty(0, dtype=torch.uint8), None)
+        half, g = SimpleNamespace(dtype=torch.float16), SimpleNamespace(dtype=dt)
+        return pw._dense_bytes(m, half, dt, 0, False) > 0, pw._grad_dense_bytes(m, g) > 0
+
+    for dt in DTYPES:
+        assert routes(12608, 384, 1536, dt) == (True, True) and routes(16000, 48, 2048, dt)[0]
+        assert not routes(32768, 48, 2048, torch.float16)[0] and not routes(40000, 192, 1024, torch.float16)[0]
+        assert routes(50432, 1024, 96, dt)[1] == (dt == torch.float16) and routes(8192, 1536, 96, dt)[1]
+    assert not routes(16384, 384, 160, torch.float32)[1] and routes(8192, 768, 128, torch.float32)[1]
+
+
 def test_dense_argument_errors():
     from quant_models import _native as N
     from quant_models import ops
