@@ -134,20 +134,15 @@ bool layer(PyObject* desc, PyObject* blob, PyObject* x, PyObject* residual, PyOb
     return true;
 }
 
-// Launches run without the interpreter lock, as through ctypes: one that waits
-// for room in the queue must not hold up the other threads, or a host function
-// in that queue that needs the lock.
+// Allocations and launches run without the interpreter lock, as through torch
+// and ctypes: one that waits for memory or for room in the queue must not hold
+// up the other threads, or a host function in that queue that needs the lock.
 struct Unlocked {
     PyThreadState* state = PyEval_SaveThread();
     Unlocked() = default;
     Unlocked(const Unlocked&) = delete;
     ~Unlocked() { PyEval_RestoreThread(state); }
 };
-template <class F, class... A>
-int launch(F f, A... a) {
-    Unlocked u;
-    return f(a...);
-}
 
 PyObject* done(int rc, const at::Tensor& y) {
     if (rc != RPFQ_OK) Py_RETURN_NONE;
@@ -165,24 +160,27 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 8 || !number(a[6], &flags) || !number(a[7], &guard) || !layer(a[0], a[1], a[2], a[4], a[5], c) ||
         !vec(a[3], 2 * c.d->n_complex, &bias))
         Py_RETURN_NONE;
-    const float* scale = nullptr;
-    at::Tensor s;
     const int64_t in = 2 * c.d->k_complex;
     const bool scaled = c.xdt != RPFQ_F16 && (guard & 1);
     int kernel = -1;
     if (scaled && (guard & 2) && in <= 4096 &&
         api.rpfq_wide_linear_kernel(c.d, c.m, RPFQ_F16, c.ydt, (int)flags, &kernel) == RPFQ_OK && kernel == RPFQ_KERNEL_DMA)
         Py_RETURN_NONE;
-    c.take();
-    if (scaled) {
-        s = at::empty({c.m}, c.x->options().dtype(at::kFloat));
-        scale = s.const_data_ptr<float>();
-        if (launch(api.rpfq_row_scales, c.x->data_ptr(), c.xdt, c.m, in, s.data_ptr<float>(), c.stream) != RPFQ_OK)
-            Py_RETURN_NONE;
+    int rc = RPFQ_OK;
+    {
+        Unlocked u;
+        c.take();
+        at::Tensor s;
+        if (scaled) {
+            s = at::empty({c.m}, c.x->options().dtype(at::kFloat));
+            rc = api.rpfq_row_scales(c.x->data_ptr(), c.xdt, c.m, in, s.data_ptr<float>(), c.stream);
+        }
+        if (rc == RPFQ_OK)
+            rc = api.rpfq_wide_linear_scaled(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m,
+                                             scaled ? s.const_data_ptr<float>() : nullptr, bias, c.res, c.y.data_ptr(),
+                                             c.ydt, (int)flags, c.stream);
     }
-    return done(launch(api.rpfq_wide_linear_scaled, c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m,
-                       scale, bias, c.res, c.y.data_ptr(), c.ydt, (int)flags, c.stream),
-                c.y);
+    return done(rc, c.y);
     END_HANDLE_TH_ERRORS
 }
 
@@ -200,10 +198,14 @@ PyObject* layer_norm_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!vec(a[3], in, &w) || !vec(a[4], in, &b) || !vec(a[6], 2 * c.d->n_complex, &bias) ||
         api.rpfq_layer_norm_wide_linear_fusable(c.d, c.m, c.xdt, c.ydt, &fusable) != RPFQ_OK || !fusable)
         Py_RETURN_NONE;
-    c.take();
-    return done(launch(api.rpfq_layer_norm_wide_linear, c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt,
-                       c.m, w, b, eps, bias, c.y.data_ptr(), c.ydt, (int)flags, c.stream),
-                c.y);
+    int rc;
+    {
+        Unlocked u;
+        c.take();
+        rc = api.rpfq_layer_norm_wide_linear(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m, w, b,
+                                             eps, bias, c.y.data_ptr(), c.ydt, (int)flags, c.stream);
+    }
+    return done(rc, c.y);
     END_HANDLE_TH_ERRORS
 }
 
@@ -218,10 +220,15 @@ PyObject* act_quant_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 8 || !number(a[3], &bits) || !number(a[7], &flags) || !layer(a[0], a[1], a[2], a[5], a[6], c) || !vec(a[4], 2 * c.d->n_complex, &bias) ||
         api.rpfq_layer_norm_wide_linear_fusable(c.d, c.m, c.xdt, c.ydt, &fusable) != RPFQ_OK || !fusable)
         Py_RETURN_NONE;
-    c.take();
-    return done(launch(api.rpfq_act_quant_wide_linear, c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt,
-                       c.m, (int)bits, 0, nullptr, nullptr, 0.0f, bias, c.res, c.y.data_ptr(), c.ydt, (int)flags, c.stream),
-                c.y);
+    int rc;
+    {
+        Unlocked u;
+        c.take();
+        rc = api.rpfq_act_quant_wide_linear(c.d, c.blob->data_ptr(), c.blob->nbytes(), c.x->data_ptr(), c.xdt, c.m,
+                                            (int)bits, 0, nullptr, nullptr, 0.0f, bias, c.res, c.y.data_ptr(), c.ydt,
+                                            (int)flags, c.stream);
+    }
+    return done(rc, c.y);
     END_HANDLE_TH_ERRORS
 }
 
@@ -235,10 +242,15 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!q || q->dim() != 3 || h < 1 || q->size(2) != 192 * h ||
         q->numel() == 0 || !rows16(*q))
         Py_RETURN_NONE;
-    at::Tensor y = at::empty({q->size(0), q->size(1), 64 * h}, q->options());
-    return done(launch(api.rpfq_attention, q->data_ptr(), dtype_code(q->scalar_type()), q->size(0), q->size(1), h, 64,
-                       scale, y.data_ptr(), c10::hip::getCurrentHIPStream(q->device().index()).stream()),
-                y);
+    at::Tensor y;
+    int rc;
+    {
+        Unlocked u;
+        y = at::empty({q->size(0), q->size(1), 64 * h}, q->options());
+        rc = api.rpfq_attention(q->data_ptr(), dtype_code(q->scalar_type()), q->size(0), q->size(1), h, 64, scale,
+                                y.data_ptr(), c10::hip::getCurrentHIPStream(q->device().index()).stream());
+    }
+    return done(rc, y);
     END_HANDLE_TH_ERRORS
 }
 
