@@ -611,7 +611,8 @@ size_t rpfq_linear_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int back
  * or the sum is not finite.
  * w_parts[n_parts] (device): values whose absolute sum bounds every |w|
  * (the scales rpfq_quantize_wide wrote for w; 0 only if w is all 0).
- * x_scale [M] (out): the power-of-two scale of each row of x, read by
+ * x_scale [M] (out): the power-of-two scale of each row of x (negative, 0 or
+ * inf: a row summed in plain float32, with inf or NaN, of zeros), read by
  * rpfq_linear_f32_grad.  x, w, y 16-byte, work 256-byte aligned.
  * Replaces F.linear(x, A_q, bias) of RPFQ-ViT-main/quant_models/quant_i.py:554
  * on float32 activations in training.

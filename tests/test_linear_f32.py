@@ -337,6 +337,41 @@ def test_transformed_gradients_take_torch_products(monkeypatch):
 
 
 @pytest.mark.gpu
+def test_split_product_in_a_captured_graph():
+    """Forward and gradients captured once and replayed on other operands, some
+    with rows that are summed apart: every replay gives the eager bits."""
+    from quant_models import ops
+
+    x, w, b, gy = _inputs(1500, 136, 264)
+    parts, gb = w.abs().max().reshape(1), torch.empty(136, device=DEV)
+
+    def step():
+        y, scale = ops.linear_f32(x, w, b, parts)
+        return (y, *ops.linear_f32_grad(gy, x, w, parts, scale, grad_b=gb), gb)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = step()
+    for k in range(5):
+        x.normal_()
+        gy.normal_()
+        if k == 1:
+            x[5, 3], gy[7, 9] = float("nan"), float("inf")
+        if k == 2:
+            x[11, 7], gy[900:] = 2.0 ** 25, gy[900:] * 2.0 ** -30
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in outs]
+        for a, c in zip(got, step()):
+            assert torch.equal(a.view(torch.int32), c.view(torch.int32)) or torch.equal(a.nan_to_num(7.0), c.nan_to_num(7.0))
+
+
+@pytest.mark.gpu
 def test_operands_that_do_not_fit_are_refused():
     """By F.linear's own error from the layer, by the host checks below it."""
     from quant_models import ops
