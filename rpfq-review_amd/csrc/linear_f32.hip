@@ -35,8 +35,8 @@ constexpr int kF32NoRow = -100000;
 // What the passes of a call leave for the ones behind them, in its workspace.
 struct F32Words {
     int emax;   // gw: largest exponent of a row's product of maxima, or kF32NoRow
-    int gw;     // gw has rows that f32_exact_gw_kernel adds
-    int rows;   // rows of y / gx that f32_exact_rows_kernel writes
+    int gw;     // gw has rows that f32_exact_grad_kernel adds
+    int rows;   // rows of y / gx that f32_exact_rows writes
 };
 // Most blocks of the gy pass where it also sums columns: 4 a CU.
 constexpr int kColBlocks = 1024;
@@ -45,7 +45,7 @@ __device__ __forceinline__ int f32_scale_exp(float s) {  // s = 2^e
     return (int)((__float_as_uint(s) >> 23) & 0xffu) - 127;
 }
 
-// Rows of gw that f32_exact_gw_kernel sums, by the scales of gy's and x's row:
+// Rows of gw that f32_exact_grad_kernel sums, by the scales of gy's and x's row:
 // inf or NaN (0), a wide row (negative), or a product of maxima more than 2^14
 // below the largest such product.
 __device__ __forceinline__ bool gw_listed(float r, float sx, int emax) {
@@ -610,7 +610,7 @@ __global__ void __launch_bounds__(256, 2) f32_gw_kernel(F32GwArgs a) {
     }
 }
 
-// gw = 2^emax (1 after f32_exact_gw_kernel) times the sum of the splits'
+// gw = 2^emax (1 after f32_exact_grad_kernel) times the sum of the splits'
 // partials, in their order.
 __global__ void __launch_bounds__(256) f32_gw_reduce_kernel(const float* part, int64_t n4, int splits, const F32Words* word,
                                                            float* gw) {
@@ -769,17 +769,17 @@ __device__ __forceinline__ void f32_exact_store(const F32Exact& x, int64_t i0, i
 }
 
 // The listed rows of y = x w^T + bias (BC) or gx = gy w, or every row where w
-// has no scale.  C: the contraction.
+// has no scale: block `first` of `blocks`.  C: the contraction.
 template <bool BC>
-__global__ void __launch_bounds__(256, 2) f32_exact_rows_kernel(F32Exact x, int C, const F32Words* word, const float* wscale) {
-    __shared__ float lds[4 * kExHalf];
+__device__ __forceinline__ void f32_exact_rows(F32Exact x, float* lds, int C, const F32Words* word, const float* wscale,
+                                               int first, int blocks) {
     if (wscale[0] == 0.0f)
         x.list = nullptr;
     else
         x.I = word->rows;
     const int tj = (x.J + 127) / 128;
     const int64_t tiles = (x.I + 127) / 128 * tj;
-    for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+    for (int64_t t = first; t < tiles; t += blocks) {
         F32ExactSum s;
         s.zero();
         f32_exact_add<true, BC>(x, lds, t / tj * 128, (int)(t % tj) * 128, 0, C, nullptr, s);
@@ -787,28 +787,49 @@ __global__ void __launch_bounds__(256, 2) f32_exact_rows_kernel(F32Exact x, int 
     }
 }
 
-// Adds the listed rows' share to gw (splits = 1) or to the partial sums, which
-// leave their unit 2^emax with it (the listed rows may lie far above).  Split sp takes the listed ones of the rows of split sp of
-// f32_gw_kernel, in their order, 1,024 rows at a time through LDS.
-__global__ void __launch_bounds__(256, 2) f32_exact_gw_kernel(F32Exact x, int64_t M, int64_t per, int splits,
-                                                             const float* gscale, const float* xscale, const F32Words* word) {
+__global__ void __launch_bounds__(256, 2) f32_exact_y_kernel(F32Exact x, int C, const F32Words* word, const float* wscale) {
+    __shared__ float lds[4 * kExHalf];
+    f32_exact_rows<true>(x, lds, C, word, wscale, blockIdx.x, gridDim.x);
+}
+
+// Both gradients' share in one launch: the first gx_blocks blocks the listed
+// rows of gx; the others, one per tile of gw and row split of f32_gw_kernel,
+// add the listed rows' share to gw (splits = 1) or to the partial sums, which
+// leave their unit 2^emax with it (the listed rows may lie far above), in the
+// rows' order, 1,024 rows at a time through LDS.
+struct F32ExactGrad {
+    F32Exact gx, gw;
+    int gx_blocks, N;
+    int64_t M, per;
+    int splits;
+    const float *gscale, *xscale, *wscale;
+    const F32Words* word;
+};
+__global__ void __launch_bounds__(256, 2) f32_exact_grad_kernel(F32ExactGrad a) {
     __shared__ float lds[4 * kExHalf];
     __shared__ int rows[1024], total[4];
-    if (word->gw == 0) return;
-    const int emax = word->emax, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int tj = (x.J + 127) / 128, j0 = (int)(blockIdx.x % tj) * 128;
-    const int64_t i0 = (int64_t)(blockIdx.x / tj) * 128;
-    const int64_t m1 = min(M, ((int64_t)blockIdx.y + 1) * per);
-    x.out += (int64_t)blockIdx.y * x.I * x.J;
+    if ((int)blockIdx.x < a.gx_blocks) {
+        f32_exact_rows<false>(a.gx, lds, a.N, a.word, a.wscale, blockIdx.x, a.gx_blocks);
+        return;
+    }
+    if (a.word->gw == 0) return;
+    F32Exact x = a.gw;
+    const int emax = a.word->emax, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int tj = (x.J + 127) / 128, tiles = (int)((x.I + 127) / 128) * tj;
+    const int unit = blockIdx.x - a.gx_blocks, sp = unit / tiles, tile = unit - sp * tiles;
+    const int j0 = tile % tj * 128;
+    const int64_t i0 = (int64_t)(tile / tj) * 128;
+    const int64_t m1 = min(a.M, ((int64_t)sp + 1) * a.per);
+    x.out += (int64_t)sp * x.I * x.J;
     F32ExactSum s;
     s.zero();
-    for (int64_t m0 = (int64_t)blockIdx.y * per; m0 < m1; m0 += 1024) {
+    for (int64_t m0 = (int64_t)sp * a.per; m0 < m1; m0 += 1024) {
         bool on[4];
         int n = 0;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const int64_t m = m0 + 4 * threadIdx.x + t;
-            on[t] = m < m1 && gw_listed(gscale[m], xscale[m], emax);
+            on[t] = m < m1 && gw_listed(a.gscale[m], a.xscale[m], emax);
             n += on[t];
         }
         int before = n;  // of the lanes up to this one
@@ -831,7 +852,7 @@ __global__ void __launch_bounds__(256, 2) f32_exact_gw_kernel(F32Exact x, int64_
         if (count) f32_exact_add<false, false>(x, lds, i0, j0, 0, count, rows, s);
         __syncthreads();  // total and rows are read
     }
-    f32_exact_store<true>(x, i0, j0, s, splits > 1 && emax != kF32NoRow ? emax : 0);
+    f32_exact_store<true>(x, i0, j0, s, a.splits > 1 && emax != kF32NoRow ? emax : 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -945,24 +966,9 @@ static hipError_t f32_gemm(F32Args& a, hipStream_t s) {
     return f32_gemm_go<4>(a, s);
 }
 
-// a [M, C], out [M, J], b [J, C] (BC) or [C, J].
-template <bool BC>
-static hipError_t exact_rows(const float* a, const float* b, const float* bias, float* out, const int* list, int64_t M,
-                             int64_t J, int64_t C, const F32Words* word, const float* wscale, hipStream_t s) {
-    F32Exact x = {};
-    x.a = a;
-    x.b = b;
-    x.bias = bias;
-    x.out = out;
-    x.list = list;
-    x.lda = C;
-    x.ldb = BC ? C : J;
-    x.I = M;
-    x.J = (int)J;
-    const int64_t tiles = (M + 127) / 128 * ((J + 127) / 128), most = 2 * (int64_t)device_cus();
-    hipLaunchKernelGGL((f32_exact_rows_kernel<BC>), dim3((unsigned)(tiles < most ? tiles : most)), dim3(256), 0, s, x, (int)C,
-                       word, wscale);
-    return hipGetLastError();
+// Blocks of f32_exact_rows for rows x J outputs.
+static int exact_blocks(int64_t rows, int64_t J) {
+    return (int)std::min<int64_t>((rows + 127) / 128 * ((J + 127) / 128), 2 * (int64_t)device_cus());
 }
 
 #define RPFQ_TRY(e)                           \
@@ -992,7 +998,18 @@ hipError_t launch_linear_f32(const float* x, const float* w, const float* bias, 
     a.KS = (int)(p.Kp / 32);
     a.wf_bytes = (int)p.wf_bytes;
     RPFQ_TRY(f32_gemm(a, s));
-    return exact_rows<true>(x, w, bias, y, list, M, N, K, word, wscale, s);
+    F32Exact e = {};
+    e.a = x;
+    e.b = w;
+    e.bias = bias;
+    e.out = y;
+    e.list = list;
+    e.lda = e.ldb = K;
+    e.I = M;
+    e.J = (int)N;
+    hipLaunchKernelGGL(f32_exact_y_kernel, dim3(exact_blocks(M, N)), dim3(256), 0, s, e, (int)K, (const F32Words*)word,
+                       (const float*)wscale);
+    return hipGetLastError();
 }
 
 hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* w, int64_t M, int64_t N, int64_t K,
@@ -1004,6 +1021,15 @@ hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* 
     F32Words* word = reinterpret_cast<F32Words*>(base + 64);
     int* list = reinterpret_cast<int*>(base + p.blist_at);
     float* gscale = reinterpret_cast<float*>(base + p.gs_at);
+    F32ExactGrad e = {};
+    e.M = M;
+    e.N = (int)N;
+    e.splits = p.splits;
+    e.gscale = gscale;
+    e.xscale = xscale;
+    e.wscale = wscale;
+    e.word = word;
+    int exact = 0;  // blocks
     RPFQ_TRY(split_w<1>(w, N, K, parts, nparts, base + p.bw_at, wscale, word, s));
     if (gb)
         RPFQ_TRY((split_rows<1, true>(gy, M, p.Mp, N, p.Np, xscale, nullptr, word, list, base + p.g_at, gscale, s,
@@ -1022,7 +1048,15 @@ hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* 
         a.KS = (int)(p.Np / 32);
         a.wf_bytes = (int)p.bwf_bytes;
         RPFQ_TRY(f32_gemm(a, s));
-        RPFQ_TRY(exact_rows<false>(gy, w, nullptr, gx, list, M, K, N, word, wscale, s));
+        e.gx.a = gy;
+        e.gx.b = w;
+        e.gx.out = gx;
+        e.gx.list = list;
+        e.gx.lda = N;
+        e.gx.ldb = K;
+        e.gx.I = M;
+        e.gx.J = (int)K;
+        exact = e.gx_blocks = exact_blocks(M, K);
     }
     if (gw) {
         RPFQ_TRY(split_rows<2>(x, M, p.Mp, K, p.Kp, xscale, gscale, word, nullptr, base + p.bx_at, nullptr, s));
@@ -1044,24 +1078,24 @@ hipError_t launch_linear_f32_grad(const float* gy, const float* x, const float* 
         g.splits = p.splits;
         hipLaunchKernelGGL(f32_gw_kernel, dim3(g.tiles_n * g.tiles_k * g.splits), dim3(256), kGwLds, s, g);
         RPFQ_TRY(hipGetLastError());
-        F32Exact x2 = {};
-        x2.a = gy;
-        x2.b = x;
-        x2.out = g.part;
-        x2.lda = N;
-        x2.ldb = K;
-        x2.I = N;
-        x2.J = (int)K;
-        hipLaunchKernelGGL(f32_exact_gw_kernel, dim3((unsigned)(((N + 127) / 128) * ((K + 127) / 128)), p.splits), dim3(256), 0,
-                           s, x2, M, (int64_t)g.per * 16, p.splits, (const float*)gscale, xscale, (const F32Words*)word);
+        e.gw.a = gy;
+        e.gw.b = x;
+        e.gw.out = g.part;
+        e.gw.lda = N;
+        e.gw.ldb = K;
+        e.gw.I = N;
+        e.gw.J = (int)K;
+        e.per = (int64_t)g.per * 16;
+        exact += (int)(((N + 127) / 128) * ((K + 127) / 128)) * p.splits;
+    }
+    hipLaunchKernelGGL(f32_exact_grad_kernel, dim3((unsigned)exact), dim3(256), 0, s, e);
+    RPFQ_TRY(hipGetLastError());
+    if (gw && p.splits > 1) {
+        const int64_t n4 = N * K / 4;
+        const int grid = (int)((n4 + 255) / 256 < 2048 ? (n4 + 255) / 256 : 2048);
+        hipLaunchKernelGGL(f32_gw_reduce_kernel, dim3(grid), dim3(256), 0, s,
+                           (const float*)reinterpret_cast<float*>(base + p.part_at), n4, p.splits, (const F32Words*)word, gw);
         RPFQ_TRY(hipGetLastError());
-        if (p.splits > 1) {
-            const int64_t n4 = N * K / 4;
-            const int grid = (int)((n4 + 255) / 256 < 2048 ? (n4 + 255) / 256 : 2048);
-            hipLaunchKernelGGL(f32_gw_reduce_kernel, dim3(grid), dim3(256), 0, s, (const float*)g.part, n4, p.splits,
-                               (const F32Words*)word, gw);
-            RPFQ_TRY(hipGetLastError());
-        }
     }
     return hipSuccess;
 }
