@@ -311,8 +311,8 @@ class PackedWide:
             flags = int(flags) | N.FLAG_GELU
         host = N.host()
         if host is not None and row_scale is None and _launch_recorder is None:
-            y = host.linear(ctypes.addressof(self.desc), self.blob, x, bias, residual, out_dtype, int(flags),
-                            int(RANGE_GUARD) + 2 * int(PRESCALE_ROWS))
+            y = host.linear(ctypes.addressof(self.desc), self.blob, x, bias, residual, out_dtype, flags,
+                            RANGE_GUARD + 2 * PRESCALE_ROWS)
             if y is not None:
                 return y
         N.require_device(x, bias, residual, row_scale)
@@ -477,7 +477,7 @@ class PackedWide:
         ln_fusable(); gelu as in linear() (not with a residual)."""
         host = N.host()
         if host is not None and layer_norm is None:
-            y = host.act_quant_linear(ctypes.addressof(self.desc), self.blob, x, int(bits), bias, residual, out_dtype,
+            y = host.act_quant_linear(ctypes.addressof(self.desc), self.blob, x, bits, bias, residual, out_dtype,
                                       N.FLAG_GELU if gelu else 0)
             if y is not None:
                 return y
@@ -776,7 +776,7 @@ def attention(qkv: torch.Tensor, num_heads: int, scale: float) -> torch.Tensor:
     bf16, heads of 64 values, N <= ATTENTION_MAX_TOKENS; rpfq_attention)."""
     host = N.host()
     if host is not None:
-        out = host.attention(qkv, num_heads, float(scale))
+        out = host.attention(qkv, num_heads, scale)
         if out is not None:
             return out
     if qkv.dim() != 3 or num_heads < 1 or qkv.shape[2] % (3 * num_heads):
