@@ -319,9 +319,10 @@ PRESCALED_LN = os.environ.get("RPFQ_PRESCALED_LN", "1") != "0"
 # step's own codes (rpfq_wide_linear_grad_x) instead of the library GEMM on
 # A_q: "1" on (each grad_y element of a float32 step then carries one fp16
 # rounding, 2^-11 relative, and the fused fp16 coefficients replace A_q),
-# "0" (default) off.  Measured on ViT-B/16 bs64, MI355X: float32 steps gain
-# 2-5% (the kernel is ~3x faster than the float32 library GEMM); fp16
-# autocast steps lose 20% (2,042 -> 1,626 images/s: the per-step repack and
+# "0" (default) off.  Measured on ViT-B/16 bs64, MI355X: float32 steps 880
+# images/s where the split products reach 1,345 (its forward and weight
+# gradient stay the float32 library GEMM; against those, 2-5% faster); fp16
+# autocast steps lose 20% (2,000 -> 1,620 images/s: the per-step repack and
 # a host read of each rotated layer's angles cost more than the kernel,
 # which is slower than the library's fp16 GEMM on the decoded weight).
 QAT_PACKED_GRAD = os.environ.get("RPFQ_QAT_PACKED_GRAD", "0")
